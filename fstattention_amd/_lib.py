@@ -68,6 +68,9 @@ SIGNATURES = {
                                     c_void_p]),
     "fsta_probe_empty_launch": (c_int, [c_int32, c_int32, c_void_p]),
     "fsta_probe_hbm_read": (c_int, [c_void_p, c_size_t, c_int32, c_int32, c_void_p, c_void_p]),
+    "fsta_quantize_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int32]),
+    "fsta_quantize_fp8": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32,
+                                  c_void_p, c_size_t, c_void_p]),
     "fsta_merge_states": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
                                   c_int32, c_int32, c_void_p]),
 }

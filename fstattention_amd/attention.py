@@ -176,7 +176,14 @@ def quantize_kv_fp8(k: torch.Tensor, v: torch.Tensor):
     """``k, v [Z,H,Nk,D]`` -> ``(k8, v8, k_scale, v_scale)`` for ``fst_attention``'s 8-bit K/V storage:
     ``float8_e4m3fn`` tensors and one float32 scale per (batch, head) slice (``[Z*H]``) chosen so that
     the slice's largest magnitude maps to the format's largest value (448).  ``k8 * k_scale`` is the K
-    the kernel computes with.  Plain tensor operations; a model would write its KV cache this way."""
+    the kernel computes with.  On the GPU one or two launches of a kernel of the library; tensors it does not take (on
+    the host, float64, of different shapes, rows that are no multiple of 16 bytes, a gradient asked for) go through the
+    same steps as tensor operations, with the same bytes."""
+    if k.is_cuda and k.dim() == 4 and v.device == k.device and v.shape == k.shape and v.dtype == k.dtype and k.dtype in _DTYPES and \
+            k.shape[2] * k.shape[3] % 16 == 0 and k.numel() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0 and \
+            not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)):
+        return (_OPS or _ops()).quantize_kv(k, v)
+
     def one(t):
         amax = t.float().abs().amax(dim=(2, 3))
         scale = torch.where(amax > 0, amax / _FP8_MAX, torch.ones_like(amax))

@@ -24,6 +24,7 @@ SOURCES = [
     "fsta_tree_order.hip",
     "fsta_tree_build.hip",
     "fsta_merge.hip",
+    "fsta_quantize.hip",
     "fsta_attention_generic.hip",
     "fsta_attention_mfma.hip",
     "fsta_attention_mfma16.hip",

@@ -160,9 +160,32 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tenso
     return {a_idx, a_mask, l_idx, bits, count, plan, st};
 }
 
+// k, v [Z, H, Nk, D] of one shape and one type (float32 / float16 / bfloat16) on the GPU -> e4m3 bytes of both and a
+// float32 scale per (batch, head) slice each.
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> quantize_kv(const at::Tensor& k, const at::Tensor& v) {
+    TORCH_CHECK_VALUE(k.dim() == 4 && v.sizes() == k.sizes() && v.scalar_type() == k.scalar_type(),
+                      "k and v must be [batch, heads, keys, head_dim] of one shape and dtype");
+    TORCH_CHECK_VALUE(k.is_cuda() && v.device() == k.device(), "k and v must live on one GPU");
+    const int code = dtype_code(k.scalar_type());
+    TORCH_CHECK_VALUE(code >= 0, "k and v must be float32, float16 or bfloat16");
+    const int64_t slices = k.size(0) * k.size(1), elements = k.size(2) * k.size(3);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(k.device());
+    const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(k.device().index()).stream();
+    const at::Tensor kc = k.contiguous(), vc = v.contiguous();
+    const auto fp8 = k.options().dtype(at::kFloat8_e4m3fn), f32 = k.options().dtype(at::kFloat);
+    at::Tensor k8 = at::empty(k.sizes(), fp8), v8 = at::empty(k.sizes(), fp8);
+    at::Tensor k_scale = at::empty({slices}, f32), v_scale = at::empty({slices}, f32);
+    const size_t need = fsta_quantize_workspace_bytes(slices, elements, code);
+    at::Tensor work = need ? at::empty({(int64_t)need}, k.options().dtype(at::kByte)) : at::Tensor();
+    check_rc(fsta_quantize_fp8(kc.data_ptr(), vc.data_ptr(), k8.data_ptr(), v8.data_ptr(), k_scale.data_ptr<float>(),
+                               v_scale.data_ptr<float>(), slices, elements, code, need ? work.data_ptr() : nullptr, need, stream));
+    return {k8, v8, k_scale, v_scale};
+}
+
 }  // namespace
 
 TORCH_LIBRARY(fsta, m) {
+    m.def("quantize_kv(Tensor k, Tensor v) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("precompute(Tensor(a!) lineage, Tensor level_lookup, int block_m, int max_ancestors, bool mutate_lineage, "
           "bool want_bool_mask, Tensor(b!)? status) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
     m.def("attention_fwd(Tensor q, Tensor k, Tensor v, Tensor ancestor_idx, Tensor mask_bits, Tensor anc_count, "
@@ -173,6 +196,7 @@ TORCH_LIBRARY(fsta, m) {
 TORCH_LIBRARY_IMPL(fsta, CUDA, m) {
     m.impl("attention_fwd", &attention_fwd);
     m.impl("precompute", &precompute);
+    m.impl("quantize_kv", &quantize_kv);
 }
 // tensors that all live on the host end up here: same message as for a mixed call
 TORCH_LIBRARY_IMPL(fsta, CPU, m) {

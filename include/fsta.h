@@ -333,6 +333,20 @@ int fsta_merge_states(const void* o_a, const float* lse_a, const void* o_b, cons
                       void* stream);
 
 /*
+ * K and V -> the 8-bit storage of fsta_attention_fwd_kv8 (no counterpart in the reference):
+ * per slice scale = max |x| / 448 (1 for a slice of zeros), byte = x / scale as OCP e4m3,
+ * rounded to nearest even.
+ *   a, b [slices, elements] of dtype (b may be NULL: one tensor), 16-byte aligned,
+ *   elements a multiple of 16; a8, b8 the bytes, a_scale, b_scale float32 [slices].
+ *   fsta_quantize_workspace_bytes: device memory (4-byte aligned) the call wants; 0 for
+ *   slices small enough to be kept in one workgroup's registers.
+ */
+size_t fsta_quantize_workspace_bytes(int64_t slices, int64_t elements, int32_t dtype);
+int fsta_quantize_fp8(const void* a, const void* b, void* a8, void* b8, float* a_scale, float* b_scale,
+                      int64_t slices, int64_t elements, int32_t dtype, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
+/*
  * new_parent[rank[i]] = rank[parent[i]] (-1 for roots): the parent array of the same
  * forest after node i has been renamed rank[i], e.g. with the rank of
  * fsta_dfs_order.  No counterpart in the reference (see fsta_dfs_order).  rank must

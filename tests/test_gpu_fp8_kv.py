@@ -82,6 +82,38 @@ def test_short_and_single_tile_lists():
     run_fp8(np.full(40, -1, dtype=np.int64), 32, 1, 2, 64, torch.bfloat16, 14)       # roots only: no ancestor tile
 
 
+@pytest.mark.parametrize("keys,d,dtype", [(1, 64, torch.bfloat16), (128, 128, torch.bfloat16), (129, 128, torch.float16),
+                                          (512, 128, torch.bfloat16), (513, 128, torch.bfloat16), (1023, 64, torch.float16),
+                                          (512, 128, torch.float32), (515, 128, torch.float32), (2100, 64, torch.float32),
+                                          (64, 16, torch.float32), (4000, 128, torch.bfloat16)])
+def test_quantize_matches_the_formula(keys, d, dtype):
+    """Slices on both sides of the one-launch limit (65536 elements), whole and partial pieces: bytes and scales of the
+    kernel are those of the formula, evaluated on the host, for ordinary values, zeros, tiny and huge magnitudes, infinities
+    and NaN."""
+    g = torch.Generator().manual_seed(keys + d)
+    k = torch.randn((2, 4, keys, d), generator=g).to(dtype)
+    v = torch.randn((2, 4, keys, d), generator=g) * torch.logspace(-3, 3, keys * d)[torch.randperm(keys * d, generator=g)].view(keys, d)
+    v = v.to(dtype)
+    k[0, 1] = 0.0
+    k[0, 2] *= 1e-4 if dtype is torch.float16 else 1e-36        # a scale near the end of the type's range
+    k[0, 3, 0, 3] = float("inf")
+    k[1, 0, -1, -1] = float("nan")
+    k[1, 1] = -k[1, 1].abs()
+    k[1, 1, 0, :4] = -0.0
+    if dtype is not torch.float32 and keys * d >= 65536:        # every bit pattern that is a finite number
+        bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+        v[1, 3].view(-1)[:65536] = torch.where(bits.isfinite(), bits, torch.zeros_like(bits))
+    got = quantize_kv_fp8(k.cuda(), v.cuda())
+    for t, t8, scale in ((k, got[0], got[2]), (v, got[1], got[3])):
+        amax = t.float().abs().amax(dim=(2, 3))
+        want = torch.where(amax > 0, amax * torch.tensor(1.0 / 448.0, dtype=torch.float32), torch.ones_like(amax))
+        assert torch.equal(scale.cpu().nan_to_num(nan=-1.0), want.view(-1).nan_to_num(nan=-1.0))
+        want8 = (t.float() / want[:, :, None, None]).to(torch.float8_e4m3fn)
+        a, b = t8.cpu().view(torch.uint8), want8.view(torch.uint8)
+        same = (a == b) | ((a & 0x7f == 0x7f) & (b & 0x7f == 0x7f))     # (the sign of a NaN is nobody's)
+        assert bool(same.all()), f"{int((~same).sum())} bytes differ"
+
+
 def test_argument_errors():
     parent = trees.random_recursive_parents(64, 5)
     a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32)
