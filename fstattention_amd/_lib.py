@@ -49,6 +49,7 @@ SIGNATURES = {
                                    c_int32, c_int32, c_int32, c_float, c_uint32, c_void_p]),
     "fsta_attention_workspace_bytes": (c_size_t, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                                   c_int32, c_float, c_uint32]),
+    "fsta_attention_uses_workspace": (c_int, [c_int32] * 8 + [c_float, c_uint32]),
     "fsta_attention_fwd_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
                                       c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
@@ -56,6 +57,10 @@ SIGNATURES = {
     "fsta_attention_fwd_kv8": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                        c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                        c_int32, c_int32, c_float, c_void_p]),
+    "fsta_attention_kv8_workspace_bytes": (c_size_t, [c_int32] * 8 + [c_float]),
+    "fsta_attention_fwd_kv8_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                          c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
+                                          c_int32, c_int32, c_float, c_void_p, c_size_t, c_void_p]),
     "fsta_lineage_from_parents": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                           c_void_p]),
     "fsta_dfs_order": (c_int, [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,

@@ -109,6 +109,100 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
     return (tiles + per - 1) / per;
 }
 
+// How the cache kernel (32 query rows per workgroup, tree and prefix in one launch) takes a launch: waves per workgroup
+// and runs of prefix tiles (runs = 0: not at all).  Shape and flags only.
+//
+// The number of runs is the one with the shortest predicted time.  The prediction, fitted to 650 timings over 8-256 rows,
+// 8-400 slices and 64-24000 keys (10 % mean error; the run count it picks costs 2 % over the best one):
+//   1.6 (launch) + rounds of workgroups * start_end + the larger of
+//     workgroups on the fullest CU * tiles * tile   (a CU's matrix cores, L2 and LDS)      [us]
+//     rounds * tiles per wave * wave_tile           (one wave's chain)
+//   but no less than the prefix read once at `tb` TB/s (rereading by the other row groups: a fraction `again` each),
+//   + for more than one run `join` and the float32 parts, written and read once at `join_tb` TB/s.
+struct CacheCost {
+    float start_end8, start_end4, tile, wave_tile, join, join_tb, tb, again;
+};
+constexpr CacheCost kCost16[2] = {{2.85f, 2.2f, 0.118f, 0.7f, 2.35f, 5.6f, 6.0f, 0.36f},      // head_dim 64
+                                  {3.5f, 2.9f, 0.276f, 0.0f, 2.9f, 6.4f, 5.6f, 0.21f}};      // head_dim 128
+constexpr CacheCost kCost8[2] = {{3.2f, 2.3f, 0.106f, 0.67f, 2.06f, 3.2f, 4.0f, 0.17f},       // the same on 8-bit K/V
+                                 {3.8f, 3.4f, 0.172f, 0.82f, 2.2f, 3.6f, 4.2f, 0.16f}};
+constexpr int kCacheMaxRows = 512;    // longer trees: their own kernels (a workgroup of the cache kernel reads the prefix for 32 rows)
+constexpr int kGpuCus = 256;
+
+CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, int block_m, float sm_scale, uint32_t flags,
+                     bool kv8) {
+    CachePlan c = {8, 0, 0};
+    const int prefix = nk - nq;
+    if (slices <= 0 || nq <= 0 || prefix <= 0 || nq > kCacheMaxRows) return c;
+    if ((flags & (FSTA_FLAG_GENERIC | FSTA_FLAG_WIDE_WAVES | FSTA_FLAG_STREAM | FSTA_FLAG_SHARE_TILES)) || !(sm_scale > 0.f) ||
+        !cache_kernel_supported(dtype, head_dim, block_m))
+        return c;
+    const int tiles = (prefix + kKeyTile - 1) / kKeyTile;
+    const int64_t groups = (nq + 31) / 32, wgs1 = slices * groups;
+    if (!kv8) {
+        // Enough rows and keys to be bound by the matrix cores: the dense prefix kernel, which shares every tile among 128
+        // rows (256 rows, 32 slices, 16384 keys, bf16: 119 us against 139; 8192 keys: 76 against 74).
+        const double dense_tiles = (double)((nq + kDenseRows - 1) / kDenseRows) * (double)slices * tiles / kGpuCus;
+        if (nq >= 96 && prefix >= kDenseMinKeys && dense_tiles >= (head_dim == 128 ? 64.0 : 110.0)) return c;
+        // Many workgroups with little to do each: the tree kernel, whose workgroups of 64 rows read half as much and start
+        // faster (97 rows, 154 slices, 283 keys: 16.5 against 17.7 us; 119 rows, 396 slices, 1487 keys: 90 against 106).
+        if (head_dim == 128 && wgs1 > 512 && (prefix < 600 || (wgs1 > 1200 && nq > 96 && prefix < kDenseMinKeys))) return c;
+    }
+    const int forced = (int)((flags >> 8) & 0xffu);
+    const CacheCost& k = (kv8 ? kCost8 : kCost16)[head_dim == 128 ? 1 : 0];
+    const double bytes = (double)slices * prefix * head_dim * (kv8 ? 2.0 : 4.0) * 1e-6;      // prefix K and V, MB
+    double best = 0.0;
+    // candidates: one run, and the counts that fill the CUs once, twice, ..; a run has work for half of a workgroup's waves
+    for (int i = 0; i <= 4; ++i) {
+        const int64_t fill = i == 0 ? 1 : (int64_t)kGpuCus * i / wgs1;
+        const int want = forced ? forced : (int)(fill > 64 ? 64 : fill);
+        if (i > 0 && (forced || want <= 1 || tiles / want < 4)) continue;
+        const int per = (tiles + want - 1) / want;
+        const int runs = (tiles + per - 1) / per;
+        const int64_t wgs = wgs1 * runs;
+        // more workgroups than CUs: four waves each, so that one workgroup's start and end lie under another's tiles
+        const int waves = wgs > kGpuCus ? 4 : 8;
+        const double on_cu = (double)((wgs + kGpuCus - 1) / kGpuCus);
+        const int at_once = (head_dim == 128 ? 1 : 2) * (waves == 4 ? 2 : 1);
+        const double rounds = (double)(((int64_t)on_cu + at_once - 1) / at_once);
+        const double t_tiles = per + 3.0;                        // (a few ancestor tiles and the own rows)
+        const double chain = rounds * (double)((per + 3 + waves - 1) / waves) * k.wave_tile;
+        const double work = on_cu * t_tiles * k.tile;
+        double t = 1.6 + rounds * (waves == 8 ? k.start_end8 : k.start_end4) + (chain > work ? chain : work);
+        const double mem = 1.6 + k.start_end8 + bytes / k.tb * (1.0 + k.again * (double)(groups - 1));
+        if (mem > t) t = mem;
+        if (runs > 1) t += k.join + 2.0 * runs * (double)slices * nq * head_dim * 4e-6 / k.join_tb;
+        if (c.runs == 0 || t < best) {
+            best = t;
+            c.waves = waves;
+            c.runs = runs;
+            c.run_tiles = per;
+        }
+    }
+    return c;
+}
+
+// launches it; FSTA_EUNSUPPORTED where the plan says no or the lists need too much LDS
+int launch_cache(AttnParams p, int dtype, int out_dtype, int head_dim, bool kv8, bool fast_pv, CachePlan c, void* workspace,
+                 size_t workspace_bytes, size_t wanted_bytes, hipStream_t s) {
+    if (c.runs < 1) return FSTA_EUNSUPPORTED;
+    const int64_t slices = p.heads_total;
+    if (c.runs > 1 && (!workspace || workspace_bytes < wanted_bytes)) {      // (too small a workspace: no runs, as documented)
+        c.waves = slices * ((p.nq + 31) / 32) > kGpuCus ? 4 : 8;
+        c.runs = 1;
+        c.run_tiles = (p.prefix + kKeyTile - 1) / kKeyTile;
+    }
+    if (c.runs > 1 && reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(FSTA_EINVAL, "fsta_attention_fwd_ws: workspace must be 16-byte aligned");
+    if (c.runs > 1) {
+        p.part_o = static_cast<float*>(workspace);
+        p.part_lse = p.part_o + (size_t)c.runs * slices * p.nq * head_dim;
+    }
+    const int rc = launch_attention_cache(p, dtype, head_dim, kv8, fast_pv, c, s);
+    if (rc != FSTA_OK || c.runs == 1) return rc;
+    return launch_merge_splits(p.part_o, p.part_lse, c.runs, slices * p.nq, head_dim, p.o, out_dtype, p.lse, s);
+}
+
 }  // namespace
 
 extern "C" size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk,
@@ -119,9 +213,22 @@ extern "C" size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, i
     int split_tiles = 0;
     const int64_t slices = (int64_t)batch * heads;
     const int runs = plan_dense_prefix(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, &split_tiles);
-    if (runs > 0) return key_split_bytes(runs + 1, slices, nq, head_dim);
-    const int splits = plan_key_splits(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, &split_tiles);
-    return splits > 1 ? key_split_bytes(splits, slices, nq, head_dim) : 0;
+    size_t bytes = runs > 0 ? key_split_bytes(runs + 1, slices, nq, head_dim) : 0;
+    if (runs == 0) {
+        const int splits = plan_key_splits(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, &split_tiles);
+        if (splits > 1) bytes = key_split_bytes(splits, slices, nq, head_dim);
+    }
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+    if (c.runs > 1 && key_split_bytes(c.runs, slices, nq, head_dim) > bytes) bytes = key_split_bytes(c.runs, slices, nq, head_dim);
+    return bytes;
+}
+
+extern "C" int fsta_attention_uses_workspace(int32_t batch, int32_t heads, int32_t nq, int32_t nk, int32_t head_dim,
+                                             int32_t dtype, int32_t block_m, int32_t max_ancestors, float sm_scale,
+                                             uint32_t flags) {
+    if (fsta_attention_workspace_bytes(batch, heads, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, flags) == 0) return 0;
+    const CachePlan c = plan_cache((int64_t)batch * heads, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+    return c.runs == 1 ? 0 : 1;
 }
 
 extern "C" int fsta_attention_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -201,6 +308,14 @@ extern "C" int fsta_attention_fwd_ws(const void* q, const void* k, const void* v
     p.stream_mode = (flags & FSTA_FLAG_STREAM) ? 1 : 0;
 
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (p.plan) {
+        const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+        const size_t wanted = c.runs > 1 ? fsta_attention_workspace_bytes(batch, heads, nq, nk, head_dim, dtype, block_m, max_ancestors,
+                                                                          sm_scale, flags) : 0;
+        const int rc = launch_cache(p, dtype, out_dtype, head_dim, false, (flags & FSTA_FLAG_FAST_PV) != 0, c, workspace, workspace_bytes,
+                                    wanted, s);
+        if (rc != FSTA_EUNSUPPORTED) return rc;
+    }
     if (workspace && p.plan) {
         // a long prefix goes to the dense prefix kernel, run by run (slots 1 .. runs of the workspace); the tree
         // kernel then does the tree part and, in its epilogue, joins it with those partial results into o / lse
@@ -272,6 +387,25 @@ extern "C" int fsta_attention_fwd_kv8(const void* q, const void* k8, const void*
                                       int32_t plan_key_shift, int32_t batch, int32_t heads, int32_t nq, int32_t nk,
                                       int32_t head_dim, int32_t dtype, int32_t out_dtype, int32_t block_m,
                                       int32_t max_ancestors, int32_t num_blocks, float sm_scale, void* stream) {
+    return fsta_attention_fwd_kv8_ws(q, k8, v8, k_scale, v_scale, o, lse, block_plan, plan_key_shift, batch, heads, nq, nk,
+                                     head_dim, dtype, out_dtype, block_m, max_ancestors, num_blocks, sm_scale, nullptr, 0, stream);
+}
+
+extern "C" size_t fsta_attention_kv8_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk, int32_t head_dim,
+                                                     int32_t dtype, int32_t block_m, int32_t max_ancestors, float sm_scale) {
+    (void)max_ancestors;
+    if (batch <= 0 || heads <= 0 || nq <= 0 || nk <= nq || block_m <= 0) return 0;
+    const int64_t slices = (int64_t)batch * heads;
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, 0, true);
+    return c.runs > 1 ? key_split_bytes(c.runs, slices, nq, head_dim) : 0;
+}
+
+extern "C" int fsta_attention_fwd_kv8_ws(const void* q, const void* k8, const void* v8, const float* k_scale,
+                                         const float* v_scale, void* o, float* lse, const uint32_t* block_plan,
+                                         int32_t plan_key_shift, int32_t batch, int32_t heads, int32_t nq, int32_t nk,
+                                         int32_t head_dim, int32_t dtype, int32_t out_dtype, int32_t block_m,
+                                         int32_t max_ancestors, int32_t num_blocks, float sm_scale, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
     if (batch < 0 || heads < 0 || nq < 0 || nk < nq)
         return fail(FSTA_EINVAL, "fsta_attention_fwd_kv8: batch=%d heads=%d nq=%d nk=%d (need nk >= nq >= 0)", batch,
                     heads, nq, nk);
@@ -312,5 +446,10 @@ extern "C" int fsta_attention_fwd_kv8(const void* q, const void* k8, const void*
     p.share_tiles = 0;
     p.k_scale = k_scale; p.v_scale = v_scale;
     p.merge_parts = 0; p.dry_run = 0; p.stream_mode = 0;
-    return launch_attention_mfma16_kv8(p, dtype, head_dim, static_cast<hipStream_t>(stream));
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, 0, true);
+    const int rc = launch_cache(p, dtype, out_dtype, head_dim, true, false, c, workspace, workspace_bytes,
+                                c.runs > 1 ? key_split_bytes(c.runs, slices, nq, head_dim) : 0, s);
+    if (rc != FSTA_EUNSUPPORTED) return rc;
+    return launch_attention_mfma16_kv8(p, dtype, head_dim, s);
 }

@@ -123,6 +123,15 @@ int launch_attention_prefix(const AttnParams& p, int dtype, int head_dim, bool f
 bool prefix_kernel_supported(int dtype, int head_dim);
 // workgroups that stay and walk a list of (block, slice) pairs; FSTA_EUNSUPPORTED where the launch has too few pairs or a prefix
 int launch_attention_stream(const AttnParams& p, int dtype, int head_dim, bool fast_pv, hipStream_t stream);
+// tree and prefix by workgroups of 32 query rows whose waves deal the tiles out among themselves
+struct CachePlan {
+    int waves;          // per workgroup: 8, or 4 (twice the workgroups per CU)
+    int runs;           // of prefix tiles; above 1 every run writes a float32 part into its slot of part_o / part_lse
+    int run_tiles;      // prefix tiles per run (no run is empty)
+};
+bool cache_kernel_supported(int dtype, int head_dim, int block_m);
+int launch_attention_cache(const AttnParams& p, int dtype, int head_dim, bool kv8, bool fast_pv, const CachePlan& plan,
+                           hipStream_t stream);
 int launch_attention_mfma16_kv8(const AttnParams& p, int dtype, int head_dim, hipStream_t stream);
 bool mfma_supported(int dtype, int head_dim, int block_m);
 // joins `splits` partial results (layout of AttnParams::part_o / part_lse) into o (and lse, may be null)

@@ -62,20 +62,39 @@ __global__ __launch_bounds__(kMergeThreads) void merge_splits_kernel(
                                                             : idx / chunks_per_row;
     if (row >= rows) return;
     const int chunk = (int)(idx - row * chunks_per_row);
-    float m = -INFINITY;
-    for (int s = 0; s < splits; ++s) m = fmaxf(m, part_lse[(size_t)s * rows + row]);
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    float sum = 0.f;
     const size_t part_stride = (size_t)rows * chunks_per_row;   // in float4
     const float4* src = reinterpret_cast<const float4*>(part_o) + (size_t)row * chunks_per_row + chunk;
-    for (int s = 0; s < splits; ++s) {
-        const float l = part_lse[(size_t)s * rows + row];
-        const float w = l == -INFINITY ? 0.f : exp2f(l - m);   // a part without keys drops out
-        const float4 x = src[(size_t)s * part_stride];
-        if (w > 0.f) {
-            acc[0] += w * x.x; acc[1] += w * x.y; acc[2] += w * x.z; acc[3] += w * x.w;
+    // Four parts at a time, all their loads ahead of the first use (a part's weight decides nothing about its load: one
+    // round trip per four parts instead of two per part).  A part's rows are finite, also where it has no keys.
+    float m = -INFINITY, sum = 0.f;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < splits; s0 += 4) {
+        float l[4];
+        float4 x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int s = min(s0 + u, splits - 1);
+            l[u] = part_lse[(size_t)s * rows + row];
+            x[u] = src[(size_t)s * part_stride];
+        }
+        float m_new = m;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (s0 + u >= splits) l[u] = -INFINITY;
+            m_new = fmaxf(m_new, l[u]);
+        }
+        const float safe = m_new == -INFINITY ? 0.f : m_new;
+        const float old = exp2f(m - safe);      // exp2(-inf) = 0
+        sum *= old;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] *= old;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float w = exp2f(l[u] - safe);
+            acc[0] += w * x[u].x; acc[1] += w * x[u].y; acc[2] += w * x[u].z; acc[3] += w * x[u].w;
             sum += w;
         }
+        m = m_new;
     }
     const float inv = sum > 0.f ? 1.f / sum : 0.f;
     struct alignas(sizeof(T) * 4) Pack { T v[4]; };

@@ -90,17 +90,21 @@ std::tuple<at::Tensor, at::Tensor> attention_fwd(const at::Tensor& q, const at::
             TORCH_CHECK_VALUE(!s->has_value() || ((*s)->scalar_type() == at::kFloat && (*s)->numel() == Z * H &&
                                              (*s)->is_contiguous() && (*s)->device() == q.device()),
                         "k_scale / v_scale must be contiguous float32 tensors of batch*heads entries on q's device");
-        check_rc(fsta_attention_fwd_kv8(q.data_ptr(), k.data_ptr(), v.data_ptr(), static_cast<const float*>(ptr_or_null(k_scale)),
+        const size_t need = Nk > Nq ? fsta_attention_kv8_workspace_bytes((int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
+                                                                         (int32_t)block_m, (int32_t)max_ancestors, (float)sm_scale) : 0;
+        at::Tensor parts = need ? at::empty({(int64_t)need}, q.options().dtype(at::kByte)) : at::Tensor();
+        check_rc(fsta_attention_fwd_kv8_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), static_cast<const float*>(ptr_or_null(k_scale)),
                                         static_cast<const float*>(ptr_or_null(v_scale)), o.data_ptr(), lse_ptr, plan_ptr,
                                         (int32_t)key_shift, (int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
                                         (int32_t)out_dtype_code, (int32_t)block_m, (int32_t)max_ancestors, (int32_t)nb,
-                                        (float)sm_scale, stream));
+                                        (float)sm_scale, need ? parts.data_ptr() : nullptr, need, stream));
         return {o, lse};
     }
     // a shared prefix may be worth cutting into key runs: the library says how much workspace that takes
     at::Tensor work;
     size_t work_bytes = 0;
-    if (Nk > Nq) {
+    if (Nk > Nq && fsta_attention_uses_workspace((int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code, (int32_t)block_m,
+                                                 (int32_t)max_ancestors, (float)sm_scale, (uint32_t)flags)) {
         work_bytes = fsta_attention_workspace_bytes((int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
                                                     (int32_t)block_m, (int32_t)max_ancestors, (float)sm_scale, (uint32_t)flags);
         if (work_bytes) work = at::empty({(int64_t)work_bytes}, q.options().dtype(at::kByte));

@@ -212,6 +212,10 @@ int fsta_attention_fwd(const void* q, const void* k, const void* v, void* o, flo
 size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk,
                                       int32_t head_dim, int32_t dtype, int32_t block_m,
                                       int32_t max_ancestors, float sm_scale, uint32_t flags);
+/* 0 where a workspace of that size would not be touched (nor need be provided), else 1. */
+int fsta_attention_uses_workspace(int32_t batch, int32_t heads, int32_t nq, int32_t nk, int32_t head_dim,
+                                  int32_t dtype, int32_t block_m, int32_t max_ancestors, float sm_scale,
+                                  uint32_t flags);
 int fsta_attention_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
                           const int64_t* ancestor_idx, const uint32_t* mask_bits,
                           const int32_t* anc_count, const int64_t* leaf_idx,
@@ -241,6 +245,23 @@ int fsta_attention_fwd_kv8(const void* q, const void* k8, const void* v8, const 
                            int32_t plan_key_shift, int32_t batch, int32_t heads, int32_t nq, int32_t nk,
                            int32_t head_dim, int32_t dtype, int32_t out_dtype, int32_t block_m,
                            int32_t max_ancestors, int32_t num_blocks, float sm_scale, void* stream);
+
+/*
+ * The same with a caller-provided device workspace, so that a long prefix in front
+ * of few (batch, head) slices can be cut into runs of keys, as
+ * fsta_attention_fwd_ws does for 16-bit K and V.  fsta_attention_kv8_workspace_bytes:
+ * bytes wanted (16-byte aligned), 0 when the launch would not be cut; without (or with
+ * too small) a workspace the call is fsta_attention_fwd_kv8.
+ */
+size_t fsta_attention_kv8_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk,
+                                          int32_t head_dim, int32_t dtype, int32_t block_m,
+                                          int32_t max_ancestors, float sm_scale);
+int fsta_attention_fwd_kv8_ws(const void* q, const void* k8, const void* v8, const float* k_scale,
+                              const float* v_scale, void* o, float* lse, const uint32_t* block_plan,
+                              int32_t plan_key_shift, int32_t batch, int32_t heads, int32_t nq, int32_t nk,
+                              int32_t head_dim, int32_t dtype, int32_t out_dtype, int32_t block_m,
+                              int32_t max_ancestors, int32_t num_blocks, float sm_scale,
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * parent[n_nodes] int64 (parent[i] < i, -1 for roots) -> level_lookup [n_nodes]

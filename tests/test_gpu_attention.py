@@ -267,6 +267,24 @@ def test_prefix_cut_into_key_runs(dtype, block_m, d, prefix, splits):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nodes,block_m,d,z,h,prefix,splits", [
+    (1, 32, 128, 1, 1, 1, None),            # one key of prefix, one node
+    (5, 32, 64, 1, 2, 31, None),            # a partial tile only
+    (32, 32, 128, 1, 3, 32, None),          # one whole tile
+    (40, 64, 128, 1, 2, 257, None),         # one tile more than waves, the last with one key
+    (100, 128, 64, 1, 3, 300, 9),           # a run per tile, the last one shorter
+    (200, 32, 128, 1, 5, 96, 3),            # seven blocks with lists of their own
+    (300, 64, 64, 2, 9, 520, None),
+    (60, 64, 128, 2, 72, 130, None),        # more workgroups than CUs: four waves each
+    (33, 64, 128, 3, 43, 1000, None)])
+def test_cache_kernel_edges(dtype, nodes, block_m, d, z, h, prefix, splits):
+    """The kernel that takes tree and prefix in one launch: remainders of tiles, waves, runs and row groups."""
+    parent = trees.random_recursive_parents(nodes, nodes + prefix, window=24)
+    run_tree(parent, block_m, z, h, d, dtype, 5, prefix=prefix, key_splits=splits, native_out=True,
+             want_kernel="attn_cache_kernel")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("scale", [0.3, 1.0])
 def test_dense_prefix_kernel_with_peaked_weights(dtype, scale):
     """A long prefix goes to the dense prefix kernel.  Scores scaled up until one or two keys carry nearly all the

@@ -69,6 +69,14 @@ def test_shared_prefix(prefix):
     run_fp8(parent, 64, 1, 4, 128, torch.bfloat16, 9, prefix=prefix)
 
 
+@pytest.mark.parametrize("nodes,block_m,d,z,h,prefix", [(1, 32, 128, 1, 1, 1), (40, 64, 64, 1, 2, 287), (70, 32, 128, 1, 3, 2050),
+                                                        (129, 64, 128, 2, 60, 600), (30, 64, 64, 1, 8, 5000)])
+def test_prefix_remainders_and_runs(nodes, block_m, d, z, h, prefix):
+    """Remainders of tiles and waves, several runs of keys, more workgroups than CUs."""
+    parent = trees.random_recursive_parents(nodes, prefix, window=24)
+    run_fp8(parent, block_m, z, h, d, torch.bfloat16 if nodes % 2 else torch.float16, 15, prefix=prefix)
+
+
 def test_per_slice_scales_and_no_scales():
     parent = trees.medusa_parents(n=256, seed=77)
     run_fp8(parent, 64, 2, 4, 128, torch.bfloat16, 11, spread=64.0)
