@@ -116,6 +116,7 @@ def load():
 
 TORCH_OPS_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_fsta_torch.so")
 _ops = None
+calls = None      # the entry points as plain C functions (module `_fsta_torch`), once load_torch_ops() has run
 
 
 def load_torch_ops():
@@ -126,8 +127,15 @@ def load_torch_ops():
     load()
     if not os.path.exists(TORCH_OPS_PATH):
         raise ImportError(f"{TORCH_OPS_PATH} is missing: build it with `python -m fstattention_amd.build`")
+    import importlib.machinery
+    import importlib.util
     import torch
-    torch.ops.load_library(TORCH_OPS_PATH)
+    # the file is the operator registration and a Python module in one
+    loader = importlib.machinery.ExtensionFileLoader("_fsta_torch", TORCH_OPS_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_fsta_torch", TORCH_OPS_PATH, loader=loader))
+    loader.exec_module(module)
+    global calls
+    calls = module
     _ops = torch.ops.fsta
     return _ops
 

@@ -228,6 +228,17 @@ def fst_attention(q, k, v, ancestor_idx, ancestor_mask, leaf_idx, sm_scale,
     mis-handles raise ``ValueError`` here (non-contiguous tensors, index
     tensors whose shapes do not match ``BLOCK_M`` / ``MAX_ANCESTORS``).
     """
+    flags = 0
+    if fast_pv or generic or wide_waves or key_splits or share_tiles or stream_blocks:
+        flags = (_lib.FLAG_FAST_PV if fast_pv else 0) | (_lib.FLAG_GENERIC if generic else 0) | \
+            (_lib.FLAG_WIDE_WAVES if wide_waves else 0) | (_lib.flag_key_splits(key_splits) if key_splits else 0) | \
+            (_lib.FLAG_SHARE_TILES if share_tiles else 0) | \
+            (_lib.FLAG_STREAM if stream_blocks else 0)
+    # an ordinary call (packed inputs in hand or remembered, nothing to complain about) is one C function
+    out = (_CALLS or _calls()).attention(q, k, v, ancestor_idx, ancestor_mask, leaf_idx, sm_scale, BLOCK_M, MAX_ANCESTORS,
+                                         out_dtype, return_lse, flags, k_scale, v_scale)
+    if out is not NotImplemented:
+        return out
     # shape constraints (the reference's two assertions)
     Lq, Lk, Lv = q.shape[-1], k.shape[-1], v.shape[-1]
     assert Lq == Lk and Lk == Lv
@@ -257,12 +268,6 @@ def fst_attention(q, k, v, ancestor_idx, ancestor_mask, leaf_idx, sm_scale,
     out_code = _DTYPES.get(out_dtype or q.dtype)
     if out_code is None:
         raise ValueError("q must be float32/float16/bfloat16 and out_dtype the input dtype or torch.float32")
-    flags = 0
-    if fast_pv or generic or wide_waves or key_splits or share_tiles or stream_blocks:
-        flags = (_lib.FLAG_FAST_PV if fast_pv else 0) | (_lib.FLAG_GENERIC if generic else 0) | \
-            (_lib.FLAG_WIDE_WAVES if wide_waves else 0) | (_lib.flag_key_splits(key_splits) if key_splits else 0) | \
-            (_lib.FLAG_SHARE_TILES if share_tiles else 0) | \
-            (_lib.FLAG_STREAM if stream_blocks else 0)
     # everything else (the remaining checks, o and L, the workspace of key runs, the launch on the current stream)
     # happens in the registered operator, csrc/fsta_torch_binding.cpp
     o, lse = (_OPS or _ops()).attention_fwd(q, k, v, ancestor_idx, packed.mask_bits, packed.anc_count, leaf_idx, packed.plan,
@@ -272,12 +277,22 @@ def fst_attention(q, k, v, ancestor_idx, ancestor_mask, leaf_idx, sm_scale,
 
 
 _OPS = None
+_CALLS = None
 
 
 def _ops():
     global _OPS
     _OPS = _lib.load_torch_ops()
     return _OPS
+
+
+def _calls():
+    """The module of plain C functions, told about the type and the table it reads."""
+    global _CALLS
+    _ops()
+    _lib.calls.setup(PackedTreeMask, _PACKED)
+    _CALLS = _lib.calls
+    return _CALLS
 
 
 def shift_for_prefix(ancestor_idx: torch.Tensor, leaf_idx: torch.Tensor, prefix: int,

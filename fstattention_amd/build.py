@@ -128,23 +128,32 @@ def build_library(verbose: bool = True, jobs: int | None = None, timeline: bool 
 
 
 TORCH_OPS_PATH = os.path.join(PKG_DIR, "_fsta_torch.so")
+TORCH_SOURCES = ["fsta_torch_binding.cpp", "fsta_torch_python.cpp"]
 
 
 def build_torch_ops(verbose: bool = True) -> str:
     """Compiles ``csrc/fsta_torch_binding.cpp`` (host code: the ``torch.ops.fsta`` registration on top of
-    the C ABI) with the host compiler against this interpreter's torch and links it to ``libfsta.so``."""
+    the C ABI) and ``csrc/fsta_torch_python.cpp`` (the same entry points as a Python module) with the host
+    compiler against this interpreter's torch and links them to ``libfsta.so``."""
+    import sysconfig
+
     import torch
     from torch.utils import cpp_extension as ce
     cxx = os.environ.get("CXX") or shutil.which("g++")
     if not cxx:
         raise RuntimeError("g++ not found (set CXX)")
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    includes = [f"-I{d}" for d in ce.include_paths("cuda")]
+    includes = [f"-I{d}" for d in (*ce.include_paths("cuda"), sysconfig.get_paths()["include"])]
     tmp = TORCH_OPS_PATH + ".tmp"
-    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-deprecated-declarations",
-          *includes, os.path.join(CSRC, "fsta_torch_binding.cpp"), "-o", tmp,
-          f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-ltorch",
+    flags = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-deprecated-declarations"]
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    objs = [os.path.join(OBJ_DIR, f.replace(".cpp", ".host.o")) for f in TORCH_SOURCES]
+    with ThreadPoolExecutor(max_workers=len(objs)) as pool:
+        list(pool.map(lambda so: _run([cxx, *flags, *includes, "-c", os.path.join(CSRC, so[0]), "-o", so[1]]),
+                      zip(TORCH_SOURCES, objs)))
+    _run([cxx, "-shared", *objs, "-o", tmp,
+          f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-ltorch", "-ltorch_python",
           f"-L{PKG_DIR}", "-l:libfsta.so", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"])
     os.replace(tmp, TORCH_OPS_PATH)
     if verbose:

@@ -5,16 +5,15 @@
 // reference fstattention.py:153-181 does in Python (shape checks, allocation of o and L, launch), so
 // that an eager caller pays the dispatcher and one allocation per call instead of a page of Python.
 // Device memory, streams and the device guard are torch's; everything below the C ABI is libfsta's.
-#include <ATen/ATen.h>
+#include "fsta_torch.h"
+
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
 
-#include <tuple>
-
 #include "../../include/fsta.h"
 
-namespace {
+namespace fsta_torch {
 
 int dtype_code(at::ScalarType t) {
     switch (t) {
@@ -25,11 +24,11 @@ int dtype_code(at::ScalarType t) {
     }
 }
 
-void check_rc(int rc) {
+static void check_rc(int rc) {
     TORCH_CHECK(rc == FSTA_OK, "libfsta error ", rc, ": ", fsta_last_error());
 }
 
-const void* ptr_or_null(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
+static const void* ptr_or_null(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
 // q [Z,H,Nq,D], k/v [Z,H,Nk,D] (16-bit or float32; k/v float8_e4m3fn for 8-bit storage with optional
 // per-slice scales), the reference's index tensors, their packed forms, the block plan (or None).
@@ -186,7 +185,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> quantize_kv(const at:
     return {k8, v8, k_scale, v_scale};
 }
 
-}  // namespace
+}  // namespace fsta_torch
+
+using namespace fsta_torch;
 
 TORCH_LIBRARY(fsta, m) {
     m.def("quantize_kv(Tensor k, Tensor v) -> (Tensor, Tensor, Tensor, Tensor)");
