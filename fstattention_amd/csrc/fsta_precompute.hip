@@ -21,16 +21,141 @@ __host__ __device__ inline size_t precompute_lds_words(int64_t n_words, int mask
     return (size_t)(2 * n_words) + (size_t)mask_words * block_m + block_m + 4;
 }
 
+// The steps both kernels below share, once the ancestor set of block `j` is a bitmap in LDS.  `out`: where the block's
+// results go (the tensors of the whole call; optional ones may be null).
+struct BlockOutputs {
+    int64_t* ancestor_idx;     // [nb, max_anc]
+    uint8_t* ancestor_mask;    // [nb, block_m, max_anc] or null
+    int64_t* leaf_idx;         // [nb, block_m]
+    uint32_t* mask_bits;       // [nb, mask_words, block_m] or null
+    int32_t* anc_count;        // [nb] or null
+    uint32_t* plan;            // block plan or null
+};
+
+// Exclusive prefix sum of the per-word popcounts -> rank of every ancestor, their number in misc[2]; by the first wave,
+// each lane a run of consecutive words.
+__device__ __forceinline__ void rank_ancestors(const uint32_t* bitmap, uint32_t* rank_base, uint32_t* misc, int n_words) {
+    const int tid = threadIdx.x;
+    const int per_lane = (n_words + 63) / 64;
+    const int w_begin = min(tid * per_lane, n_words);
+    const int w_end = min(w_begin + per_lane, n_words);
+    uint32_t local = 0u;
+    for (int w = w_begin; w < w_end; ++w) local += __popc(bitmap[w]);
+    uint32_t incl = local;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t up = __shfl_up(incl, d, 64);
+        if (tid >= d) incl += up;
+    }
+    uint32_t run = incl - local;
+    for (int w = w_begin; w < w_end; ++w) { rank_base[w] = run; run += __popc(bitmap[w]); }
+    if (tid == 63) misc[2] = incl;
+}
+
+// ancestor_idx: ascending ids, left aligned, -1 padded (utils.py:112,120), the block plan receives the same ids as 32-bit
+// keys; leaves: ids of the block's range that are not in the set, the range not clipped to n_nodes (utils.py:121-122).
+// Ids at or above `set_end` are in no set.  misc[3]: first key of the last ancestor tile in use.
+__device__ __forceinline__ void write_lists(const BlockOutputs& out, int j, int64_t lo, int64_t n_nodes, int64_t set_end, int block_m,
+                                            int max_anc, int kept, const uint32_t* bitmap, const uint32_t* rank_base, uint32_t* misc) {
+    const int tid = threadIdx.x, threads = blockDim.x;
+    const int n_words = (int)((set_end + 31) >> 5);
+    uint32_t* rec = out.plan ? out.plan + (size_t)j * plan_layout(block_m, max_anc).block_words : nullptr;
+    const uint32_t last_tile_first = kept > 0 ? (uint32_t)((kept - 1) & ~31) : 0xffffffffu;   // first slot of the last tile in use
+    int64_t* list = out.ancestor_idx + (size_t)j * max_anc;
+    for (int c = kept + tid; c < max_anc; c += threads) list[c] = -1;
+    auto entry = [&](uint32_t r, uint32_t id) {
+        if (r >= (uint32_t)max_anc) return;
+        list[r] = (int64_t)id;
+        if (rec) rec[kPlanHeaderWords + r] = id;
+        if (r == last_tile_first) misc[3] = id;
+    };
+    if (set_end <= 16 * (int64_t)threads) {      // a thread per id: its stores depend on nothing but two reads
+        for (int i = tid; i < (int)set_end; i += threads) {
+            const uint32_t word = bitmap[i >> 5], bit = 1u << (i & 31);
+            if (word & bit) entry(rank_base[i >> 5] + __popc(word & (bit - 1u)), (uint32_t)i);
+        }
+    } else {                                     // many ids, few of them set: a thread per word
+        for (int w = tid; w < n_words; w += threads) {
+            uint32_t bits = bitmap[w];
+            for (uint32_t r = rank_base[w]; bits; ++r) {
+                entry(r, (uint32_t)(w * 32 + __ffs(bits) - 1));
+                bits &= bits - 1u;
+            }
+        }
+    }
+    if (out.anc_count && tid == 0) out.anc_count[j] = kept;
+    for (int r = tid; r < block_m; r += threads) {
+        const int64_t id = lo + r;
+        const bool is_anc = id < n_nodes && ((bitmap[id >> 5] >> (id & 31)) & 1u);
+        out.leaf_idx[(size_t)j * block_m + r] = is_anc ? -1 : id;
+    }
+}
+
+// The block's mask words in every form asked for, and the rest of the block plan.
+__device__ __forceinline__ void write_masks(const BlockOutputs& out, int j, int64_t lo, int64_t n_nodes, int block_m, int max_anc,
+                                            int mask_words, int kept, const uint32_t* bitmap, const uint32_t* mbits,
+                                            const uint32_t* misc) {
+    const int tid = threadIdx.x, threads = blockDim.x;
+    const PlanLayout layout = plan_layout(block_m, max_anc);
+    uint32_t* rec = out.plan ? out.plan + (size_t)j * layout.block_words : nullptr;
+    if (out.mask_bits) {
+        for (int e = tid; e < mask_words * block_m; e += threads)
+            out.mask_bits[(size_t)j * mask_words * block_m + e] = mbits[e];
+    }
+    if (rec) {
+        // Block plan: what the attention kernel would otherwise derive from the lists in every
+        // workgroup.  An empty slot repeats a row its tile holds anyway (the first key of the last
+        // ancestor tile in use, the first leaf of a group of 32 rows), so that every tile is
+        // gathered with the same number of requests; its mask bits are zero by construction.
+        const int tiles = layout.tiles, groups = block_m / 32;
+        const uint32_t spare = kept > 0 ? misc[3] : (uint32_t)lo;
+        for (int c = kept + tid; c < tiles * 32; c += threads) rec[kPlanHeaderWords + c] = spare;
+        if (tid == 0) rec[0] = (uint32_t)kept;
+        else if (tid < kPlanHeaderWords && (tid < kPlanLeafValid || tid - kPlanLeafValid >= groups)) rec[tid] = 0u;
+        if (tid < block_m) {   // (block_m <= 128: the first two waves)
+            const int64_t id = lo + tid;
+            const bool is_anc = id < n_nodes && ((bitmap[id >> 5] >> (id & 31)) & 1u);
+            const uint64_t vote = __ballot(!is_anc);
+            const uint32_t mine = (tid & 32) ? (uint32_t)(vote >> 32) : (uint32_t)vote;   // this group of 32 rows
+            const uint32_t first_leaf = mine ? (uint32_t)(lo + (tid & ~31) + __builtin_ctz(mine)) : (uint32_t)lo;
+            uint32_t* grp = rec + layout.common_words + (tid >> 5) * layout.group_words;
+            grp[tid & 31] = is_anc ? first_leaf : (uint32_t)id;
+            if ((tid & 31) == 0) rec[kPlanLeafValid + (tid >> 5)] = mine;
+        }
+        for (int e = tid; e < groups * tiles * 32; e += threads) {
+            const int g = e / (tiles * 32), rem = e - g * tiles * 32;   // rem = 32 * tile + row within the group
+            rec[layout.common_words + g * layout.group_words + 32 + rem] = mbits[(rem >> 5) * block_m + g * 32 + (rem & 31)];
+        }
+    }
+    if (out.ancestor_mask) {
+        // one byte per (row, ancestor slot); 8 slots of a row per store where the layout allows
+        uint8_t* bytes = out.ancestor_mask + (size_t)j * block_m * max_anc;
+        if (max_anc % 8 == 0 && reinterpret_cast<uintptr_t>(bytes) % 8 == 0) {
+            const int per_row = max_anc / 8;
+            for (int e = tid; e < block_m * per_row; e += threads) {
+                const int r = e / per_row, c = (e - r * per_row) * 8;
+                const uint32_t bits = (mbits[(c >> 5) * block_m + r] >> (c & 31)) & 0xffu;
+                // bit i -> byte i: three doubling steps spread the 8 bits over 64
+                uint64_t x = bits;
+                x = (x | (x << 28)) & 0x0000000f0000000full;
+                x = (x | (x << 14)) & 0x0003000300030003ull;
+                x = (x | (x << 7)) & 0x0101010101010101ull;
+                reinterpret_cast<uint64_t*>(bytes)[e] = x;
+            }
+        } else {
+            const int n_out = block_m * max_anc;
+            for (int e = tid; e < n_out; e += threads) {
+                const int r = e / max_anc, c = e - r * max_anc;
+                bytes[e] = (uint8_t)((mbits[(c >> 5) * block_m + r] >> (c & 31)) & 1u);
+            }
+        }
+    }
+}
+
 __global__ __launch_bounds__(kMaxThreads) void block_precompute_kernel(
     int64_t* __restrict__ lineage, const int64_t* __restrict__ level_lookup,
     int64_t n_nodes, int64_t width, int block_m, int max_anc, int mask_words, int mutate, int staged,
-    int64_t* __restrict__ ancestor_idx, uint8_t* __restrict__ ancestor_mask,
-    int64_t* __restrict__ leaf_idx, uint32_t* __restrict__ mask_bits,
-    int32_t* __restrict__ anc_count, uint32_t* __restrict__ plan, const int64_t* __restrict__ parent,
-    uint32_t* __restrict__ status) {
-    // `parent` != NULL (fsta_precompute_from_parents): the block's lineage rows are not read but built here, from the
-    // parent array (copied into LDS as int32 behind the staged rows); `lineage` and `level_lookup` are then outputs
-    // (each may be NULL) and `staged` is 1.
+    BlockOutputs out, uint32_t* __restrict__ status) {
     extern __shared__ uint32_t lds[];
     const int n_words = (int)((n_nodes + 31) >> 5);
     uint32_t* bitmap = lds;                                   // ancestor set of this block
@@ -58,53 +183,12 @@ __global__ __launch_bounds__(kMaxThreads) void block_precompute_kernel(
         }
     };
     int64_t first[kBatch];
-    if (!parent) load_batch(tid, first);
-    int32_t* par_s = vals_s + (size_t)block_m * width;      // [n_nodes], from-parents mode only
+    load_batch(tid, first);
     uint32_t err = 0u;
-    if (parent) {
-        for (int64_t i = tid; i < n_nodes; i += threads) {
-            const int64_t pp = parent[i];
-            const bool ok = pp >= -1 && pp < i;
-            if (!ok) err |= FSTA_PRE_BAD_NODE_ID;
-            par_s[i] = ok ? (int32_t)pp : -1;
-        }
-    }
-
     for (int w = tid; w < n_words; w += threads) bitmap[w] = 0u;
     for (int e = tid; e < mask_words * block_m; e += threads) mbits[e] = 0u;
     if (tid < 4) misc[tid] = 0u;
-    if (parent) {
-        __syncthreads();
-        // One lane per row walks to the root once and notes the ancestors in hop order (every hop goes to a smaller
-        // id, so the walk ends), then turns its row around into level order, -1 padded (layout of utils.py:66-75:
-        // column l = the ancestor at level l; the node's own column holds -1 until the self entry goes in).
-        for (int r = tid; r < block_m; r += threads) {
-            int32_t lv = -1;
-            if (r < rows) {
-                int32_t* row = vals_s + (size_t)r * width;
-                int32_t depth = 0;
-                for (int32_t a = par_s[lo + r]; a >= 0; a = par_s[a]) {
-                    if (depth < width) row[depth] = a;
-                    ++depth;
-                }
-                if (depth >= width) {          // deeper than the rows are wide: flagged, the row counts as empty
-                    err |= FSTA_PRE_BAD_LEVEL;
-                    depth = 0;
-                } else {
-                    lv = depth;
-                }
-                for (int32_t a = 0, b = depth - 1; a < b; ++a, --b) {
-                    const int32_t x = row[a];
-                    row[a] = row[b];
-                    row[b] = x;
-                }
-                for (int32_t l = depth; l < width; ++l) row[l] = -1;
-                if (level_lookup) const_cast<int64_t*>(level_lookup)[lo + r] = lv >= 0 ? lv : 0;
-            }
-            lvl_s[r] = lv;
-        }
-    }
-    for (int r = tid; r < block_m && !parent; r += threads) {
+    for (int r = tid; r < block_m; r += threads) {
         int32_t lv = -1;  // -1 = nothing to insert (pad row or invalid level)
         if (r < rows) {
             int64_t l = level_lookup[lo + r];
@@ -137,33 +221,16 @@ __global__ __launch_bounds__(kMaxThreads) void block_precompute_kernel(
             if (staged) vals_s[e] = keep;
         }
     };
-    if (parent) {
-        __syncthreads();      // the rows are complete
-        for (uint32_t e = tid; e < n_elem; e += threads) {
-            const int32_t v = vals_s[e];
-            if (v < 0) saw_pad = true;
-            else {
-                const uint32_t bit = 1u << (v & 31);
-                if (!(bitmap[v >> 5] & bit)) atomicOr(&bitmap[v >> 5], bit);
-            }
-            if (lineage) {      // the rows as the lineage tensor (with the self entries when asked for)
-                const uint32_t r = e / (uint32_t)width, l = e - r * (uint32_t)width;
-                lineage[lo * width + e] = (mutate && (int32_t)l == lvl_s[r]) ? lo + r : (int64_t)v;
-            }
-        }
-    } else {
     take_batch(tid, first);
     for (uint32_t e0 = tid + (uint32_t)threads * kBatch; e0 < n_elem; e0 += (uint32_t)threads * kBatch) {
         int64_t val[kBatch];
         load_batch(e0, val);
         take_batch(e0, val);
     }
-    }
     if (saw_pad) misc[0] = 1u;
     __syncthreads();
 
-    // 2. exclusive prefix sum of the per-word popcounts -> rank of every ancestor; the first
-    //    wave scans, each lane a run of consecutive words
+    // 2. rank of every ancestor
     if (tid < 64) {
         // The reference drops the smallest unique value unconditionally (utils.py:119, the
         // `[1:]`); that is the -1 padding whenever one is present.  Without any -1 in the block
@@ -174,57 +241,17 @@ __global__ __launch_bounds__(kMaxThreads) void block_precompute_kernel(
             }
         }
         __builtin_amdgcn_wave_barrier();
-        const int per_lane = (n_words + 63) / 64;
-        const int w_begin = min(tid * per_lane, n_words);
-        const int w_end = min(w_begin + per_lane, n_words);
-        uint32_t local = 0u;
-        for (int w = w_begin; w < w_end; ++w) local += __popc(bitmap[w]);
-        uint32_t incl = local;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t up = __shfl_up(incl, d, 64);
-            if (tid >= d) incl += up;
-        }
-        uint32_t run = incl - local;
-        for (int w = w_begin; w < w_end; ++w) { rank_base[w] = run; run += __popc(bitmap[w]); }
-        if (tid == 63) misc[2] = incl;
+        rank_ancestors(bitmap, rank_base, misc, n_words);
     }
     __syncthreads();
     const uint32_t total = misc[2];
     if (total > (uint32_t)max_anc) err |= FSTA_PRE_TOO_MANY_ANCESTORS;
     const int kept = (int)min(total, (uint32_t)max_anc);
 
-    // 3. ancestor_idx: ascending ids, left aligned, -1 padded (utils.py:112,120); the block plan
-    //    receives the same ids as 32-bit keys
-    const PlanLayout layout = plan_layout(block_m, max_anc);
-    uint32_t* rec = plan ? plan + (size_t)j * layout.block_words : nullptr;
-    const uint32_t last_tile_first = kept > 0 ? (uint32_t)((kept - 1) & ~31) : 0xffffffffu;   // first slot of the last tile in use
-    for (int c = kept + tid; c < max_anc; c += threads) ancestor_idx[(size_t)j * max_anc + c] = -1;
-    for (int w = tid; w < n_words; w += threads) {
-        uint32_t bits = bitmap[w];
-        uint32_t r = rank_base[w];
-        while (bits) {
-            const int b = __ffs(bits) - 1;
-            bits &= bits - 1u;
-            if (r < (uint32_t)max_anc) {
-                ancestor_idx[(size_t)j * max_anc + r] = (int64_t)w * 32 + b;
-                if (rec) rec[kPlanHeaderWords + r] = (uint32_t)(w * 32 + b);
-                if (r == last_tile_first) misc[3] = (uint32_t)(w * 32 + b);
-            }
-            ++r;
-        }
-    }
-    if (anc_count && tid == 0) anc_count[j] = kept;
+    // 3. the lists
+    write_lists(out, j, lo, n_nodes, n_nodes, block_m, max_anc, kept, bitmap, rank_base, misc);
 
-    // 4. leaves: ids of the block's range that are not in the set; the range is
-    //    not clipped to n_nodes (utils.py:121-122)
-    for (int r = tid; r < block_m; r += threads) {
-        const int64_t id = lo + r;
-        const bool is_anc = id < n_nodes && ((bitmap[id >> 5] >> (id & 31)) & 1u);
-        leaf_idx[(size_t)j * block_m + r] = is_anc ? -1 : id;
-    }
-
-    // 5. mask: row r holds its lineage plus itself in its own level column
+    // 4. mask: row r holds its lineage plus itself in its own level column
     //    (utils.py:124-127); membership of ancestor c in that row
     //    A thread walks a run of consecutive levels of one row.  Ancestors along a path have
     //    increasing ids, hence increasing ranks: the bits of a run fall into one or two mask words,
@@ -258,66 +285,176 @@ __global__ __launch_bounds__(kMaxThreads) void block_precompute_kernel(
         }
     }
     __syncthreads();
+    write_masks(out, j, lo, n_nodes, block_m, max_anc, mask_words, kept, bitmap, mbits, misc);
 
-    if (mask_bits) {
-        for (int e = tid; e < mask_words * block_m; e += threads)
-            mask_bits[(size_t)j * mask_words * block_m + e] = mbits[e];
-    }
-    if (rec) {
-        // Block plan: what the attention kernel would otherwise derive from the lists in every
-        // workgroup.  An empty slot repeats a row its tile holds anyway (the first key of the last
-        // ancestor tile in use, the first leaf of a group of 32 rows), so that every tile is
-        // gathered with the same number of requests; its mask bits are zero by construction.
-        const int tiles = layout.tiles, groups = block_m / 32;
-        const uint32_t spare = kept > 0 ? misc[3] : (uint32_t)lo;
-        for (int c = kept + tid; c < tiles * 32; c += threads) rec[kPlanHeaderWords + c] = spare;
-        if (tid == 0) rec[0] = (uint32_t)kept;
-        else if (tid < kPlanHeaderWords && (tid < kPlanLeafValid || tid - kPlanLeafValid >= groups)) rec[tid] = 0u;
-        if (tid < block_m) {   // (block_m <= 128: the first two waves)
-            const int64_t id = lo + tid;
-            const bool is_anc = id < n_nodes && ((bitmap[id >> 5] >> (id & 31)) & 1u);
-            const uint64_t vote = __ballot(!is_anc);
-            const uint32_t mine = (tid & 32) ? (uint32_t)(vote >> 32) : (uint32_t)vote;   // this group of 32 rows
-            const uint32_t first_leaf = mine ? (uint32_t)(lo + (tid & ~31) + __builtin_ctz(mine)) : (uint32_t)lo;
-            uint32_t* grp = rec + layout.common_words + (tid >> 5) * layout.group_words;
-            grp[tid & 31] = is_anc ? first_leaf : (uint32_t)id;
-            if ((tid & 31) == 0) rec[kPlanLeafValid + (tid >> 5)] = mine;
-        }
-        for (int e = tid; e < groups * tiles * 32; e += threads) {
-            const int g = e / (tiles * 32), rem = e - g * tiles * 32;   // rem = 32 * tile + row within the group
-            rec[layout.common_words + g * layout.group_words + 32 + rem] = mbits[(rem >> 5) * block_m + g * 32 + (rem & 31)];
-        }
-    }
-    if (ancestor_mask) {
-        // one byte per (row, ancestor slot); 8 slots of a row per store where the layout allows
-        uint8_t* out = ancestor_mask + (size_t)j * block_m * max_anc;
-        if (max_anc % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0) {
-            const int per_row = max_anc / 8;
-            for (int e = tid; e < block_m * per_row; e += threads) {
-                const int r = e / per_row, c = (e - r * per_row) * 8;
-                const uint32_t bits = (mbits[(c >> 5) * block_m + r] >> (c & 31)) & 0xffu;
-                // bit i -> byte i: three doubling steps spread the 8 bits over 64
-                uint64_t x = bits;
-                x = (x | (x << 28)) & 0x0000000f0000000full;
-                x = (x | (x << 14)) & 0x0003000300030003ull;
-                x = (x | (x << 7)) & 0x0101010101010101ull;
-                reinterpret_cast<uint64_t*>(out)[e] = x;
-            }
-        } else {
-            const int n_out = block_m * max_anc;
-            for (int e = tid; e < n_out; e += threads) {
-                const int r = e / max_anc, c = e - r * max_anc;
-                out[e] = (uint8_t)((mbits[(c >> 5) * block_m + r] >> (c & 31)) & 1u);
-            }
-        }
-    }
-
-    // 6. the caller's lineage receives the self entries (utils.py:118,125)
-    if (mutate && !parent) {
+    // 5. the caller's lineage receives the self entries (utils.py:118,125)
+    if (mutate) {
         for (int r = tid; r < rows; r += threads)
             if (lvl_s[r] >= 0) lineage[(lo + r) * width + lvl_s[r]] = lo + r;
     }
     if (err) atomicOr(status, err);
+}
+
+// The same results from the parent array: no lineage row exists anywhere, the ancestors of a node are met on the way to
+// its root.  A path of depth d is a chain of d dependent LDS reads (about 110 cycles each), so 2^levels lanes share a row:
+// the tables jump[b][i] = 2^b-th ancestor of i, made by doubling, let lane t start at ancestor t + 1 and go on in steps
+// of 2^levels.  The path is walked twice, once to set the bits of the block's ancestor set and once, when the set is ranked,
+// to set the row's mask bits.  Only nodes below the block's end can be on a path: the rest of the array is neither read nor
+// doubled.  2048 nodes of 70 levels on average, blocks of 128 rows: 23.8 us with one lane per row and rows in LDS.
+//
+// LDS (words): bitmap[W] | rank_base[W] | mbits[mask_words * M] | lvl[M] | misc[4] | jump, (levels + 1) tables of 16-bit ids
+constexpr uint32_t kNoNode = 0xffffu;
+constexpr int kMaxLevels = 4;
+
+__global__ __launch_bounds__(kMaxThreads) void block_from_parents_kernel(
+    const int64_t* __restrict__ parent, int n_nodes, int width, int block_m, int max_anc, int mask_words, int levels,
+    int insert_self, int64_t* __restrict__ lineage, int64_t* __restrict__ level_lookup, BlockOutputs out,
+    uint32_t* __restrict__ status, uint32_t* __restrict__ host_flags) {
+    extern __shared__ uint32_t lds[];
+    const int n_words = (n_nodes + 31) >> 5;
+    uint32_t* bitmap = lds;
+    uint32_t* rank_base = bitmap + n_words;
+    uint32_t* mbits = rank_base + n_words;
+    int32_t* lvl_s = reinterpret_cast<int32_t*>(mbits + (size_t)mask_words * block_m);
+    uint32_t* misc = reinterpret_cast<uint32_t*>(lvl_s + block_m);          // [0] a row is too deep, [2] total count, [3] a listed ancestor
+    uint16_t* jump = reinterpret_cast<uint16_t*>(misc + 4);                 // [levels + 1][stride]
+    const int stride = (n_nodes + 1) & ~1;
+
+    const int tid = threadIdx.x;
+    const int threads = blockDim.x;
+    const int j = blockIdx.x;
+    const int lo = j * block_m;
+    const int rows = min(block_m, n_nodes - lo);
+    const int hi = lo + rows;
+    uint32_t err = 0u;
+
+    auto load_batch = [&](int i0, int64_t (&val)[kBatch]) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const int i = i0 + b * threads;
+            val[b] = i < hi ? parent[i] : -1;
+        }
+    };
+    auto take_batch = [&](int i0, const int64_t (&val)[kBatch]) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const int i = i0 + b * threads;
+            if (i >= hi) break;
+            const bool ok = val[b] >= -1 && val[b] < i;          // every hop goes to a smaller id: the walks end
+            if (!ok) err |= FSTA_PRE_BAD_NODE_ID;
+            jump[i] = (uint16_t)(ok && val[b] >= 0 ? (uint32_t)val[b] : kNoNode);
+        }
+    };
+    int64_t val[kBatch];
+    load_batch(tid, val);
+    for (int w = tid; w < n_words; w += threads) bitmap[w] = 0u;
+    for (int e = tid; e < mask_words * block_m; e += threads) mbits[e] = 0u;
+    if (tid < 4) misc[tid] = 0u;
+    take_batch(tid, val);
+    for (int i0 = tid + threads * kBatch; i0 < hi; i0 += threads * kBatch) {
+        load_batch(i0, val);
+        take_batch(i0, val);
+    }
+    __syncthreads();
+    for (int b = 0; b < levels; ++b) {
+        const uint16_t* from = jump + (size_t)b * stride;
+        uint16_t* to = jump + (size_t)(b + 1) * stride;
+#pragma unroll 4
+        for (int i = tid; i < hi; i += threads) {
+            const uint32_t a = from[i];
+            to[i] = a == kNoNode ? (uint16_t)kNoNode : from[a];
+        }
+        __syncthreads();
+    }
+
+    // calls visit(ancestor, hop) for the ancestors of row r that fall to lane t of its 2^levels
+    const uint16_t* far = jump + (size_t)levels * stride;
+    auto walk = [&](int r, int t, auto&& visit) {
+        uint32_t a = jump[lo + r];
+        for (int b = 0; b < levels; ++b)
+            if (((t >> b) & 1) && a != kNoNode) a = jump[(size_t)b * stride + a];
+        for (int hop = t; a != kNoNode; hop += 1 << levels) {
+            visit(a, hop);
+            a = far[a];
+        }
+    };
+    auto mark = [&](uint32_t a, int) {
+        const uint32_t bit = 1u << (a & 31);
+        if (!(bitmap[a >> 5] & bit)) atomicOr(&bitmap[a >> 5], bit);
+    };
+
+    // 1. the block's ancestor set, and every row's depth (the lanes of a row are neighbours in one wave)
+    const int lanes_of_rows = block_m << levels;
+    for (int e = tid; e < lanes_of_rows; e += threads) {
+        const int r = e >> levels, t = e & ((1 << levels) - 1);
+        int32_t depth = 0;
+        if (r < rows)
+            walk(r, t, [&](uint32_t a, int hop) {
+                mark(a, hop);
+                ++depth;
+            });
+        for (int d = 1; d < (1 << levels); d <<= 1) depth += __shfl_xor(depth, d, 64);
+        if (t == 0) {
+            int32_t lv = r < rows ? depth : -1;
+            if (lv >= width) {          // deeper than the rows are wide: flagged, the row counts as empty
+                err |= FSTA_PRE_BAD_LEVEL;
+                lv = -1;
+                misc[0] = 1u;
+            }
+            lvl_s[r] = lv;
+            if (r < rows && level_lookup) level_lookup[lo + r] = lv >= 0 ? lv : 0;
+        }
+    }
+    __syncthreads();
+    if (misc[0]) {      // (the set again, without the rows that are too deep)
+        for (int w = tid; w < n_words; w += threads) bitmap[w] = 0u;
+        __syncthreads();
+        for (int e = tid; e < lanes_of_rows; e += threads)
+            if (lvl_s[e >> levels] >= 0) walk(e >> levels, e & ((1 << levels) - 1), mark);
+        __syncthreads();
+    }
+
+    // 2. ranks (every row of a lineage tensor made from parents has a -1 somewhere, its own column: the value that the
+    //    reference drops, utils.py:119, is always that one)
+    if (tid < 64) rank_ancestors(bitmap, rank_base, misc, (hi + 31) >> 5);
+    __syncthreads();
+    const uint32_t total = misc[2];
+    if (total > (uint32_t)max_anc) err |= FSTA_PRE_TOO_MANY_ANCESTORS;
+    const int kept = (int)min(total, (uint32_t)max_anc);
+
+    // 3. the lists
+    write_lists(out, j, lo, n_nodes, hi, block_m, max_anc, kept, bitmap, rank_base, misc);
+
+    // 4. mask: a row's ancestors and the row itself (utils.py:124-127); the lineage row where it is wanted
+    for (int e = tid; e < lanes_of_rows; e += threads) {
+        const int r = e >> levels, t = e & ((1 << levels) - 1);
+        const int32_t depth = lvl_s[r];
+        if (r >= rows) continue;
+        int64_t* line = lineage ? lineage + (size_t)(lo + r) * width : nullptr;
+        auto set = [&](uint32_t a) {
+            const uint32_t word = bitmap[a >> 5], bit = 1u << (a & 31);
+            if (!(word & bit)) return;
+            const uint32_t rank = rank_base[a >> 5] + __popc(word & (bit - 1u));
+            if (rank < (uint32_t)max_anc) atomicOr(&mbits[(rank >> 5) * block_m + r], 1u << (rank & 31));
+        };
+        if (depth >= 0) {
+            walk(r, t, [&](uint32_t a, int hop) {
+                set(a);
+                if (line) line[depth - 1 - hop] = (int64_t)a;
+            });
+            if (t == 0) set((uint32_t)(lo + r));
+        }
+        if (line)
+            for (int l = max(depth, 0) + t; l < width; l += 1 << levels) line[l] = l == depth && insert_self ? lo + r : -1;
+    }
+    __syncthreads();
+    write_masks(out, j, lo, n_nodes, block_m, max_anc, mask_words, kept, bitmap, mbits, misc);
+    if (err && status) atomicOr(status, err);
+    if (err && host_flags) {      // (pinned host memory: plain stores, a word per flag)
+        if (err & FSTA_PRE_TOO_MANY_ANCESTORS) host_flags[0] = 1u;
+        if (err & FSTA_PRE_BAD_NODE_ID) host_flags[1] = 1u;
+        if (err & FSTA_PRE_BAD_LEVEL) host_flags[2] = 1u;
+    }
 }
 
 constexpr int kPackMaxTiles = 512;   // ancestor tiles a block plan written by pack_mask_kernel can have
@@ -481,6 +618,15 @@ __global__ __launch_bounds__(kThreads) void lineage_rows_kernel(
     if (err) atomicOr(status, err);
 }
 
+__global__ __launch_bounds__(kThreads) void shift_index_kernel(const int64_t* __restrict__ a, int64_t n_a, const int64_t* __restrict__ b,
+                                                               int64_t n_b, int64_t shift, int64_t* __restrict__ out_a,
+                                                               int64_t* __restrict__ out_b) {
+    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i >= n_a + n_b) return;
+    const int64_t v = i < n_a ? a[i] : b[i - n_a];
+    (i < n_a ? out_a[i] : out_b[i - n_a]) = v >= 0 ? v + shift : v;
+}
+
 }  // namespace
 }  // namespace fsta
 
@@ -531,8 +677,8 @@ extern "C" int fsta_precompute(int64_t* lineage, const int64_t* level_lookup, in
     const int threads = entries >= 2048 || (size_t)block_m * max_ancestors >= 8192 ? kMaxThreads : kThreads;
     hipLaunchKernelGGL(block_precompute_kernel, dim3((unsigned)nb), dim3(threads), lds,
                        static_cast<hipStream_t>(stream), lineage, level_lookup, n_nodes, width,
-                       block_m, max_ancestors, mask_words, mutate_lineage, staged, ancestor_idx,
-                       ancestor_mask, leaf_idx, mask_bits, anc_count, block_plan, nullptr, status);
+                       block_m, max_ancestors, mask_words, mutate_lineage, staged,
+                       BlockOutputs{ancestor_idx, ancestor_mask, leaf_idx, mask_bits, anc_count, block_plan}, status);
     FSTA_HIP_OK(hipGetLastError());
     return FSTA_OK;
 }
@@ -542,38 +688,73 @@ extern "C" int fsta_precompute_from_parents(const int64_t* parent, int64_t n_nod
                                             int64_t* level_lookup, int64_t* ancestor_idx, uint8_t* ancestor_mask,
                                             int64_t* leaf_idx, uint32_t* mask_bits, int32_t* anc_count,
                                             uint32_t* block_plan, uint32_t* status, void* stream) {
+    if (n_nodes > 0 && !status) return fail(FSTA_EINVAL, "fsta_precompute_from_parents: null pointer");
+    return fsta_precompute_from_parents_flags(parent, n_nodes, width, block_m, max_ancestors, insert_self, lineage, level_lookup,
+                                              ancestor_idx, ancestor_mask, leaf_idx, mask_bits, anc_count, block_plan, status,
+                                              nullptr, stream);
+}
+
+extern "C" int fsta_precompute_from_parents_flags(const int64_t* parent, int64_t n_nodes, int64_t width, int32_t block_m,
+                                                  int32_t max_ancestors, int32_t insert_self, int64_t* lineage,
+                                                  int64_t* level_lookup, int64_t* ancestor_idx, uint8_t* ancestor_mask,
+                                                  int64_t* leaf_idx, uint32_t* mask_bits, int32_t* anc_count,
+                                                  uint32_t* block_plan, uint32_t* status, uint32_t* host_flags, void* stream) {
     if (n_nodes < 0 || width < 1 || block_m < 1 || max_ancestors < 1)
         return fail(FSTA_EINVAL, "fsta_precompute_from_parents: n_nodes=%lld width=%lld block_m=%d max_ancestors=%d",
                     (long long)n_nodes, (long long)width, block_m, max_ancestors);
     if (n_nodes == 0) return FSTA_OK;
-    if (!parent || !ancestor_idx || !leaf_idx || !status) return fail(FSTA_EINVAL, "fsta_precompute_from_parents: null pointer");
+    if (!parent || !ancestor_idx || !leaf_idx || (!status && !host_flags))
+        return fail(FSTA_EINVAL, "fsta_precompute_from_parents: null pointer");
     if (block_m > 4096) return fail(FSTA_EUNSUPPORTED, "fsta_precompute_from_parents: block_m=%d > 4096", block_m);
     if (block_plan && !plan_block_size_ok(block_m))
         return fail(FSTA_EINVAL, "fsta_precompute_from_parents: a block plan needs block_m 32, 64 or 128 (got %d)", block_m);
     if (misaligned(parent, 8) || misaligned(lineage, 8) || misaligned(level_lookup, 8) || misaligned(ancestor_idx, 8) ||
         misaligned(leaf_idx, 8))
         return fail(FSTA_EINVAL, "fsta_precompute_from_parents: parent, lineage, level_lookup, ancestor_idx and leaf_idx must be 8-byte aligned");
-    if (misaligned(mask_bits, 4) || misaligned(anc_count, 4) || misaligned(status, 4) || misaligned(block_plan, 16))
-        return fail(FSTA_EINVAL, "fsta_precompute_from_parents: mask_bits, anc_count and status must be 4-byte aligned, block_plan 16-byte");
+    if (misaligned(mask_bits, 4) || misaligned(anc_count, 4) || misaligned(status, 4) || misaligned(host_flags, 4) ||
+        misaligned(block_plan, 16))
+        return fail(FSTA_EINVAL, "fsta_precompute_from_parents: mask_bits, anc_count, status and host_flags must be 4-byte aligned, block_plan 16-byte");
     const int mask_words = fsta_mask_words(max_ancestors);
     const int64_t n_words = (n_nodes + 31) >> 5;
-    // tables, the block's rows and the parent array, all in one workgroup's LDS
-    const double need = 4.0 * ((double)precompute_lds_words(n_words, mask_words, block_m) + (double)block_m * (double)width + (double)n_nodes);
+    const double tables = 4.0 * (double)precompute_lds_words(n_words, mask_words, block_m);
+    const double need = tables + 4.0 * ((double)block_m * (double)width + (double)n_nodes);      // (the documented limit)
     if (need > 160.0 * 1024)
         return fail(FSTA_EUNSUPPORTED, "fsta_precompute_from_parents: n_nodes=%lld width=%lld block_m=%d max_ancestors=%d need %.0f "
                     "bytes of LDS (limit 163840): fsta_lineage_from_parents + fsta_precompute take any size",
                     (long long)n_nodes, (long long)width, block_m, max_ancestors, need);
-    const size_t lds = (size_t)need;
+    // Lanes per row: doubling costs a barrier per level, a walk levels + depth / 2^levels dependent reads, twice; rows of
+    // `width` columns are 2^levels = sqrt(width) lanes' work, as far as the workgroup has lanes and LDS for the tables
+    // (with one level they are as large as the limit above allows for; n_nodes < 2^16 - 1 follows from it).
+    int levels = 0;
+    while (levels < kMaxLevels && (int64_t)1 << (2 * levels + 2) <= width && (block_m << (levels + 1)) <= kMaxThreads &&
+           tables + 2.0 * (levels + 2) * (double)(n_nodes + 1) <= 160.0 * 1024)
+        ++levels;
+    const size_t lds = (size_t)tables + 2u * (size_t)(levels + 1) * (size_t)((n_nodes + 1) & ~(int64_t)1);
     if (lds > 64 * 1024) {
-        const int rc = allow_full_lds<&block_precompute_kernel>();
+        const int rc = allow_full_lds<&block_from_parents_kernel>();
         if (rc != FSTA_OK) return rc;
     }
     const int64_t nb = (n_nodes + block_m - 1) / block_m;
-    const size_t entries = (size_t)block_m * (size_t)width;
-    const int threads = entries >= 2048 || (size_t)block_m * max_ancestors >= 8192 || n_nodes >= 2048 ? kMaxThreads : kThreads;
-    hipLaunchKernelGGL(block_precompute_kernel, dim3((unsigned)nb), dim3(threads), lds, static_cast<hipStream_t>(stream), lineage,
-                       level_lookup, n_nodes, width, block_m, max_ancestors, mask_words, insert_self ? 1 : 0, 1, ancestor_idx,
-                       ancestor_mask, leaf_idx, mask_bits, anc_count, block_plan, parent, status);
+    const int threads = (block_m << levels) > kThreads || (size_t)block_m * max_ancestors >= 8192 || n_nodes >= 2048 ? kMaxThreads : kThreads;
+    hipLaunchKernelGGL(block_from_parents_kernel, dim3((unsigned)nb), dim3(threads), lds, static_cast<hipStream_t>(stream), parent,
+                       (int)n_nodes, (int)width, block_m, max_ancestors, mask_words, levels, insert_self ? 1 : 0, lineage, level_lookup,
+                       BlockOutputs{ancestor_idx, ancestor_mask, leaf_idx, mask_bits, anc_count, block_plan}, status, host_flags);
+    FSTA_HIP_OK(hipGetLastError());
+    return FSTA_OK;
+}
+
+// out = in + shift where in >= 0, for two index arrays in one launch
+extern "C" int fsta_shift_index(const int64_t* a, int64_t n_a, const int64_t* b, int64_t n_b, int64_t shift, int64_t* out_a,
+                                int64_t* out_b, void* stream) {
+    if (n_a < 0 || n_b < 0 || n_a + n_b > (int64_t)0x7fffffff * kThreads)
+        return fail(FSTA_EINVAL, "fsta_shift_index: n_a=%lld n_b=%lld", (long long)n_a, (long long)n_b);
+    if (n_a + n_b == 0) return FSTA_OK;
+    if ((n_a && (!a || !out_a)) || (n_b && (!b || !out_b))) return fail(FSTA_EINVAL, "fsta_shift_index: null pointer");
+    if (misaligned(a, 8) || misaligned(b, 8) || misaligned(out_a, 8) || misaligned(out_b, 8))
+        return fail(FSTA_EINVAL, "fsta_shift_index: the arrays must be 8-byte aligned");
+    const unsigned grid = (unsigned)((n_a + n_b + kThreads - 1) / kThreads);
+    hipLaunchKernelGGL(shift_index_kernel, dim3(grid), dim3(kThreads), 0, static_cast<hipStream_t>(stream), a, n_a, b, n_b, shift,
+                       out_a, out_b);
     FSTA_HIP_OK(hipGetLastError());
     return FSTA_OK;
 }

@@ -7,10 +7,17 @@
 #include <Python.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <pybind11/pybind11.h>
+
+#include <cstring>
 
 #include "../../include/fsta.h"
 #include "fsta_torch.h"
@@ -161,6 +168,172 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
 }
 
+// ---- front-end of a decoding step (integer work; outputs are new tensors, arguments are checked in precompute.py) -------
+// A return code of the library other than FSTA_OK comes back as a Python int.
+
+const at::Tensor& tensor_arg(PyObject* o) {
+    TORCH_CHECK_TYPE(THPVariable_Check(o), "expected a torch.Tensor");
+    return THPVariable_Unpack(o);
+}
+
+int64_t int_arg(PyObject* o) {
+    int64_t v;
+    TORCH_CHECK_TYPE(as_int(o, &v), "expected an int");
+    return v;
+}
+
+struct OnStream {      // the tensors' device and torch's current stream on it
+    explicit OnStream(const at::Tensor& t)
+        : guard(t.device()), stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream()) {}
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard;
+    const hipStream_t stream;
+};
+
+// The status word of a call: the caller's, or a zeroed one when somebody is going to look at it, or one nobody reads
+at::Tensor status_word(PyObject* given, bool read, const at::Tensor& like) {
+    if (given != Py_None) return tensor_arg(given);
+    const auto i32 = like.options().dtype(at::kInt);
+    return read ? at::zeros({1}, i32) : at::empty({1}, i32);
+}
+
+template <class... T> PyObject* as_tuple(const T&... tensors) {      // undefined tensors become None
+    PyObject* tuple = PyTuple_New(sizeof...(T));
+    if (!tuple) return nullptr;
+    Py_ssize_t i = 0;
+    auto put = [&](const at::Tensor& t) {
+        PyObject* o = t.defined() ? THPVariable_Wrap(t) : (Py_INCREF(Py_None), Py_None);
+        PyTuple_SET_ITEM(tuple, i++, o);
+        return o != nullptr;
+    };
+    if ((put(tensors) && ...)) return tuple;
+    Py_DECREF(tuple);
+    return nullptr;
+}
+
+template <class T> T* data_or_null(const at::Tensor& t) { return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr; }
+
+// dfs_order(parent, light_first, read_status, status or None) -> (perm, rank, status)
+PyObject* dfs_order(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n_args == 4, "dfs_order takes 4 arguments");
+    const at::Tensor parent = tensor_arg(args[0]).contiguous();
+    const OnStream on(parent);
+    const int64_t n = parent.size(0);
+    at::Tensor perm = at::empty({n}, parent.options()), rank = at::empty({n}, parent.options());
+    at::Tensor work = at::empty({(int64_t)FSTA_DFS_ORDER_WORKSPACE_INTS(n)}, parent.options().dtype(at::kInt));
+    at::Tensor status = status_word(args[3], args[2] == Py_True, parent);
+    const int rc = fsta_dfs_order(parent.data_ptr<int64_t>(), n, args[1] == Py_True, perm.data_ptr<int64_t>(), rank.data_ptr<int64_t>(),
+                                  work.data_ptr<int32_t>(), static_cast<uint32_t*>(status.data_ptr()), on.stream);
+    return rc != FSTA_OK ? PyLong_FromLong(rc) : as_tuple(perm, rank, status);
+    END_HANDLE_TH_ERRORS
+}
+
+// renumber_parents(parent, rank) -> new_parent
+PyObject* renumber_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n_args == 2, "renumber_parents takes 2 arguments");
+    const at::Tensor parent = tensor_arg(args[0]).contiguous(), rank = tensor_arg(args[1]).contiguous();
+    const OnStream on(parent);
+    at::Tensor out = at::empty(parent.sizes(), parent.options());
+    const int rc = fsta_renumber_parents(parent.data_ptr<int64_t>(), rank.data_ptr<int64_t>(), parent.size(0), out.data_ptr<int64_t>(),
+                                         on.stream);
+    return rc != FSTA_OK ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
+// inputs_from_parents(parent, block_m, max_ancestors, width, check, want_bool_mask, want_lineage, status or None)
+//   -> (ancestor_idx, ancestor_mask, leaf_idx, mask_bits, anc_count, plan, lineage, level_lookup, status), bits
+// `check` (then no status word is used or returned): waits for the stream, bits are the FSTA_PRE_* conditions; else 0
+PyObject* inputs_from_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n_args == 8, "inputs_from_parents takes 8 arguments");
+    const at::Tensor parent = tensor_arg(args[0]).contiguous();
+    const int64_t n = parent.size(0), block_m = int_arg(args[1]), max_anc = int_arg(args[2]), width = int_arg(args[3]);
+    const bool check = args[4] == Py_True, want_mask = args[5] == Py_True, want_lineage = args[6] == Py_True;
+    TORCH_CHECK_VALUE(block_m > 0 && block_m <= INT32_MAX && max_anc > 0 && max_anc <= INT32_MAX && width > 0,
+                      "block_m, max_ancestors and width must be positive");
+    const OnStream on(parent);
+    const int64_t nb = (n + block_m - 1) / block_m;
+    const auto i64 = parent.options();
+    const auto i32 = parent.options().dtype(at::kInt);
+    at::Tensor a_idx = at::empty({nb, max_anc}, i64), l_idx = at::empty({nb, block_m}, i64), a_mask, lineage, level, plan;
+    if (want_mask) a_mask = at::empty({nb, block_m, max_anc}, parent.options().dtype(at::kBool));
+    at::Tensor bits = at::empty({nb, (int64_t)fsta_mask_words((int32_t)max_anc), block_m}, i32), count = at::empty({nb}, i32);
+    const size_t plan_bytes = fsta_block_plan_bytes((int32_t)nb, (int32_t)block_m, (int32_t)max_anc);
+    if (plan_bytes) plan = at::empty({(int64_t)(plan_bytes / 4)}, i32);
+    if (want_lineage) {
+        lineage = at::empty({n, width}, i64);
+        level = at::empty({n}, i64);
+    }
+    // A caller that waits is told through pinned host memory; a word in device memory is for those that look later.
+    at::Tensor flags, status;
+    if (check) {
+        flags = at::empty({3}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        memset(flags.data_ptr(), 0, 3 * sizeof(int32_t));
+    }
+    if (!check) status = status_word(args[7], true, parent);
+    const int rc = fsta_precompute_from_parents_flags(
+        parent.data_ptr<int64_t>(), n, width, (int32_t)block_m, (int32_t)max_anc, 1, data_or_null<int64_t>(lineage),
+        data_or_null<int64_t>(level), a_idx.data_ptr<int64_t>(), data_or_null<uint8_t>(a_mask), l_idx.data_ptr<int64_t>(),
+        static_cast<uint32_t*>(bits.data_ptr()), count.data_ptr<int32_t>(), data_or_null<uint32_t>(plan),
+        data_or_null<uint32_t>(status), data_or_null<uint32_t>(flags), on.stream);
+    if (rc != FSTA_OK) return PyLong_FromLong(rc);
+    long found = 0;
+    if (check) {
+        hipError_t err;
+        {
+            pybind11::gil_scoped_release no_gil;
+            err = hipStreamSynchronize(on.stream);
+        }
+        TORCH_CHECK(err == hipSuccess, "kernel_inputs_from_parents_gpu: ", hipGetErrorString(err));
+        const volatile int32_t* word = flags.data_ptr<int32_t>();
+        found = (word[0] ? FSTA_PRE_TOO_MANY_ANCESTORS : 0) | (word[1] ? FSTA_PRE_BAD_NODE_ID : 0) | (word[2] ? FSTA_PRE_BAD_LEVEL : 0);
+    }
+    PyObject* tensors = as_tuple(a_idx, a_mask, l_idx, bits, count, plan, lineage, level, status);
+    return tensors ? Py_BuildValue("Nl", tensors, found) : nullptr;
+    END_HANDLE_TH_ERRORS
+}
+
+// medusa_parents(probs, n, read_status, status or None) -> (parent, status)
+PyObject* medusa_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n_args == 4, "medusa_parents takes 4 arguments");
+    const at::Tensor probs = tensor_arg(args[0]).contiguous();
+    const int64_t n = int_arg(args[1]);
+    const OnStream on(probs);
+    const int32_t depths = (int32_t)probs.size(0), topk = (int32_t)probs.size(1);
+    const int32_t code = probs.scalar_type() == at::kFloat ? FSTA_F32 : FSTA_F64;
+    at::Tensor parent = at::empty({n}, probs.options().dtype(at::kLong));
+    at::Tensor status = status_word(args[3], args[2] == Py_True, probs);
+    const size_t need = fsta_medusa_workspace_bytes(depths, topk);
+    at::Tensor work;      // (stream-ordered: free again after the launches)
+    if (need) work = at::empty({(int64_t)need}, probs.options().dtype(at::kByte));
+    uint32_t* word = static_cast<uint32_t*>(status.data_ptr());
+    const int rc = need ? fsta_medusa_tree_ws(probs.data_ptr(), code, depths, topk, (int32_t)n, parent.data_ptr<int64_t>(), word,
+                                              work.data_ptr(), need, on.stream)
+                        : fsta_medusa_tree(probs.data_ptr(), code, depths, topk, (int32_t)n, parent.data_ptr<int64_t>(), word, on.stream);
+    return rc != FSTA_OK ? PyLong_FromLong(rc) : as_tuple(parent, status);
+    END_HANDLE_TH_ERRORS
+}
+
+// shift_index(ancestor_idx, leaf_idx, shift) -> both with `shift` added to the entries that are not negative; NotImplemented
+// for anything but ordinary int64 tensors on one GPU
+PyObject* shift_index(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    if (n_args != 3 || !plain_context()) return not_implemented();
+    const at::Tensor *a = gpu_tensor(args[0]), *b = gpu_tensor(args[1]);
+    int64_t shift;
+    if (!a || !b || a->scalar_type() != at::kLong || b->scalar_type() != at::kLong || a->device() != b->device() || !as_int(args[2], &shift))
+        return not_implemented();
+    const at::Tensor ac = a->contiguous(), bc = b->contiguous();
+    const OnStream on(ac);
+    at::Tensor out_a = at::empty(ac.sizes(), ac.options()), out_b = at::empty(bc.sizes(), bc.options());
+    const int rc = fsta_shift_index(ac.data_ptr<int64_t>(), ac.numel(), bc.data_ptr<int64_t>(), bc.numel(), shift,
+                                    out_a.data_ptr<int64_t>(), out_b.data_ptr<int64_t>(), on.stream);
+    return rc != FSTA_OK ? not_implemented() : as_tuple(out_a, out_b);
+    END_HANDLE_TH_ERRORS
+}
+
 // setup(PackedTreeMask, packed_table)
 PyObject* setup(PyObject*, PyObject* args) {
     PyObject *type, *table;
@@ -172,8 +345,14 @@ PyObject* setup(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
+#define FSTA_FASTCALL(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&f)), METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {
-    {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&attention)), METH_FASTCALL, nullptr},
+    FSTA_FASTCALL(attention),
+    FSTA_FASTCALL(dfs_order),
+    FSTA_FASTCALL(renumber_parents),
+    FSTA_FASTCALL(inputs_from_parents),
+    FSTA_FASTCALL(medusa_parents),
+    FSTA_FASTCALL(shift_index),
     {"setup", &setup, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

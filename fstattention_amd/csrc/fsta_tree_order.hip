@@ -2,7 +2,7 @@
 //
 // The reference leaves "DFS ordering so that the nodes of a block share lineage" as an open
 // item (README.md:19-20); the host version is trees.dfs_order.  Integer work: one launch of one
-// workgroup for the trees of speculative decoding (a few thousand nodes), six launches of N
+// workgroup for the trees of speculative decoding (up to 8192 nodes), six launches of N
 // threads for larger ones; siblings are found through per-parent child lists, not by a sort.
 //
 //   size[i]  nodes in the subtree of i                     (every node adds 1 to each ancestor)
@@ -175,101 +175,191 @@ __global__ __launch_bounds__(kOrderThreads) void order_finish_kernel(const int64
     rank[i] = pre;
 }
 
-// Trees of a few thousand nodes (what speculative decoding builds) in ONE workgroup and launch:
-// the four steps above with every array in LDS, so that a hop or a sibling visit is an LDS
-// access and the steps are separated by barriers instead of kernel boundaries.  Siblings are
-// found through per-parent child lists (built with atomic exchanges) instead of the all-pairs
-// loop: a node visits its parent's other children only.  A list is a chain of dependent reads,
-// so children of a parent with more than kListedChildren of them (no tree of speculative decoding
-// has such nodes) scan the whole node array instead, whose reads are independent.
-// (Tried and dropped: path sums by pointer doubling and sizes level by level.  Fewer dependent
-// hops, but every round ends in a barrier of 16 waves, which costs more than the hops it saves
-// on trees up to 160 levels deep.)
+// Trees of a few thousand nodes (what speculative decoding builds) in ONE workgroup and launch, every array in LDS.
+// What bounds it is the length of dependent chains: the sums over paths go by pointer doubling (log2(depth) rounds of one
+// or two barriers instead of `depth` dependent LDS reads, and all of a thread's nodes in the same round):
+//   size: after round k, size[v] counts the nodes less than 2^k levels below v; node u adds its size[u] to that of its
+//         2^k-th ancestor (two barriers: read, add)
+//   pre:  after round k, sum[v] covers v and its next 2^k - 1 ancestors; sum and ancestor travel in one word, between two
+//         buffers (one barrier)
+// Siblings are found through per-parent child lists (built with atomic exchanges): a node visits its parent's other
+// children only.  A list is a chain of dependent reads, so children of a parent with more than kListedChildren of them (no
+// tree of speculative decoding has such nodes) scan the whole node array instead, whose reads are independent.
+// 2048 nodes, 100 levels: 27 us with a walk to the root per node for either sum.
 constexpr int kSmallThreads = 1024;
-constexpr int kSmallMaxNodes = 4096;   // 6 int32 arrays of n (+1) entries: 96 KB of LDS
+constexpr int kSmallMaxNodes = 8192;   // 18 bytes of LDS a node: 147 KB
 constexpr int kListedChildren = 64;
+constexpr int kMaxRounds = 16;
 
+__host__ __device__ inline size_t order_small_words(int n) {
+    const int half = (n + 2) / 2;      // 16-bit arrays of n (+ 1) entries, in words
+    return (size_t)(2 * n) + (size_t)(n + 1) + (size_t)(3 * half) + kMaxRounds;
+}
+
+template <int NPT>      // nodes per thread
 __global__ __launch_bounds__(kSmallThreads) void order_small_kernel(const int64_t* __restrict__ parent, int n,
                                                                     int light_first, int64_t* __restrict__ perm,
                                                                     int64_t* __restrict__ rank,
                                                                     uint32_t* __restrict__ status) {
     asm volatile("" ::"s"(parent), "s"(n), "s"(light_first), "s"(perm), "s"(rank), "s"(status));   // one batch of argument loads
     extern __shared__ int32_t small_s[];
-    int32_t* par_s = small_s;          // [n]   parent, -1 for roots
-    int32_t* size_s = par_s + n;       // [n]   nodes in the subtree
-    int32_t* off_s = size_s + n;       // [n]   sizes of the siblings visited earlier
-    int32_t* next_s = off_s + n;       // [n]   next child of the same parent
-    int32_t* head_s = next_s + n;      // [n+1] first child; entry n: the roots
-    int32_t* kids_s = head_s + n + 1;  // [n+1] number of children
-    int32_t* bad_s = kids_s + n + 1;   // [1]   malformed input
+    const int half = (n + 2) / 2;
+    int32_t* jump_s = small_s;              // [n]   2^round-th ancestor, -1 above the root; later path sums
+    int32_t* size_s = jump_s + n;           // [n]   nodes in the subtree; later path sums
+    int32_t* head_s = size_s + n;           // [n+1] first child; entry n: the roots
+    int32_t* kids_s = head_s + n + 1;       // [n+1] number of children, 16 bits each
+    uint16_t* next_s = reinterpret_cast<uint16_t*>(kids_s + half);         // [n] next child of the same parent, 0xffff: none
+    uint16_t* par_s = reinterpret_cast<uint16_t*>(kids_s + 2 * half);      // [n] parent, n for roots
+    int32_t* alive_s = kids_s + 3 * half;   // [kMaxRounds] some node still has an ancestor that far up; the last: malformed input
     const int tid = threadIdx.x;
-    if (tid == 0) *bad_s = 0;
-    for (int i = tid; i <= n; i += kSmallThreads) {
-        head_s[i] = -1;
-        kids_s[i] = 0;
+    const int threads = blockDim.x;
+    int64_t given[NPT];
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+        const int i = tid + k * threads;
+        given[k] = i < n ? parent[i] : -1;
     }
+    for (int i = tid; i <= n; i += threads) head_s[i] = -1;
+    for (int i = tid; i < half; i += threads) kids_s[i] = 0;
+    if (tid < kMaxRounds) alive_s[tid] = 0;
     __syncthreads();
-    for (int i = tid; i < n; i += kSmallThreads) {
-        const int64_t p = parent[i];
-        const bool ok = p >= -1 && p < i;     // every hop goes to a smaller id: the walks end
-        par_s[i] = ok ? (int32_t)p : -1;
+    int32_t up[NPT];         // the node's 2^round-th ancestor
+    bool more = false, bad = false;
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+        const int i = tid + k * threads;
+        if (i >= n) { up[k] = -1; continue; }
+        const bool ok = given[k] >= -1 && given[k] < i;     // every hop goes to a smaller id: the doubling ends
+        bad |= !ok;
+        up[k] = ok ? (int32_t)given[k] : -1;
+        more |= up[k] >= 0;
+        const int32_t p = up[k] >= 0 ? up[k] : n;
+        jump_s[i] = up[k];
         size_s[i] = 1;
-        if (!ok) *bad_s = 1;
+        par_s[i] = (uint16_t)p;
+        next_s[i] = (uint16_t)atomicExch(&head_s[p], i);
+        atomicAdd(&kids_s[p >> 1], (p & 1) ? 0x10000 : 1);
     }
+    if (more) alive_s[0] = 1;
+    if (bad) alive_s[kMaxRounds - 1] = 1;
     __syncthreads();
-    if (*bad_s) {      // malformed parent array: identity, the caller reads the status word
-        for (int i = tid; i < n; i += kSmallThreads) {
+    if (alive_s[kMaxRounds - 1]) {      // malformed parent array: identity, the caller reads the status word
+        for (int i = tid; i < n; i += threads) {
             perm[i] = i;
             rank[i] = i;
         }
         if (tid == 0) atomicOr(status, FSTA_PRE_BAD_NODE_ID);
         return;
     }
-    for (int i = tid; i < n; i += kSmallThreads) {
-        const int32_t p = par_s[i];
-        next_s[i] = atomicExch(&head_s[p >= 0 ? p : n], i);
-        atomicAdd(&kids_s[p >= 0 ? p : n], 1);
-        // Every node adds 1 to each of its ancestors.  Nodes with neighbouring ids meet after a
-        // few hops: where all lanes of the wave that are still walking stand on the same node,
-        // one of them adds for all (otherwise the adds of a shallow tree queue up at its root).
-        for (int32_t a = p; a >= 0; a = par_s[a]) {
-            const uint64_t walking = __ballot(true);
-            const int32_t first = __builtin_amdgcn_readfirstlane(a);
-            if (__ballot(a != first) == 0ull) {
-                if ((tid & 63) == __ffsll((long long)walking) - 1) atomicAdd(&size_s[first], __popcll(walking));
-            } else {
-                atomicAdd(&size_s[a], 1);
+    int rounds = 0;
+    while (alive_s[rounds]) {           // (at most 13 rounds for 8192 nodes)
+        int32_t below[NPT], next_up[NPT];
+#pragma unroll
+        for (int k = 0; k < NPT; ++k)
+            if (up[k] >= 0) {
+                below[k] = size_s[tid + k * threads];
+                next_up[k] = jump_s[up[k]];
             }
-        }
+        __syncthreads();
+        more = false;
+#pragma unroll
+        for (int k = 0; k < NPT; ++k)
+            if (up[k] >= 0) {
+                atomicAdd(&size_s[up[k]], below[k]);
+                jump_s[tid + k * threads] = next_up[k];
+                up[k] = next_up[k];
+                more |= up[k] >= 0;
+            }
+        ++rounds;
+        if (more) alive_s[rounds] = 1;
+        __syncthreads();
     }
-    __syncthreads();
-    for (int i = tid; i < n; i += kSmallThreads) {
+    int32_t key[NPT], at[NPT], before[NPT];     // order key, position in the child list, sizes of the siblings visited earlier
+    bool walking = false;
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+        const int i = tid + k * threads;
+        at[k] = 0xffff;
+        before[k] = key[k] = 0;
+        if (i >= n) continue;
         const int32_t p = par_s[i];
-        const int32_t my_key = light_first ? (size_s[i] << 13) | i : i;    // sizes and ids are below 2^13
-        int32_t acc = 0;
-        if (kids_s[p >= 0 ? p : n] <= kListedChildren) {
-            for (int32_t s = head_s[p >= 0 ? p : n]; s >= 0; s = next_s[s]) {
-                const int32_t sz = size_s[s];
-                const int32_t key = light_first ? (sz << 13) | s : s;
-                acc += key < my_key ? sz : 0;
-            }
+        key[k] = light_first ? (size_s[i] << 14) | i : i;    // ids are below 2^14, sizes at most 2^13
+        const int32_t kids = (kids_s[p >> 1] >> ((p & 1) * 16)) & 0xffff;
+        if (kids <= kListedChildren) {
+            at[k] = head_s[p];
+            walking = true;
         } else {
 #pragma unroll 4
             for (int32_t s = 0; s < n; ++s) {
                 const int32_t sz = size_s[s];
-                const int32_t key = light_first ? (sz << 13) | s : s;
-                acc += (par_s[s] == p && key < my_key) ? sz : 0;
+                const int32_t other = light_first ? (sz << 14) | s : s;
+                before[k] += (par_s[s] == p && other < key[k]) ? sz : 0;
             }
         }
-        off_s[i] = acc;
+    }
+    while (walking) {       // (the lists of a thread's nodes side by side)
+        walking = false;
+#pragma unroll
+        for (int k = 0; k < NPT; ++k)
+            if (at[k] != 0xffff) {
+                const int32_t sz = size_s[at[k]], next = next_s[at[k]];
+                const int32_t other = light_first ? (sz << 14) | at[k] : at[k];
+                before[k] += other < key[k] ? sz : 0;
+                at[k] = next;
+                walking |= next != 0xffff;
+            }
+    }
+    // path sums of (before + 1): ancestor + 1 in the upper, sum in the lower 16 bits of a word
+    uint32_t sum[NPT];
+    uint32_t* from = reinterpret_cast<uint32_t*>(jump_s);
+    uint32_t* to = reinterpret_cast<uint32_t*>(size_s);
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+        const int i = tid + k * threads;
+        if (i >= n) { sum[k] = 0u; continue; }
+        const uint32_t p = par_s[i];
+        sum[k] = ((p == (uint32_t)n ? 0u : p + 1u) << 16) | (uint32_t)(before[k] + 1);
+        from[i] = sum[k];
     }
     __syncthreads();
-    for (int i = tid; i < n; i += kSmallThreads) {
-        int32_t pre = -1;
-        for (int32_t cur = i; cur >= 0; cur = par_s[cur]) pre += off_s[cur] + 1;
+    for (int round = 0; round < rounds; ++round) {
+#pragma unroll
+        for (int k = 0; k < NPT; ++k) {
+            const uint32_t a = sum[k] >> 16;
+            if (a) {
+                const uint32_t other = from[a - 1u];
+                sum[k] = (other & 0xffff0000u) | ((sum[k] + other) & 0xffffu);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NPT; ++k)
+            if (tid + k * threads < n) to[tid + k * threads] = sum[k];
+        __syncthreads();
+        uint32_t* done = from;
+        from = to;
+        to = done;
+    }
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+        const int i = tid + k * threads;
+        if (i >= n) continue;
+        const int32_t pre = (int32_t)(sum[k] & 0xffffu) - 1;
         perm[pre] = i;
         rank[i] = pre;
     }
+}
+
+template <int NPT>
+int launch_order_small(const int64_t* parent, int n, int light_first, int64_t* perm, int64_t* rank, uint32_t* status, hipStream_t s) {
+    const size_t lds = order_small_words(n) * sizeof(int32_t);
+    if (lds > 64 * 1024) {
+        const int rc = allow_full_lds<&order_small_kernel<NPT>>();
+        if (rc != FSTA_OK) return rc;
+    }
+    const int threads = n >= kSmallThreads ? kSmallThreads : (n + 63) / 64 * 64;
+    hipLaunchKernelGGL(order_small_kernel<NPT>, dim3(1), dim3(threads), lds, s, parent, n, light_first ? 1 : 0, perm, rank, status);
+    FSTA_HIP_OK(hipGetLastError());
+    return FSTA_OK;
 }
 
 // new_parent[rank[i]] = rank[parent[i]]: the same forest with node i renamed rank[i]
@@ -308,15 +398,11 @@ namespace {
 int dfs_order_launch(const int64_t* parent, int64_t n_nodes, int32_t light_first, int64_t* perm, int64_t* rank,
                      int32_t* workspace, uint32_t* status, hipStream_t s) {
     if (n_nodes <= kSmallMaxNodes) {
-        const size_t lds = (size_t)(6 * n_nodes + 3) * sizeof(int32_t);
-        if (lds > 64 * 1024) {
-            const int rc = allow_full_lds<&order_small_kernel>();
-            if (rc != FSTA_OK) return rc;
-        }
-        hipLaunchKernelGGL(order_small_kernel, dim3(1), dim3(kSmallThreads), lds, s, parent, (int)n_nodes,
-                           light_first ? 1 : 0, perm, rank, status);
-        FSTA_HIP_OK(hipGetLastError());
-        return FSTA_OK;
+        const int n = (int)n_nodes;
+        if (n <= kSmallThreads) return launch_order_small<1>(parent, n, light_first, perm, rank, status, s);
+        if (n <= 2 * kSmallThreads) return launch_order_small<2>(parent, n, light_first, perm, rank, status, s);
+        if (n <= 4 * kSmallThreads) return launch_order_small<4>(parent, n, light_first, perm, rank, status, s);
+        return launch_order_small<8>(parent, n, light_first, perm, rank, status, s);
     }
     const int32_t n = (int32_t)n_nodes;
     int32_t* size = workspace;                 // [n]

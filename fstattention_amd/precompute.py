@@ -17,6 +17,18 @@ from .attention import PackedTreeMask, _cache_key, _on_device, _stream_ptr, reme
 MEDUSA_MAX_CANDIDATES = 1 << 24    # candidate paths the tree builder takes (16384 in one launch, more over a workspace)
 
 
+_CALLS = None
+
+
+def _calls():
+    """The module of plain C functions (``csrc/fsta_torch_python.cpp``): allocation of the outputs, device guard, current
+    stream and launch without a page of Python per call."""
+    global _CALLS
+    _lib.load_torch_ops()
+    _CALLS = _lib.calls
+    return _CALLS
+
+
 def _raise_for_status(status: int, max_ancestors: int):
     if status & _lib.PRE_BAD_NODE_ID:
         raise ValueError("lineage holds a node id outside [-1, n_nodes)")
@@ -98,30 +110,16 @@ def kernel_inputs_from_parents_gpu(parent: torch.Tensor, block_m: int, max_ances
     workgroup's LDS (about 16000 nodes) raise ``libfsta``'s unsupported error: use the two calls."""
     if not parent.is_cuda or parent.dtype != torch.int64 or parent.dim() != 1:
         raise ValueError("parent must be a 1-D int64 tensor on the GPU")
-    lib = _lib.load()
-    parent = parent.contiguous()
-    dev = parent.device
-    n, block_m, max_ancestors, width = parent.shape[0], int(block_m), int(max_ancestors), int(width)
-    nb = -(-n // block_m)
-    a_idx = torch.empty((nb, max_ancestors), dtype=torch.int64, device=dev)
-    l_idx = torch.empty((nb, block_m), dtype=torch.int64, device=dev)
-    a_mask = torch.empty((nb, block_m, max_ancestors), dtype=torch.bool, device=dev) if want_bool_mask else None
-    bits = torch.empty((nb, lib.fsta_mask_words(max_ancestors), block_m), dtype=torch.int32, device=dev)
-    count = torch.empty((nb,), dtype=torch.int32, device=dev)
-    plan_bytes = lib.fsta_block_plan_bytes(nb, block_m, max_ancestors)
-    plan = torch.empty((plan_bytes // 4,), dtype=torch.int32, device=dev) if plan_bytes else None
-    lineage = torch.empty((n, width), dtype=torch.int64, device=dev) if want_lineage else None
-    level = torch.empty((n,), dtype=torch.int64, device=dev) if want_lineage else None
-    if status is None:
-        status = torch.zeros((1,), dtype=torch.int32, device=dev)
-    ptr = lambda t: t.data_ptr() if t is not None else None
-    with _on_device(dev):
-        _lib.check(lib.fsta_precompute_from_parents(parent.data_ptr(), n, width, block_m, max_ancestors, 1, ptr(lineage),
-                                                    ptr(level), a_idx.data_ptr(), ptr(a_mask), l_idx.data_ptr(),
-                                                    bits.data_ptr(), count.data_ptr(), ptr(plan), status.data_ptr(),
-                                                    _stream_ptr(dev)))
-    if check:
+    block_m, max_ancestors, width = int(block_m), int(max_ancestors), int(width)
+    # (without a status word of the caller's the outcome comes back with the wait for the stream)
+    out = (_CALLS or _calls()).inputs_from_parents(parent, block_m, max_ancestors, width, bool(check) and status is None,
+                                                   bool(want_bool_mask), bool(want_lineage), status)
+    if out.__class__ is int:
+        _lib.check(out)
+    (a_idx, a_mask, l_idx, bits, count, plan, lineage, level, status), st = out
+    if check and status is not None:
         st = int(status.item())
+    if st:
         if st & _lib.PRE_BAD_LEVEL:
             raise ValueError(f"tree is deeper than width={width}")
         if st & _lib.PRE_BAD_NODE_ID:
@@ -184,19 +182,10 @@ def dfs_order_gpu(parent: torch.Tensor, children: str = "index", check: bool = T
         raise ValueError("parent must be a 1-D int64 tensor on the GPU")
     if children not in ("index", "light_first"):
         raise ValueError(f"children={children!r}: expected 'index' or 'light_first'")
-    lib = _lib.load()
-    parent = parent.contiguous()
-    dev = parent.device
-    n = parent.shape[0]
-    perm = torch.empty((n,), dtype=torch.int64, device=dev)
-    rank = torch.empty((n,), dtype=torch.int64, device=dev)
-    work = torch.empty((_lib.dfs_order_workspace_ints(n),), dtype=torch.int32, device=dev)
-    if status is None:
-        status = torch.zeros((1,), dtype=torch.int32, device=dev)
-    with _on_device(dev):
-        _lib.check(lib.fsta_dfs_order(parent.data_ptr(), n, 1 if children == "light_first" else 0,
-                                      perm.data_ptr(), rank.data_ptr(), work.data_ptr(),
-                                      status.data_ptr(), _stream_ptr(dev)))
+    out = (_CALLS or _calls()).dfs_order(parent, children == "light_first", bool(check), status)
+    if out.__class__ is int:
+        _lib.check(out)
+    perm, rank, status = out
     if check and int(status.item()) & _lib.PRE_BAD_NODE_ID:
         raise ValueError("parent[i] must lie in [-1, i)")
     return perm, rank
@@ -207,13 +196,10 @@ def renumber_parents_gpu(parent: torch.Tensor, perm: torch.Tensor, rank: torch.T
     if not (parent.is_cuda and rank.is_cuda) or parent.dtype != torch.int64 or rank.dtype != torch.int64 or \
             parent.shape != rank.shape or parent.dim() != 1:
         raise ValueError("parent and rank must be 1-D int64 tensors of one length on the GPU")
-    lib = _lib.load()
-    parent, rank = parent.contiguous(), rank.contiguous()
-    new_parent = torch.empty_like(parent)
-    with _on_device(parent.device):
-        _lib.check(lib.fsta_renumber_parents(parent.data_ptr(), rank.data_ptr(), parent.shape[0],
-                                             new_parent.data_ptr(), _stream_ptr(parent.device)))
-    return new_parent
+    out = (_CALLS or _calls()).renumber_parents(parent, rank)
+    if out.__class__ is int:
+        _lib.check(out)
+    return out
 
 
 def medusa_parents_gpu(probs: torch.Tensor, n: int, check: bool = False, status=None) -> torch.Tensor:
@@ -245,22 +231,10 @@ def medusa_parents_gpu(probs: torch.Tensor, n: int, check: bool = False, status=
                          f"{MEDUSA_MAX_CANDIDATES} and depths * topk <= 1024")
     if probs.dtype not in (torch.float32, torch.float64):
         probs = probs.to(torch.float64)
-    probs = probs.contiguous()
-    lib = _lib.load()
-    dev = probs.device
-    parent = torch.empty((n,), dtype=torch.int64, device=dev)
-    if status is None:
-        status = torch.zeros((1,), dtype=torch.int32, device=dev)
-    code = _lib.F32 if probs.dtype == torch.float32 else _lib.F64
-    need = lib.fsta_medusa_workspace_bytes(depths, topk)
-    with _on_device(dev):
-        if need:
-            work = torch.empty((need,), dtype=torch.uint8, device=dev)     # (stream-ordered: free again after the launches)
-            _lib.check(lib.fsta_medusa_tree_ws(probs.data_ptr(), code, depths, topk, n, parent.data_ptr(), status.data_ptr(),
-                                               work.data_ptr(), need, _stream_ptr(dev)))
-        else:
-            _lib.check(lib.fsta_medusa_tree(probs.data_ptr(), code, depths, topk, n, parent.data_ptr(), status.data_ptr(),
-                                            _stream_ptr(dev)))
+    out = (_CALLS or _calls()).medusa_parents(probs, int(n), bool(check), status)
+    if out.__class__ is int:
+        _lib.check(out)
+    parent, status = out
     if check and int(status.item()) & _lib.TREE_NOT_PREFIX_CLOSED:
         raise ValueError("the kept paths are not closed under prefixes (probabilities above 1 or not numbers)")
     return parent

@@ -280,8 +280,8 @@ int fsta_lineage_from_parents(const int64_t* parent, int64_t n_nodes, int64_t wi
 /*
  * fsta_lineage_from_parents and fsta_precompute in one launch, for the trees of a
  * decoding step that is rebuilt every step (README.md:15-16): every workgroup
- * copies parent[n_nodes] into its LDS, builds the lineage rows of its own query
- * block there (layout of utils.py:66-75, `width` columns) and goes on as
+ * copies the parent array into its LDS, walks there what would be the lineage rows
+ * of its own query block (layout of utils.py:66-75, `width` columns) and does what
  * fsta_precompute does (utils.py:104-129), without the lineage ever travelling
  * through memory.  Outputs and status bits are those of fsta_precompute on the
  * lineage of fsta_lineage_from_parents, bit for bit; lineage [n_nodes, width] and
@@ -289,8 +289,8 @@ int fsta_lineage_from_parents(const int64_t* parent, int64_t n_nodes, int64_t wi
  * with each node's id in its own level column when insert_self != 0 (what
  * fsta_precompute leaves in the caller's tensor).  A tree deeper than width - 1
  * sets FSTA_PRE_BAD_LEVEL, a parent entry outside [-1, i) FSTA_PRE_BAD_NODE_ID
- * (such a node counts as a root).  Everything lives in one workgroup's LDS:
- * 4 * (n_nodes + block_m * width) bytes beside fsta_precompute's tables, 160 KB in
+ * (such a node counts as a root).  Limit: fsta_precompute's tables and
+ * 4 * (n_nodes + block_m * width) bytes of LDS, 160 KB in
  * all -- about 16000 nodes at width 64, block_m 128; larger problems are refused
  * with FSTA_EUNSUPPORTED (use the two calls).  No counterpart in the reference.
  * Alignment as fsta_precompute; parent 8 bytes.
@@ -300,6 +300,29 @@ int fsta_precompute_from_parents(const int64_t* parent, int64_t n_nodes, int64_t
                                  int64_t* level_lookup, int64_t* ancestor_idx, uint8_t* ancestor_mask,
                                  int64_t* leaf_idx, uint32_t* mask_bits, int32_t* anc_count,
                                  uint32_t* block_plan, uint32_t* status, void* stream);
+
+/*
+ * The same for a caller that looks at the outcome before it goes on: besides (or,
+ * with status == NULL, instead of) the status word the conditions are reported in
+ * host_flags[3], pinned HOST memory that the device can write (hipHostMalloc),
+ * zeroed by the caller before the launch and read after synchronising with the
+ * stream: [0] FSTA_PRE_TOO_MANY_ANCESTORS, [1] FSTA_PRE_BAD_NODE_ID,
+ * [2] FSTA_PRE_BAD_LEVEL, each 0 or 1.  Spares the fill and the copy of a word in
+ * device memory.
+ */
+int fsta_precompute_from_parents_flags(const int64_t* parent, int64_t n_nodes, int64_t width, int32_t block_m,
+                                       int32_t max_ancestors, int32_t insert_self, int64_t* lineage,
+                                       int64_t* level_lookup, int64_t* ancestor_idx, uint8_t* ancestor_mask,
+                                       int64_t* leaf_idx, uint32_t* mask_bits, int32_t* anc_count,
+                                       uint32_t* block_plan, uint32_t* status, uint32_t* host_flags, void* stream);
+
+/*
+ * out = in + shift for the entries of two index arrays that are not negative, in one
+ * launch: ancestor_idx and leaf_idx for K/V laid out as [prefix | tree] (reference
+ * fstattention.py:211-212).  Either array may be empty (n 0, NULL).  8-byte aligned.
+ */
+int fsta_shift_index(const int64_t* a, int64_t n_a, const int64_t* b, int64_t n_b, int64_t shift, int64_t* out_a,
+                     int64_t* out_b, void* stream);
 
 /*
  * Depth-first (pre-order) renumbering of a forest, the node order the reference

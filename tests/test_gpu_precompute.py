@@ -392,3 +392,63 @@ def test_kernel_inputs_from_parents_in_one_launch():
     big = torch.from_numpy(trees.random_recursive_parents(60000, 6, 64)).cuda()
     with pytest.raises(_lib.FstaError, match="LDS"):
         kernel_inputs_from_parents_gpu(big, 128, 64, 64)
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 2048, 2049, 4097, 8191, 8192, 8193])
+def test_dfs_order_at_the_edges_of_the_one_workgroup_kernel(n):
+    """Nodes per thread 1, 2, 4, 8 and the first size of the six-launch way; a chain has the most rounds, a star the largest
+    family, a forest of short trees the most roots."""
+    shapes = [trees.random_recursive_parents(n, n, 32), np.arange(-1, n - 1, dtype=np.int64), np.zeros(n, dtype=np.int64),
+              np.arange(n, dtype=np.int64) // 3 - 1]
+    shapes[2][0] = -1
+    for parent in shapes:
+        want = trees.dfs_order(parent, "light_first")
+        perm, rank = dfs_order_gpu(torch.from_numpy(parent).cuda(), "light_first")
+        np.testing.assert_array_equal(perm.cpu().numpy(), want)
+        np.testing.assert_array_equal(rank.cpu().numpy()[want], np.arange(n))
+
+
+@pytest.mark.parametrize("width,n,block_m", [(1, 40, 32), (3, 100, 16), (4, 129, 32), (15, 300, 48), (16, 257, 64), (64, 2048, 128),
+                                             (255, 700, 64), (256, 2100, 32), (1000, 1000, 16), (9, 8200, 128)])
+def test_kernel_inputs_from_parents_by_lanes_per_row(width, n, block_m):
+    """Row widths on both sides of every change of the number of lanes that share a row (1 to 16), with a path of exactly
+    `width` - 1 ancestors; then the same tree in rows one column too narrow: flagged, those rows empty, the others as before."""
+    parent = trees.random_recursive_parents(n, width, max(2, 2 * n // max(width, 8)))
+    level = trees.levels_from_parents(parent)
+    parent[level >= width] = -1
+    parent[:min(width, n)] = np.arange(-1, min(width, n) - 1)
+    level = trees.levels_from_parents(parent)
+    parent[level >= width] = -1                      # (now at most width - 1 deep, and somewhere exactly that)
+    max_anc = trees.required_max_ancestors(parent, block_m, 16)
+    dev = torch.from_numpy(parent).cuda()
+    for w in (width, width - 1):
+        if w < 1:
+            continue
+        lineage, level = trees.lineage_from_parents(parent, min_width=width)
+        lin, lvl = lineage.numpy()[:, :w].copy(), level.numpy().copy()
+        too_deep = lvl >= w
+        lin[too_deep], lvl[too_deep] = -1, 0
+        *got, glin, glvl, status = kernel_inputs_from_parents_gpu(dev, block_m, max_anc, w, check=False, want_bool_mask=True,
+                                                                  want_lineage=True)
+        assert int(status.item()) == (4 if too_deep.any() else 0)
+        np.testing.assert_array_equal(glvl.cpu().numpy(), lvl)
+        if w == width:
+            want = tp.block_inputs(lin, lvl, block_m, max_anc)
+            _check(got, want)
+            np.testing.assert_array_equal(glin.cpu().numpy(), lin)
+        else:
+            np.testing.assert_array_equal((glin.cpu().numpy() == -1).all(axis=1), too_deep)
+        if w == width or not too_deep.any():
+            kernel_inputs_from_parents_gpu(dev, block_m, max_anc, w)
+        else:
+            with pytest.raises(ValueError, match="deeper"):
+                kernel_inputs_from_parents_gpu(dev, block_m, max_anc, w)
+
+
+def test_shift_for_prefix_on_device_and_host_tensors():
+    from fstattention_amd import shift_for_prefix
+    a = torch.randint(-1, 50, (3, 37))
+    b = torch.randint(-1, 50, (3, 16))
+    for x, y in ((a, b), (a.cuda(), b.cuda()), (a.cuda().t(), b.cuda()), (a.cuda()[:0], b.cuda())):
+        for got, src in zip(shift_for_prefix(x, y, 1000), (x, y)):
+            assert torch.equal(got, torch.where(src >= 0, src + 1000, src))
