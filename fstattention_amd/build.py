@@ -26,6 +26,7 @@ SOURCES = [
     "fsta_merge.hip",
     "fsta_quantize.hip",
     "fsta_attention_generic.hip",
+    "fsta_attention_f32.hip",
     "fsta_attention_mfma.hip",
     "fsta_attention_mfma16.hip",
     "fsta_attention_prefix.hip",
@@ -45,7 +46,7 @@ HIPCC_FLAGS = [
 # Kernels of these sources must keep everything in registers: a private array the compiler leaves
 # in scratch memory, or a spill, is reloaded through the same vmcnt queue their gather rings count on.
 NO_SCRATCH = ("fsta_attention_mfma16.hip", "fsta_attention_mfma.hip", "fsta_attention_prefix.hip",
-              "fsta_attention_cache.hip", "fsta_attention_stream.hip", "fsta_attention_generic.hip")
+              "fsta_attention_cache.hip", "fsta_attention_stream.hip", "fsta_attention_generic.hip", "fsta_attention_f32.hip")
 
 
 def _hipcc() -> str:

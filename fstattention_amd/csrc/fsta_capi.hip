@@ -379,6 +379,10 @@ extern "C" int fsta_attention_fwd_ws(const void* q, const void* k, const void* v
         // streams them and takes any length
         if (rc != FSTA_EUNSUPPORTED) return rc;
     }
+    if (dtype == FSTA_F32 && !(flags & FSTA_FLAG_GENERIC)) {
+        const int rc = launch_attention_f32(p, head_dim, s);
+        if (rc != FSTA_EUNSUPPORTED) return rc;
+    }
     return launch_attention_generic(p, dtype, head_dim, s);
 }
 

@@ -114,6 +114,8 @@ void note_launch(const LaunchNote& note);
 
 // launchers, one per translation unit
 int launch_attention_generic(const AttnParams& p, int dtype, int head_dim, hipStream_t stream);
+// float32 on the matrix cores, head_dim 64 / 128; FSTA_EUNSUPPORTED for the others
+int launch_attention_f32(const AttnParams& p, int head_dim, hipStream_t stream);
 int launch_attention_mfma(const AttnParams& p, int dtype, int head_dim, bool fast_pv,
                           hipStream_t stream);
 int launch_attention_mfma16(const AttnParams& p, int dtype, int head_dim, bool fast_pv,

@@ -955,3 +955,13 @@ def test_non_default_stream():
         o = fst_attention(*dev, 0.125, BLOCK_M=cfg.block_m, MAX_ANCESTORS=max_anc)
     s.synchronize()
     assert_close(o, want, torch.float32, "side stream")
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n,block_m,window,prefix", [(1, 16, None, 0), (17, 16, None, 0), (96, 32, 2, 0), (130, 64, 16, 0),
+                                                     (300, 128, None, 0), (200, 64, 3, 1), (64, 32, 8, 16), (77, 32, 8, 143), (40, 16, 4, 1000)])
+def test_float32_on_the_matrix_cores(d, n, block_m, window, prefix):
+    """No, one and several tiles of 16 keys per wave (4 and 8 waves), ragged last tiles, prefixes around a tile and of many
+    tiles per wave."""
+    parent = trees.random_recursive_parents(n, 50 + n, window=window)
+    run_tree(parent, block_m, 2, 3, d, torch.float32, n + prefix, prefix=prefix, want_kernel="attn_f32_kernel")
