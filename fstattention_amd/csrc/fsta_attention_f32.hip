@@ -59,7 +59,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
     const float* q_row = qb + (size_t)min(row0 + i, p.nq - 1) * D + 4 * g;
     f32x4 q[kQLoads];
 #pragma unroll
-    for (int s = 0; s < kQLoads; ++s) q[s] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(q_row + 16 * s));
+    for (int s = 0; s < kQLoads; ++s) q[s] = *reinterpret_cast<const f32x4*>(q_row + 16 * s);
 
     n_anc = min(max(__builtin_amdgcn_readfirstlane(n_anc), 0), p.max_anc);
     const int anc_tiles = (n_anc + kKeys - 1) / kKeys;
@@ -239,10 +239,12 @@ int launch_one(const AttnParams& p, hipStream_t stream) {
 
 int launch_attention_f32(const AttnParams& p, int head_dim, hipStream_t stream) {
     if (head_dim != 64 && head_dim != 128) return FSTA_EUNSUPPORTED;
-    // a wave per tile of the longest list the call allows for, as far as a workgroup goes
+    // Four waves, so that several workgroups share a CU and one's arithmetic lies under another's round trips, also where a
+    // wave then takes two or three tiles (eight waves for up to 8 tiles, 512 rows, 16 heads, head_dim 128: 18.6 us, four:
+    // 14.6; 4096 rows, 32 heads: 412, 310); eight once every wave of four would walk ten tiles (long prefixes).
     const int tiles = (p.max_anc + kKeys - 1) / kKeys + (p.prefix + kKeys - 1) / kKeys;
-    if (head_dim == 64) return tiles < 4 ? launch_one<64, 4>(p, stream) : launch_one<64, 8>(p, stream);
-    return tiles < 4 ? launch_one<128, 4>(p, stream) : launch_one<128, 8>(p, stream);
+    if (head_dim == 64) return tiles < 40 ? launch_one<64, 4>(p, stream) : launch_one<64, 8>(p, stream);
+    return tiles < 40 ? launch_one<128, 4>(p, stream) : launch_one<128, 8>(p, stream);
 }
 
 }  // namespace fsta
