@@ -312,7 +312,7 @@ def shift_for_prefix(ancestor_idx: torch.Tensor, leaf_idx: torch.Tensor, prefix:
     if packed is None:
         return shifted
     limit = None if packed.key_limit is None else packed.key_limit + prefix
-    return shifted + (packed._replace(key_shift=packed.key_shift + prefix, key_limit=limit),)
+    return shifted + (PackedTreeMask(*packed[:5], packed.key_shift + prefix, limit),)
 
 
 def merge_attention_states(o_a: torch.Tensor, lse_a: torch.Tensor, o_b: torch.Tensor, lse_b: torch.Tensor):

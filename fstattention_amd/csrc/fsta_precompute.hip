@@ -316,7 +316,7 @@ __global__ __launch_bounds__(kMaxThreads) void block_from_parents_kernel(
     uint32_t* rank_base = bitmap + n_words;
     uint32_t* mbits = rank_base + n_words;
     int32_t* lvl_s = reinterpret_cast<int32_t*>(mbits + (size_t)mask_words * block_m);
-    uint32_t* misc = reinterpret_cast<uint32_t*>(lvl_s + block_m);          // [0] a row is too deep, [2] total count, [3] a listed ancestor
+    uint32_t* misc = reinterpret_cast<uint32_t*>(lvl_s + block_m);          // [0] a row is too deep, [1] conditions met, [2] total count, [3] a listed ancestor
     uint16_t* jump = reinterpret_cast<uint16_t*>(misc + 4);                 // [levels + 1][stride]
     const int stride = (n_nodes + 1) & ~1;
 
@@ -447,14 +447,14 @@ __global__ __launch_bounds__(kMaxThreads) void block_from_parents_kernel(
         if (line)
             for (int l = max(depth, 0) + t; l < width; l += 1 << levels) line[l] = l == depth && insert_self ? lo + r : -1;
     }
+    if (err) atomicOr(&misc[1], err);
     __syncthreads();
-    write_masks(out, j, lo, n_nodes, block_m, max_anc, mask_words, kept, bitmap, mbits, misc);
-    if (err && status) atomicOr(status, err);
-    if (err && host_flags) {      // (pinned host memory: plain stores, a word per flag)
-        if (err & FSTA_PRE_TOO_MANY_ANCESTORS) host_flags[0] = 1u;
-        if (err & FSTA_PRE_BAD_NODE_ID) host_flags[1] = 1u;
-        if (err & FSTA_PRE_BAD_LEVEL) host_flags[2] = 1u;
+    if (tid == 0) {
+        if (status && misc[1]) atomicOr(status, misc[1]);
+        // (a word per block in pinned host memory: one plain store each, nothing of the device's is waited for)
+        if (host_flags) __hip_atomic_store(host_flags + j, 1u | (misc[1] << 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    write_masks(out, j, lo, n_nodes, block_m, max_anc, mask_words, kept, bitmap, mbits, misc);
 }
 
 constexpr int kPackMaxTiles = 512;   // ancestor tiles a block plan written by pack_mask_kernel can have

@@ -2,10 +2,16 @@
 #pragma once
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 
 #include <tuple>
 
 namespace fsta_torch {
+
+// An uninitialised tensor of the device's allocator, without the dispatcher's 0.4 us (every output here is written whole)
+inline at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor& like) {
+    return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), c10::nullopt));
+}
 
 // FSTA_* code of a storage type, -1 for types the library does not take
 int dtype_code(at::ScalarType t);

@@ -78,9 +78,9 @@ std::tuple<at::Tensor, at::Tensor> attention_fwd(const at::Tensor& q, const at::
 
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
     const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream();
-    at::Tensor o = at::empty(q.sizes(), q.options().dtype(out_dtype_code == FSTA_F32 ? at::kFloat : q.scalar_type()));
+    at::Tensor o = fresh(q.sizes(), out_dtype_code == FSTA_F32 ? at::kFloat : q.scalar_type(), q);
     // the reference allocates L and drops it (fstattention.py:158-160,181); here it only exists when asked for
-    at::Tensor lse = return_lse ? at::empty({Z * H, Nq}, q.options().dtype(at::kFloat)) : at::Tensor();
+    at::Tensor lse = return_lse ? fresh({Z * H, Nq}, at::kFloat, q) : at::Tensor();
     float* lse_ptr = return_lse ? lse.data_ptr<float>() : nullptr;
     const uint32_t* plan_ptr = static_cast<const uint32_t*>(ptr_or_null(plan));
     if (kv8) {
@@ -91,7 +91,7 @@ std::tuple<at::Tensor, at::Tensor> attention_fwd(const at::Tensor& q, const at::
                         "k_scale / v_scale must be contiguous float32 tensors of batch*heads entries on q's device");
         const size_t need = Nk > Nq ? fsta_attention_kv8_workspace_bytes((int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
                                                                          (int32_t)block_m, (int32_t)max_ancestors, (float)sm_scale) : 0;
-        at::Tensor parts = need ? at::empty({(int64_t)need}, q.options().dtype(at::kByte)) : at::Tensor();
+        at::Tensor parts = need ? fresh({(int64_t)need}, at::kByte, q) : at::Tensor();
         check_rc(fsta_attention_fwd_kv8_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), static_cast<const float*>(ptr_or_null(k_scale)),
                                         static_cast<const float*>(ptr_or_null(v_scale)), o.data_ptr(), lse_ptr, plan_ptr,
                                         (int32_t)key_shift, (int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
@@ -106,7 +106,7 @@ std::tuple<at::Tensor, at::Tensor> attention_fwd(const at::Tensor& q, const at::
                                                  (int32_t)max_ancestors, (float)sm_scale, (uint32_t)flags)) {
         work_bytes = fsta_attention_workspace_bytes((int32_t)Z, (int32_t)H, (int32_t)Nq, (int32_t)Nk, (int32_t)D, code,
                                                     (int32_t)block_m, (int32_t)max_ancestors, (float)sm_scale, (uint32_t)flags);
-        if (work_bytes) work = at::empty({(int64_t)work_bytes}, q.options().dtype(at::kByte));
+        if (work_bytes) work = fresh({(int64_t)work_bytes}, at::kByte, q);
     }
     check_rc(fsta_attention_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse_ptr,
                                    a_idx.data_ptr<int64_t>(), static_cast<const uint32_t*>(mask_bits.data_ptr()),
@@ -175,11 +175,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> quantize_kv(const at:
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(k.device());
     const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(k.device().index()).stream();
     const at::Tensor kc = k.contiguous(), vc = v.contiguous();
-    const auto fp8 = k.options().dtype(at::kFloat8_e4m3fn), f32 = k.options().dtype(at::kFloat);
-    at::Tensor k8 = at::empty(k.sizes(), fp8), v8 = at::empty(k.sizes(), fp8);
-    at::Tensor k_scale = at::empty({slices}, f32), v_scale = at::empty({slices}, f32);
+    at::Tensor k8 = fresh(k.sizes(), at::kFloat8_e4m3fn, k), v8 = fresh(k.sizes(), at::kFloat8_e4m3fn, k);
+    at::Tensor k_scale = fresh({slices}, at::kFloat, k), v_scale = fresh({slices}, at::kFloat, k);
     const size_t need = fsta_quantize_workspace_bytes(slices, elements, code);
-    at::Tensor work = need ? at::empty({(int64_t)need}, k.options().dtype(at::kByte)) : at::Tensor();
+    at::Tensor work = need ? fresh({(int64_t)need}, at::kByte, k) : at::Tensor();
     check_rc(fsta_quantize_fp8(kc.data_ptr(), vc.data_ptr(), k8.data_ptr(), v8.data_ptr(), k_scale.data_ptr<float>(),
                                v_scale.data_ptr<float>(), slices, elements, code, need ? work.data_ptr() : nullptr, need, stream));
     return {k8, v8, k_scale, v_scale};

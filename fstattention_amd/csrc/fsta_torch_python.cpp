@@ -22,6 +22,8 @@
 #include "../../include/fsta.h"
 #include "fsta_torch.h"
 
+using fsta_torch::fresh;
+
 namespace {
 
 PyObject* g_packed_type = nullptr;      // attention.PackedTreeMask
@@ -189,11 +191,9 @@ struct OnStream {      // the tensors' device and torch's current stream on it
     const hipStream_t stream;
 };
 
-// The status word of a call: the caller's, or a zeroed one when somebody is going to look at it, or one nobody reads
-at::Tensor status_word(PyObject* given, bool read, const at::Tensor& like) {
-    if (given != Py_None) return tensor_arg(given);
-    const auto i32 = like.options().dtype(at::kInt);
-    return read ? at::zeros({1}, i32) : at::empty({1}, i32);
+// The status word of a call: the caller's or a zeroed one
+at::Tensor status_word(PyObject* given, const at::Tensor& like) {
+    return given != Py_None ? tensor_arg(given) : at::zeros({1}, like.options().dtype(at::kInt));
 }
 
 template <class... T> PyObject* as_tuple(const T&... tensors) {      // undefined tensors become None
@@ -210,6 +210,29 @@ template <class... T> PyObject* as_tuple(const T&... tensors) {      // undefine
     return nullptr;
 }
 
+// Watches the words of fsta_precompute_from_parents_flags until all of them are set (a wait for the stream costs 10 us more
+// than the kernel takes).  Asks the runtime now and then, so that a launch that failed ends the wait with its error.
+long watch_flags(const volatile int32_t* words, int64_t n, hipStream_t stream) {
+    long found = 0;
+    int spins = 0;
+    bool drained = false;
+    for (int64_t j = 0; j < n;) {
+        if (const int32_t word = words[j]) {
+            found |= word >> 1;
+            ++j;
+            continue;
+        }
+        TORCH_CHECK(!drained, "kernel_inputs_from_parents_gpu: the kernel ended without reporting");
+        if (++spins % 4096 == 0) {
+            const hipError_t err = hipStreamQuery(stream);
+            TORCH_CHECK(err == hipSuccess || err == hipErrorNotReady, "kernel_inputs_from_parents_gpu: ", hipGetErrorString(err));
+            drained = err == hipSuccess;      // (the word is looked at once more)
+        }
+        __builtin_ia32_pause();
+    }
+    return found;
+}
+
 template <class T> T* data_or_null(const at::Tensor& t) { return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr; }
 
 // dfs_order(parent, light_first, read_status, status or None) -> (perm, rank, status)
@@ -219,11 +242,14 @@ PyObject* dfs_order(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor parent = tensor_arg(args[0]).contiguous();
     const OnStream on(parent);
     const int64_t n = parent.size(0);
-    at::Tensor perm = at::empty({n}, parent.options()), rank = at::empty({n}, parent.options());
-    at::Tensor work = at::empty({(int64_t)FSTA_DFS_ORDER_WORKSPACE_INTS(n)}, parent.options().dtype(at::kInt));
-    at::Tensor status = status_word(args[3], args[2] == Py_True, parent);
+    at::Tensor perm = fresh({n}, at::kLong, parent), rank = fresh({n}, at::kLong, parent);
+    // (a status word that nobody reads is one int more of workspace)
+    const int64_t ints = (int64_t)FSTA_DFS_ORDER_WORKSPACE_INTS(n);
+    at::Tensor work = fresh({ints + 1}, at::kInt, parent), status;
+    if (args[3] != Py_None || args[2] == Py_True) status = status_word(args[3], parent);
+    uint32_t* word = status.defined() ? static_cast<uint32_t*>(status.data_ptr()) : reinterpret_cast<uint32_t*>(work.data_ptr<int32_t>() + ints);
     const int rc = fsta_dfs_order(parent.data_ptr<int64_t>(), n, args[1] == Py_True, perm.data_ptr<int64_t>(), rank.data_ptr<int64_t>(),
-                                  work.data_ptr<int32_t>(), static_cast<uint32_t*>(status.data_ptr()), on.stream);
+                                  work.data_ptr<int32_t>(), word, on.stream);
     return rc != FSTA_OK ? PyLong_FromLong(rc) : as_tuple(perm, rank, status);
     END_HANDLE_TH_ERRORS
 }
@@ -234,7 +260,7 @@ PyObject* renumber_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) 
     TORCH_CHECK_TYPE(n_args == 2, "renumber_parents takes 2 arguments");
     const at::Tensor parent = tensor_arg(args[0]).contiguous(), rank = tensor_arg(args[1]).contiguous();
     const OnStream on(parent);
-    at::Tensor out = at::empty(parent.sizes(), parent.options());
+    at::Tensor out = fresh(parent.sizes(), at::kLong, parent);
     const int rc = fsta_renumber_parents(parent.data_ptr<int64_t>(), rank.data_ptr<int64_t>(), parent.size(0), out.data_ptr<int64_t>(),
                                          on.stream);
     return rc != FSTA_OK ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
@@ -243,7 +269,8 @@ PyObject* renumber_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) 
 
 // inputs_from_parents(parent, block_m, max_ancestors, width, check, want_bool_mask, want_lineage, status or None)
 //   -> (ancestor_idx, ancestor_mask, leaf_idx, mask_bits, anc_count, plan, lineage, level_lookup, status), bits
-// `check` (then no status word is used or returned): waits for the stream, bits are the FSTA_PRE_* conditions; else 0
+// `check` (then no status word is used or returned): waits until every block has reported, bits are the FSTA_PRE_* conditions;
+// else 0
 PyObject* inputs_from_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
     TORCH_CHECK_TYPE(n_args == 8, "inputs_from_parents takes 8 arguments");
@@ -254,24 +281,23 @@ PyObject* inputs_from_parents(PyObject*, PyObject* const* args, Py_ssize_t n_arg
                       "block_m, max_ancestors and width must be positive");
     const OnStream on(parent);
     const int64_t nb = (n + block_m - 1) / block_m;
-    const auto i64 = parent.options();
-    const auto i32 = parent.options().dtype(at::kInt);
-    at::Tensor a_idx = at::empty({nb, max_anc}, i64), l_idx = at::empty({nb, block_m}, i64), a_mask, lineage, level, plan;
-    if (want_mask) a_mask = at::empty({nb, block_m, max_anc}, parent.options().dtype(at::kBool));
-    at::Tensor bits = at::empty({nb, (int64_t)fsta_mask_words((int32_t)max_anc), block_m}, i32), count = at::empty({nb}, i32);
+    at::Tensor a_idx = fresh({nb, max_anc}, at::kLong, parent), l_idx = fresh({nb, block_m}, at::kLong, parent), a_mask, lineage, level, plan;
+    if (want_mask) a_mask = fresh({nb, block_m, max_anc}, at::kBool, parent);
+    at::Tensor bits = fresh({nb, (int64_t)fsta_mask_words((int32_t)max_anc), block_m}, at::kInt, parent), count = fresh({nb}, at::kInt, parent);
     const size_t plan_bytes = fsta_block_plan_bytes((int32_t)nb, (int32_t)block_m, (int32_t)max_anc);
-    if (plan_bytes) plan = at::empty({(int64_t)(plan_bytes / 4)}, i32);
+    if (plan_bytes) plan = fresh({(int64_t)(plan_bytes / 4)}, at::kInt, parent);
     if (want_lineage) {
-        lineage = at::empty({n, width}, i64);
-        level = at::empty({n}, i64);
+        lineage = fresh({n, width}, at::kLong, parent);
+        level = fresh({n}, at::kLong, parent);
     }
-    // A caller that waits is told through pinned host memory; a word in device memory is for those that look later.
+    // A caller that waits is told through pinned host memory, a word per block; a word in device memory is for those that
+    // look later.
     at::Tensor flags, status;
-    if (check) {
-        flags = at::empty({3}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-        memset(flags.data_ptr(), 0, 3 * sizeof(int32_t));
+    if (check && nb > 0) {
+        flags = at::empty({nb}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        memset(flags.data_ptr(), 0, (size_t)nb * sizeof(int32_t));
     }
-    if (!check) status = status_word(args[7], true, parent);
+    if (!check) status = status_word(args[7], parent);
     const int rc = fsta_precompute_from_parents_flags(
         parent.data_ptr<int64_t>(), n, width, (int32_t)block_m, (int32_t)max_anc, 1, data_or_null<int64_t>(lineage),
         data_or_null<int64_t>(level), a_idx.data_ptr<int64_t>(), data_or_null<uint8_t>(a_mask), l_idx.data_ptr<int64_t>(),
@@ -279,15 +305,9 @@ PyObject* inputs_from_parents(PyObject*, PyObject* const* args, Py_ssize_t n_arg
         data_or_null<uint32_t>(status), data_or_null<uint32_t>(flags), on.stream);
     if (rc != FSTA_OK) return PyLong_FromLong(rc);
     long found = 0;
-    if (check) {
-        hipError_t err;
-        {
-            pybind11::gil_scoped_release no_gil;
-            err = hipStreamSynchronize(on.stream);
-        }
-        TORCH_CHECK(err == hipSuccess, "kernel_inputs_from_parents_gpu: ", hipGetErrorString(err));
-        const volatile int32_t* word = flags.data_ptr<int32_t>();
-        found = (word[0] ? FSTA_PRE_TOO_MANY_ANCESTORS : 0) | (word[1] ? FSTA_PRE_BAD_NODE_ID : 0) | (word[2] ? FSTA_PRE_BAD_LEVEL : 0);
+    if (check && nb > 0) {
+        pybind11::gil_scoped_release no_gil;
+        found = watch_flags(flags.data_ptr<int32_t>(), nb, on.stream);
     }
     PyObject* tensors = as_tuple(a_idx, a_mask, l_idx, bits, count, plan, lineage, level, status);
     return tensors ? Py_BuildValue("Nl", tensors, found) : nullptr;
@@ -303,11 +323,11 @@ PyObject* medusa_parents(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const OnStream on(probs);
     const int32_t depths = (int32_t)probs.size(0), topk = (int32_t)probs.size(1);
     const int32_t code = probs.scalar_type() == at::kFloat ? FSTA_F32 : FSTA_F64;
-    at::Tensor parent = at::empty({n}, probs.options().dtype(at::kLong));
-    at::Tensor status = status_word(args[3], args[2] == Py_True, probs);
+    at::Tensor parent = fresh({n}, at::kLong, probs);
+    at::Tensor status = args[3] != Py_None || args[2] == Py_True ? status_word(args[3], probs) : fresh({1}, at::kInt, probs);
     const size_t need = fsta_medusa_workspace_bytes(depths, topk);
     at::Tensor work;      // (stream-ordered: free again after the launches)
-    if (need) work = at::empty({(int64_t)need}, probs.options().dtype(at::kByte));
+    if (need) work = fresh({(int64_t)need}, at::kByte, probs);
     uint32_t* word = static_cast<uint32_t*>(status.data_ptr());
     const int rc = need ? fsta_medusa_tree_ws(probs.data_ptr(), code, depths, topk, (int32_t)n, parent.data_ptr<int64_t>(), word,
                                               work.data_ptr(), need, on.stream)
@@ -327,7 +347,7 @@ PyObject* shift_index(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         return not_implemented();
     const at::Tensor ac = a->contiguous(), bc = b->contiguous();
     const OnStream on(ac);
-    at::Tensor out_a = at::empty(ac.sizes(), ac.options()), out_b = at::empty(bc.sizes(), bc.options());
+    at::Tensor out_a = fresh(ac.sizes(), at::kLong, ac), out_b = fresh(bc.sizes(), at::kLong, bc);
     const int rc = fsta_shift_index(ac.data_ptr<int64_t>(), ac.numel(), bc.data_ptr<int64_t>(), bc.numel(), shift,
                                     out_a.data_ptr<int64_t>(), out_b.data_ptr<int64_t>(), on.stream);
     return rc != FSTA_OK ? not_implemented() : as_tuple(out_a, out_b);

@@ -304,11 +304,11 @@ int fsta_precompute_from_parents(const int64_t* parent, int64_t n_nodes, int64_t
 /*
  * The same for a caller that looks at the outcome before it goes on: besides (or,
  * with status == NULL, instead of) the status word the conditions are reported in
- * host_flags[3], pinned HOST memory that the device can write (hipHostMalloc),
- * zeroed by the caller before the launch and read after synchronising with the
- * stream: [0] FSTA_PRE_TOO_MANY_ANCESTORS, [1] FSTA_PRE_BAD_NODE_ID,
- * [2] FSTA_PRE_BAD_LEVEL, each 0 or 1.  Spares the fill and the copy of a word in
- * device memory.
+ * host_flags[ceil(n_nodes / block_m)], pinned HOST memory that the device can write
+ * (hipHostMalloc), zeroed by the caller before the launch: block j's word becomes
+ * 1 + 2 * (its FSTA_PRE_* bits) as soon as they are known.  A host that watches the
+ * words learns the outcome without waiting for the stream (about 10 us on its own);
+ * the outputs are complete when the stream is.
  */
 int fsta_precompute_from_parents_flags(const int64_t* parent, int64_t n_nodes, int64_t width, int32_t block_m,
                                        int32_t max_ancestors, int32_t insert_self, int64_t* lineage,
