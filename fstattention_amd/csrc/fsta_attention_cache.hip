@@ -149,21 +149,21 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
         k_off[i] = (uint32_t)dma_row * kRowBytes + (uint32_t)k_swz(r, dma_slot) * 16u;
         v_off[i] = (uint32_t)dma_row * kRowBytes + (uint32_t)v_swz(r, dma_slot) * 16u;
     }
+    constexpr int kRawBuffer = 0x00020000;   // descriptor word 3: raw 32-bit data
+    const int slice_bytes = (int)((uint32_t)p.nk * (uint32_t)kRowBytes);
+    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kb), 0, slice_bytes, kRawBuffer);
+    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vb), 0, slice_bytes, kRawBuffer);
     int n_anc_tiles = 0;                     // the list is [prefix tiles | ancestor tiles | the rows' own keys]
     auto issue = [&](int t, int slot) {
         unsigned char* dst = ring + slot * 2 * kHalf;
         if (t < n_pfx && (first_tile + t + 1) * kTileN <= p.prefix) {
-            // 32 consecutive rows: uniform addresses, lane offsets that never change
-            const char* ks = kb + (size_t)(first_tile + t) * kHalf;
-            const char* vs = vb + (size_t)(first_tile + t) * kHalf;
+            // 32 consecutive rows: one uniform offset, lane offsets that never change.  Buffer addressing takes both as they
+            // are (a flat address is 64-bit vector arithmetic per transfer: 8192 keys in 8 bits 35.3 us, 33.9 this way).
+            const uint32_t tile_off = (uint32_t)(first_tile + t) * (uint32_t)kHalf;
 #pragma unroll
-            for (int i = 0; i < 2 * kDma; ++i) {
-                const char* src = (i < kDma ? ks : vs) + (i % kDma) * 1024;
-                asm volatile("" : "+s"(src));    // (kept uniform: base and lane offset stay apart)
-                __builtin_amdgcn_global_load_lds(
-                    (const void __attribute__((address_space(1)))*)(src + (size_t)(i < kDma ? k_off[i % kDma] : v_off[i % kDma])),
-                    (void __attribute__((address_space(3)))*)(dst + i * 1024), 16, 0, kAux);
-            }
+            for (int i = 0; i < 2 * kDma; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(i < kDma ? k_rsrc : v_rsrc, (void __attribute__((address_space(3)))*)(dst + i * 1024), 16,
+                                                         (int)(i < kDma ? k_off[i % kDma] : v_off[i % kDma]), (int)(tile_off + (i % kDma) * 1024), 0, kAux);
         } else {
             // the partial tile at the end of the prefix, ancestor tiles, then the tile of the rows' own keys
             int rows[kDma];
