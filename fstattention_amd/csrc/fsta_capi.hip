@@ -152,9 +152,11 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
     const CacheCost& k = (kv8 ? kCost8 : kCost16)[head_dim == 128 ? 1 : 0];
     const double bytes = (double)slices * prefix * head_dim * (kv8 ? 2.0 : 4.0) * 1e-6;      // prefix K and V, MB
     double best = 0.0;
-    // candidates: one run, and the counts that fill the CUs once, twice, ..; a run has work for half of a workgroup's waves
-    for (int i = 0; i <= 4; ++i) {
-        const int64_t fill = i == 0 ? 1 : (int64_t)kGpuCus * i / wgs1;
+    // candidates: one run, the counts that fill the CUs once, twice, .., and those whose runs are one, two, .. tiles for
+    // each of eight waves, if they promise a tenth, the prediction's error (few slices: 46 rows, 8 slices, 1955 keys fill
+    // 16 CUs in one run, 15.0 us, 9.3 in eight); a run has work for half of a workgroup's waves
+    for (int i = 0; i <= 8; ++i) {
+        const int64_t fill = i == 0 ? 1 : i <= 4 ? (int64_t)kGpuCus * i / wgs1 : (tiles + 8 * (i - 4) - 1) / (8 * (i - 4));
         const int want = forced ? forced : (int)(fill > 64 ? 64 : fill);
         if (i > 0 && (forced || want <= 1 || tiles / want < 4)) continue;
         const int per = (tiles + want - 1) / want;
@@ -172,7 +174,7 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
         const double mem = 1.6 + k.start_end8 + bytes / k.tb * (1.0 + k.again * (double)(groups - 1));
         if (mem > t) t = mem;
         if (runs > 1) t += k.join + 2.0 * runs * (double)slices * nq * head_dim * 4e-6 / k.join_tb;
-        if (c.runs == 0 || t < best) {
+        if (c.runs == 0 || t < (i <= 4 ? best : 0.9 * best)) {
             best = t;
             c.waves = waves;
             c.runs = runs;
