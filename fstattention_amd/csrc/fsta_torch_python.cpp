@@ -42,10 +42,11 @@ const at::Tensor* gpu_tensor(PyObject* o) {
                : nullptr;
 }
 
-// Nobody has asked to see calls on tensors (modes, functorch, tracing)
+// Nobody has asked to see calls on tensors (modes, functorch, tracing).  Inference mode only takes ADInplaceOrView out of the
+// default set, which looks after views of and writes to arguments: there are none here.
 bool plain_context() {
-    const auto tls = c10::impl::tls_local_dispatch_key_set();
-    return tls.included_ == c10::default_included_set && !at::impl::torch_function_mode_enabled();
+    const auto included = c10::impl::tls_local_dispatch_key_set().included_ | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
+    return included == c10::default_included_set && !at::impl::torch_function_mode_enabled();
 }
 
 bool wants_grad(const at::Tensor& t) { return t.requires_grad(); }
