@@ -9,6 +9,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Dtype.h>
@@ -156,6 +157,17 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
             (i ? v_scale : k_scale) = *s;
         }
     try {
+        // profilers and other observers see the call under the name of the registered operator
+        c10::optional<at::RecordFunction> seen;
+        if (auto callbacks = at::getStepCallbacksUnlessEmpty(at::RecordScope::FUNCTION)) {
+            seen.emplace(std::move(*callbacks));
+            if (seen->needsInputs()) {
+                const c10::IValue inputs[] = {*q, *k, *v, *a_idx, *p.bits, *p.count, *l_idx};
+                seen->before("fsta::attention_fwd", c10::ArrayRef<const c10::IValue>(inputs, 7));
+            } else {
+                seen->before("fsta::attention_fwd");
+            }
+        }
         const auto out = fsta_torch::attention_fwd(*q, *k, *v, *a_idx, *p.bits, *p.count, *l_idx,
                                                    p.plan ? c10::optional<at::Tensor>(*p.plan) : c10::nullopt, p.key_shift, sm_scale,
                                                    block_m, max_anc, out_code, return_lse, flags, k_scale, v_scale);

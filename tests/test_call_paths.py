@@ -34,3 +34,16 @@ def test_inference_mode_takes_the_c_function(monkeypatch):
         got = fst_attention(*args, **options)
         assert got.is_inference()
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_a_profiler_sees_the_call():
+    args, options = _call_inputs()
+    want = fst_attention(*args, **options)
+    for shapes in (False, True):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=shapes) as prof:
+            got = fst_attention(*args, **options)
+        assert torch.equal(got, want)
+        seen = [e for e in prof.events() if e.name == "fsta::attention_fwd"]
+        assert len(seen) == 1
+        assert not shapes or [list(s) for s in seen[0].input_shapes[:3]] == [[1, 2, 64, 64]] * 3
