@@ -177,11 +177,13 @@ def quantize_kv_fp8(k: torch.Tensor, v: torch.Tensor):
     ``float8_e4m3fn`` tensors and one float32 scale per (batch, head) slice (``[Z*H]``) chosen so that
     the slice's largest magnitude maps to the format's largest value (448).  ``k8 * k_scale`` is the K
     the kernel computes with.  On the GPU one or two launches of a kernel of the library; tensors it does not take (on
-    the host, float64, of different shapes, rows that are no multiple of 16 bytes, a gradient asked for) go through the
-    same steps as tensor operations, with the same bytes."""
-    if k.is_cuda and k.dim() == 4 and v.device == k.device and v.shape == k.shape and v.dtype == k.dtype and k.dtype in _DTYPES and \
-            k.shape[2] * k.shape[3] % 16 == 0 and k.numel() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0 and \
-            not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)):
+    the host, float64, of different shapes, slices that are no multiple of 16 elements, without memory of their own --
+    traced, fake, batched by ``vmap`` --, differentiated in either direction) go through the same steps as tensor
+    operations.  Those give the kernel's bytes on the GPU; on the host, where torch divides by 448 instead of multiplying by
+    the rounded 1/448, a scale may differ by one unit in the last place."""
+    if k.is_cuda and not torch.compiler.is_compiling() and (_CALLS or _calls()).plain_tensors(k, v) and k.dim() == 4 and \
+            v.device == k.device and v.shape == k.shape and v.dtype == k.dtype and k.dtype in _DTYPES and \
+            k.shape[2] * k.shape[3] % 16 == 0 and k.numel() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0:
         return (_OPS or _ops()).quantize_kv(k, v)
 
     def one(t):

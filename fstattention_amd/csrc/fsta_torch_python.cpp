@@ -43,12 +43,14 @@ const at::Tensor* gpu_tensor(PyObject* o) {
                : nullptr;
 }
 
-// Nobody has asked to see calls on tensors (modes, functorch, tracing).  Inference mode only takes ADInplaceOrView out of the
-// default set, which looks after views of and writes to arguments: there are none here.
-bool plain_context() {
+// Nobody stands between the dispatcher and the kernels (dispatch modes, functorch, tracing).  Inference mode only takes
+// ADInplaceOrView out of the default set, which looks after views of and writes to arguments: there are none here.
+bool plain_dispatch() {
     const auto included = c10::impl::tls_local_dispatch_key_set().included_ | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
-    return included == c10::default_included_set && !at::impl::torch_function_mode_enabled();
+    return included == c10::default_included_set;
 }
+// .. and nobody has asked to see calls from Python
+bool plain_context() { return plain_dispatch() && !at::impl::torch_function_mode_enabled(); }
 
 bool wants_grad(const at::Tensor& t) { return t.requires_grad(); }
 
@@ -367,6 +369,21 @@ PyObject* shift_index(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// plain_tensors(a, b): True if an operator whose only implementation is a kernel may take both: ordinary GPU tensors that
+// nobody transforms, traces below the dispatcher or differentiates, in either direction.  (A mode that watches calls from
+// Python, such as a default device, sees the operator as any other.)
+PyObject* plain_tensors(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n_args == 2, "plain_tensors takes 2 arguments");
+    if (!plain_dispatch()) Py_RETURN_FALSE;
+    for (int i = 0; i < 2; ++i) {
+        const at::Tensor* t = gpu_tensor(args[i]);
+        if (!t || (c10::GradMode::is_enabled() && wants_grad(*t)) || t->_fw_grad(0).defined()) Py_RETURN_FALSE;
+    }
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 // setup(PackedTreeMask, packed_table)
 PyObject* setup(PyObject*, PyObject* args) {
     PyObject *type, *table;
@@ -386,6 +403,7 @@ PyMethodDef kMethods[] = {
     FSTA_FASTCALL(inputs_from_parents),
     FSTA_FASTCALL(medusa_parents),
     FSTA_FASTCALL(shift_index),
+    FSTA_FASTCALL(plain_tensors),
     {"setup", &setup, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
