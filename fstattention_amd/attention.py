@@ -307,8 +307,10 @@ def shift_for_prefix(ancestor_idx: torch.Tensor, leaf_idx: torch.Tensor, prefix:
     :class:`PackedTreeMask` that belongs to the two tensors) a third value is returned: the same
     packed inputs with the shift noted, so that they stay valid for the shifted tensors.
     """
-    shifted = (_CALLS or _calls()).shift_index(ancestor_idx, leaf_idx, prefix)      # one launch for both
-    if shifted is NotImplemented:       # (on the host, other integer types)
+    shifted = NotImplemented
+    if ancestor_idx.is_cuda and not torch.compiler.is_compiling():      # one launch for both
+        shifted = (_CALLS or _calls()).shift_index(ancestor_idx, leaf_idx, prefix)
+    if shifted is NotImplemented:       # (on the host, other integer types, traced)
         shifted = (torch.where(ancestor_idx >= 0, ancestor_idx + prefix, ancestor_idx),
                    torch.where(leaf_idx >= 0, leaf_idx + prefix, leaf_idx))
     if packed is None:

@@ -107,3 +107,17 @@ def test_quantize_as_tensor_operations_gives_the_same_bytes(dtype):
     with torch.device("cuda"):      # (a mode that watches calls from Python: the kernel)
         assert attention_module._CALLS.plain_tensors(k, v)
         _same_bytes(quantize_kv_fp8(k, v), steps)
+
+
+def test_shift_is_traceable_and_needs_no_library_on_the_host(monkeypatch):
+    a_idx = torch.arange(12).view(2, 6) - 3
+    l_idx = torch.arange(8).view(2, 4) - 1
+    want = [torch.where(t >= 0, t + 100, t) for t in (a_idx, l_idx)]
+    got = torch.compile(lambda a, l: shift_for_prefix(a, l, 100), backend="eager", fullgraph=True)(a_idx, l_idx)
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
+    monkeypatch.setattr(attention_module, "_CALLS", None)
+
+    def missing():
+        raise ImportError("library asked for")
+    monkeypatch.setattr(attention_module, "_calls", missing)
+    assert all(torch.equal(g, w) for g, w in zip(shift_for_prefix(a_idx, l_idx, 100), want))
