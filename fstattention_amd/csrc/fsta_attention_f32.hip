@@ -73,7 +73,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
         for (int e = 0; e < 4; ++e) o[b][e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     f32x4 k[kQLoads], v[4][kVb];
-    uint32_t ok = 0u;                        // bit r: key 4g + r of the tile exists and query i attends to it
+    // bit r: key 4g + r of the tile exists and query i attends to it; bit 16 + c: slot c of the tile has no key
+    uint32_t ok = 0u;
     auto request = [&](int t, int64_t id, uint32_t w) {
         int key;
         if (t < anc_tiles) {
@@ -82,14 +83,15 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
             const int first = exists ? __builtin_ctz(exists) : 0;
             // an empty slot repeats the tile's first row: no row outside the list is read
             key = there ? (int)id : -1;
-            const int spare = __shfl(key, first);
-            if (key < 0) key = max(spare, 0);
-            ok = (((w >> (kKeys * (t & 1))) & exists) >> (4 * g)) & 0xfu;
+            const int repeat = __shfl(key, first);
+            if (key < 0) key = max(repeat, 0);
+            ok = ((((w >> (kKeys * (t & 1))) & exists) >> (4 * g)) & 0xfu) | (~exists << 16);
         } else {
             const int c = (t - anc_tiles) * kKeys;
             key = min(c + i, p.prefix - 1);
             const int left = p.prefix - c - 4 * g;
             ok = left >= 4 ? 0xfu : left > 0 ? (1u << left) - 1u : 0u;
+            if (p.prefix - c < kKeys) ok |= 0xffffffffu << (16 + p.prefix - c);
         }
         const float* k_row = kb + (size_t)key * D + 4 * g;
 #pragma unroll
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
     }
     for (int t = wave; t < total; t += NW) {
         const bool more = t + NW < total;
-        const uint32_t mine = ok;
+        const uint32_t mine = ok, empty = __builtin_amdgcn_readfirstlane(ok >> 16);
         if (more) {                          // (entries of the next tile: on their way under this tile's products)
             entry = list_entry(t + NW);
             word = mask_word(t + NW);
@@ -176,6 +178,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
         for (int b = 0; b < kVb; ++b)
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[b][e] *= alpha;
+        if (empty) {
+            // slots without a key repeat a row under weight 0: nothing of it may come through, not even as 0 * infinity
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if ((empty >> (4 * g + r)) & 1u)
+#pragma unroll
+                    for (int b = 0; b < kVb; ++b) v[r][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll

@@ -965,3 +965,39 @@ def test_float32_on_the_matrix_cores(d, n, block_m, window, prefix):
     tiles per wave."""
     parent = trees.random_recursive_parents(n, 50 + n, window=window)
     run_tree(parent, block_m, 2, 3, d, torch.float32, n + prefix, prefix=prefix, want_kernel="attn_f32_kernel")
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("prefix", [0, 5, 33])
+def test_float32_slots_without_a_key_let_nothing_through(d, prefix):
+    """Slots without a key (the tail of a list, a whole tile in the middle of one, the tail of the prefix) are computed with
+    some row under weight 0: an infinity or a NaN in that row's V reaches exactly the rows that attend to it."""
+    n, block_m = 40, 32
+    parent = np.arange(-1, n - 1, dtype=np.int64)
+    parent[1] = -1                               # node 0 alone, the others a chain below node 1
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, block_m)
+    empty_idx = torch.full((a_idx.shape[0], 16), -1, dtype=torch.int64)
+    empty_mask = torch.zeros((a_idx.shape[0], block_m, 16), dtype=torch.bool)
+    a_idx, a_mask = torch.cat([empty_idx, a_idx], 1), torch.cat([empty_mask, a_mask], 2)
+    nq = a_idx.shape[0] * block_m
+    q, k, v = rand_qkv(1, 2, nq, nq + prefix, d, torch.float32, 21)
+    scale = 1.0 / math.sqrt(d)
+    if prefix:
+        a_idx, l_idx = shift_for_prefix(a_idx, l_idx, prefix)
+        v[:, :, prefix - 1, 1] = 0.0
+    v[:, :, prefix, 2] = 0.0
+    v[:, :, prefix + 1, 3] = 0.0
+    want, _ = dense_oracle(q, k, v, parent, scale, prefix=prefix, nq_pad=nq - n)
+    if prefix:
+        v[:, :, prefix - 1, 1] = float("-inf")   # every row attends to it
+        want[..., 1] = float("-inf")
+    v[:, :, prefix, 2] = float("nan")            # node 0: itself alone
+    want[:, :, 0, 2] = float("nan")
+    v[:, :, prefix + 1, 3] = float("inf")        # node 1: all of the chain
+    want[:, :, 1:n, 3] = float("inf")
+    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), scale, BLOCK_M=block_m,
+                      MAX_ANCESTORS=max_anc + 16)
+    # (row 0 and the rows that pad the last block have node 1 among their block's keys: not theirs, but keys)
+    o, want = o.cpu().double()[:, :, :n], want[:, :, :n]
+    o[:, :, 0, 3] = want[:, :, 0, 3] = 0.0
+    torch.testing.assert_close(o, want, atol=1e-5, rtol=1e-5, equal_nan=True)
