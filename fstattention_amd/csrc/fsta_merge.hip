@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_splits_kernel(
     const size_t part_stride = (size_t)rows * chunks_per_row;   // in float4
     const float4* src = reinterpret_cast<const float4*>(part_o) + (size_t)row * chunks_per_row + chunk;
     // Four parts at a time, all their loads ahead of the first use (a part's weight decides nothing about its load: one
-    // round trip per four parts instead of two per part).  A part's rows are finite, also where it has no keys.
+    // round trip per four parts instead of two per part).  A part's rows are zero where it has no keys.
     float m = -INFINITY, sum = 0.f;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < splits; s0 += 4) {
@@ -90,6 +90,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_splits_kernel(
         for (int i = 0; i < 4; ++i) acc[i] *= old;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
+            if (s0 + u >= splits) break;        // (the same in every lane; a repeated infinity under weight 0 would be a NaN)
             const float w = exp2f(l[u] - safe);
             acc[0] += w * x[u].x; acc[1] += w * x[u].y; acc[2] += w * x[u].z; acc[3] += w * x[u].w;
             sum += w;

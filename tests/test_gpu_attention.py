@@ -1001,3 +1001,22 @@ def test_float32_slots_without_a_key_let_nothing_through(d, prefix):
     o, want = o.cpu().double()[:, :, :n], want[:, :, :n]
     o[:, :, 0, 3] = want[:, :, 0, 3] = 0.0
     torch.testing.assert_close(o, want, atol=1e-5, rtol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("splits", [2, 3, 5, 6])
+def test_an_infinity_in_the_last_run_stays_one(splits):
+    """Run counts that do not fill the joining kernel's groups of four: the last run counts once, also with an infinity in it.
+    (float16: the second half of a split bfloat16 weight has either sign, which makes a NaN of it.)"""
+    dtype = torch.float16
+    parent = trees.random_recursive_parents(40, 3, window=8)
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32)
+    nq, prefix = a_idx.shape[0] * 32, 32 * splits
+    q, k, v = rand_qkv(1, 2, nq, nq + prefix, 64, dtype, 41)
+    v[:, :, prefix - 1, 5] = 0.0
+    want, _ = dense_oracle(q, k, v, parent, 0.125, prefix=prefix, nq_pad=nq - 40)
+    v[:, :, prefix - 1, 5] = float("inf")        # every row attends to it
+    want[..., 5] = float("inf")
+    a_idx, l_idx = shift_for_prefix(a_idx, l_idx, prefix)
+    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), 0.125, BLOCK_M=32,
+                      MAX_ANCESTORS=max_anc, out_dtype=torch.float32, key_splits=splits)
+    torch.testing.assert_close(o.cpu().double(), want, atol=TOL[dtype], rtol=TOL[dtype])
