@@ -14,6 +14,8 @@
 // column i; C register r holds row 8*(r/4) + 4h + r%4 of column i.  S^T = K.Q^T: the column is the query, a lane has 16
 // of a tile's 32 keys for one query, and registers 8kk .. 8kk+7 are its k-slots of O^T += V^T.P^T over keys 16kk ..
 // 16kk+15, in the order {4h .. 4h+3, 8+4h .. 8+4h+3}, which the transposing reads of V follow.
+#include <type_traits>
+
 #include "fsta_mfma_common.h"
 
 namespace fsta {
@@ -223,7 +225,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
         leaf_word = valid & (1u << ql);
     }
     const int total = n_pfx + (tree ? n_anc_tiles + 1 : 0);
+    const bool own_here = tree && (total - 1) % kWaves == wave;      // the rows' own keys are this wave's last tile
     const int mine = wave < total ? (total - wave + kWaves - 1) / kWaves : 0;      // tiles wave, wave + 8, ...
+    const int mine_shared = mine - (own_here ? 1 : 0);      // those whose keys the rows share
 #pragma unroll
     for (int i = 0; i < kSlots; ++i)
         if (i >= issued && i < mine) issue(wave + i * kWaves, i);
@@ -331,19 +335,15 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
     };
 
     // One tile ahead: at the top of iteration i the fragments of tile i are in registers, tiles behind it are on their way.
+    // (The rows' own keys come behind the loop, K fragments read as any tile's, V from the ring as it is needed there.)
     if (mine > 0) {
         wait_tiles(issued - 1);
         read_k(0);
-        read_v(0);
+        if (mine_shared > 0) read_v(0);
         tie_all();
         if (mine > kSlots) issue(wave + kSlots * kWaves, 0);
     }
-    int slot = 0;                            // ring slot of tile i
-    for (int i = 0; i < mine; ++i) {
-        const int t = wave + i * kWaves;
-        const int next_slot = slot + 1 == kSlots ? 0 : slot + 1;
-
-        // S^T = K_tile . Q^T
+    auto scores = [&]() {                    // S^T = K_tile . Q^T of the tile whose fragments are in registers
         f32x16 s;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = 0.f;
@@ -357,15 +357,19 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
                 s = MM::mfma(__builtin_bit_cast(Frag, kf[u]), qf[u], s);
             }
         }
+        return s;
+    };
+    int slot = 0;                            // ring slot of tile i
+    for (int i = 0; i < mine_shared; ++i) {
+        const int t = wave + i * kWaves;
+        const int next_slot = slot + 1 == kSlots ? 0 : slot + 1;
+
+        f32x16 s = scores();
         // mask: none for whole prefix tiles (uniform branch)
         uint32_t word = 0xffffffffu;
         if (t >= n_pfx || (first_tile + t + 1) * kTileN > p.prefix) {
-            const int ta = t - n_pfx;
-            if (t < n_pfx) {
-                word = (1u << (p.prefix - (first_tile + t) * kTileN)) - 1u;
-            } else {
-                word = ta < n_anc_tiles ? group_s[kTileN + ta * kTileN + ql] : leaf_word;
-            }
+            if (t < n_pfx) word = (1u << (p.prefix - (first_tile + t) * kTileN)) - 1u;
+            else word = group_s[kTileN + (t - n_pfx) * kTileN + ql];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)(word >> (4 * h)), 8 * (r / 4) + r % 4, 1);
@@ -450,10 +454,73 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
         pack(1);
         products(1);
         if (kSlots == 1) wait_vmcnt<0>();
-        read_v(next_slot);
+        if (i + 1 < mine_shared) read_v(next_slot);
         tie_all();
         if (i + 1 + kSlots < mine) issue(t + (1 + kSlots) * kWaves, next_slot);
         slot = next_slot;
+    }
+
+    if (own_here) {
+        // The rows' own keys: one score and the V row of that query alone, by the vector ALU.  As products under 31 zero
+        // weights an infinity or a NaN in one row's V would reach the whole group (reference fstattention.py:104-107 takes
+        // the row's own V by itself, too).
+        typedef typename std::conditional<KV8, uint32_t, u32x2>::type Raw;
+        Raw raw[kDTiles][4];                 // head dims 32 dt + 8 q4 + 4 h .. +3
+        const uint32_t v_row = lds_addr(ring + slot * 2 * kHalf) + kHalf + (uint32_t)(ql * kRowBytes);
+#pragma unroll
+        for (int dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                if constexpr (KV8) raw[dt][q4] = lds_read_b32(v_row + (uint32_t)(v_swz(ql, 2 * dt + (q4 >> 1)) * 16 + 8 * (q4 & 1) + 4 * h));
+                else raw[dt][q4] = lds_read_b64(v_row + (uint32_t)(v_swz(ql, 4 * dt + q4) * 16 + 8 * h));
+            }
+        const f32x16 s = scores();
+        uint32_t bits = 0u;                  // key ql's score: one of the registers of one half
+        const uint32_t own_bit = (1u << ql) >> (4 * h);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float score = s[r];
+            bits |= __builtin_bit_cast(uint32_t, score) & (uint32_t)__builtin_amdgcn_sbfe((int)own_bit, 8 * (r / 4) + r % 4, 1);
+        }
+        const u32x2 both = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+        const uint32_t b0 = both[0], b1 = both[1];
+        const float score = __builtin_bit_cast(float, b0 | b1) * sc;
+        // (the maximum is raised as above)
+        const bool raise = leaf_word != 0u && (score > m_i + kRescaleSlack || (m_i == -INFINITY && score > -INFINITY));
+        if (__ballot(raise) != 0ull) {
+            const float alpha = raise ? __builtin_amdgcn_exp2f(m_i - score) : 1.f;      // exp2(-inf) = 0
+            if (raise) m_i = score;
+            l_i *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+        }
+        const float w = __builtin_amdgcn_exp2f(score - (m_i == -INFINITY ? 0.f : m_i));
+        lds_wait();
+#pragma unroll
+        for (int dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) lds_tie(raw[dt][q4]);
+        if (leaf_word != 0u) {
+            if (h == 0) l_i += w;
+#pragma unroll
+            for (int dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    float x[4];
+                    if constexpr (KV8) {
+                        const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)raw[dt][q4], false);
+                        const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)raw[dt][q4], true);
+                        x[0] = lo[0], x[1] = lo[1], x[2] = hi[0], x[3] = hi[1];
+                    } else {
+                        const uint32_t lo = raw[dt][q4][0], hi = raw[dt][q4][1];
+                        x[0] = MM::low(lo), x[1] = MM::high(lo), x[2] = MM::low(hi), x[3] = MM::high(hi);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[dt][4 * q4 + e] = __builtin_fmaf(x[e], w, o[dt][4 * q4 + e]);
+                }
+        }
     }
 
     // ---- join the waves: results to LDS (16-byte pieces swizzled by the row), then every thread sums 4 * kPieces head dims

@@ -1020,3 +1020,31 @@ def test_an_infinity_in_the_last_run_stays_one(splits):
     o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), 0.125, BLOCK_M=32,
                       MAX_ANCESTORS=max_anc, out_dtype=torch.float32, key_splits=splits)
     torch.testing.assert_close(o.cpu().double(), want, atol=TOL[dtype], rtol=TOL[dtype])
+
+
+@pytest.mark.parametrize("storage", ["bf16", "f16", "f8"])
+@pytest.mark.parametrize("nodes,d,prefix,heads", [(40, 128, 40, 2), (40, 64, 700, 2), (90, 128, 2500, 1), (64, 64, 64, 300)])
+def test_cache_kernel_keeps_a_rows_own_value_to_itself(storage, nodes, d, prefix, heads):
+    """A row's own key is nobody else's: an infinity (8 bits: a NaN) in V of one node without children leaves the other rows
+    of its group alone, whatever weights they have."""
+    dtype = torch.float16 if storage == "f16" else torch.bfloat16
+    parent = np.full(nodes, -1, dtype=np.int64)          # roots only: no row is another one's ancestor
+    parent[1:6] = 0                                      # .. but for a list of one
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32)
+    nq = a_idx.shape[0] * 32
+    q, k, v = rand_qkv(1, heads, nq, nq + prefix, d, dtype, 31)
+    scale = 1.0 / math.sqrt(d)
+    if storage == "f8":
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    bad = prefix + 17
+    v.view(torch.uint8 if storage == "f8" else torch.int16)[:, :, bad, 5] = 0
+    want, _ = dense_oracle(q.double(), k.double(), v.double(), parent, scale, prefix=prefix, nq_pad=nq - nodes)
+    special = float("nan") if storage == "f8" else float("inf")
+    v[:, :, bad, 5] = special
+    want[:, :, 17, 5] = special
+    a_idx, l_idx = shift_for_prefix(a_idx, l_idx, prefix)
+    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), scale, BLOCK_M=32,
+                      MAX_ANCESTORS=max_anc, out_dtype=torch.float32)
+    from fstattention_amd import _lib
+    assert "attn_cache_kernel" in _lib.load().fsta_last_attention_kernel().decode()
+    torch.testing.assert_close(o.cpu().double(), want, atol=2e-3, rtol=2e-3, equal_nan=True)
