@@ -604,17 +604,13 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
 template <bool BF16, int D, bool KV8, int NW, bool SPLIT>
 int launch_waves(const AttnParams& p, const CachePlan& plan, hipStream_t stream) {
     const size_t lds = cache_lds_bytes<D, NW>(p.max_anc);
-    if (lds > 160 * 1024) return FSTA_EUNSUPPORTED;
     CacheGrid g;
     g.chunks = (p.nq + kRows - 1) / kRows;
     g.runs = plan.runs;
     g.run_tiles = plan.run_tiles;
     const int64_t total = (int64_t)p.heads_total * g.chunks * g.runs;
-    if (total > 0x7fffff00) return FSTA_EUNSUPPORTED;
     g.total = (int32_t)total;
     g.per_xcd = (int32_t)((total + kXcds - 1) / kXcds);
-    // (quotients by multiplication are exact while dividend * divisor < 2^32)
-    if ((uint64_t)(total + kXcds) * (uint64_t)(g.chunks > g.runs ? g.chunks : g.runs) >= 0xffffffffull) return FSTA_EUNSUPPORTED;
     g.chunks_inv = g.chunks > 1 ? (uint32_t)((0x100000000ull + g.chunks - 1) / g.chunks) : 0u;
     g.runs_inv = g.runs > 1 ? (uint32_t)((0x100000000ull + g.runs - 1) / g.runs) : 0u;
     g.block_shift = p.block_m == 32 ? 5 : p.block_m == 64 ? 6 : 7;
@@ -651,10 +647,19 @@ bool cache_kernel_supported(int dtype, int head_dim, int block_m) {
     return (dtype == FSTA_F16 || dtype == FSTA_BF16) && (head_dim == 64 || head_dim == 128) && plan_block_size_ok(block_m);
 }
 
+bool cache_kernel_takes(int64_t slices, int nq, int nk, int head_dim, bool kv8, int max_anc, const CachePlan& plan) {
+    if ((uint64_t)nk * (uint64_t)head_dim * (kv8 ? 1u : 2u) > 0xffffffffull) return false;      // 32-bit byte offsets in a slice
+    const size_t lds = head_dim == 64 ? (plan.waves == 4 ? cache_lds_bytes<64, 4>(max_anc) : cache_lds_bytes<64, 8>(max_anc))
+                                      : (plan.waves == 4 ? cache_lds_bytes<128, 4>(max_anc) : cache_lds_bytes<128, 8>(max_anc));
+    if (lds > 160 * 1024) return false;
+    const int64_t chunks = (nq + kRows - 1) / kRows, total = slices * chunks * plan.runs;
+    // (a launch's quotients by multiplication are exact while dividend * divisor < 2^32)
+    return total <= 0x7fffff00 && (uint64_t)(total + kXcds) * (uint64_t)(chunks > plan.runs ? chunks : plan.runs) < 0xffffffffull;
+}
+
 int launch_attention_cache(const AttnParams& p, int dtype, int head_dim, bool kv8, bool fast_pv, const CachePlan& plan,
                            hipStream_t stream) {
-    // (a slice is addressed with 32-bit byte offsets)
-    if (!p.plan || (uint64_t)p.nk * (uint64_t)head_dim * (kv8 ? 1u : 2u) > 0xffffffffull) return FSTA_EUNSUPPORTED;
+    if (!p.plan || !cache_kernel_takes(p.heads_total, p.nq, p.nk, head_dim, kv8, p.max_anc, plan)) return FSTA_EUNSUPPORTED;
     const bool split = dtype == FSTA_BF16 && !fast_pv;
     if (dtype == FSTA_F16)
         return kv8 ? launch_dim<false, true, false>(p, head_dim, plan, stream) : launch_dim<false, false, false>(p, head_dim, plan, stream);

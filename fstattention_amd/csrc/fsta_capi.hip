@@ -129,8 +129,8 @@ constexpr CacheCost kCost8[2] = {{3.2f, 2.3f, 0.106f, 0.67f, 2.06f, 3.2f, 4.0f, 
 constexpr int kCacheMaxRows = 512;    // longer trees: their own kernels (a workgroup of the cache kernel reads the prefix for 32 rows)
 constexpr int kGpuCus = 256;
 
-CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, int block_m, float sm_scale, uint32_t flags,
-                     bool kv8) {
+CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, int block_m, int max_anc, float sm_scale,
+                     uint32_t flags, bool kv8) {
     CachePlan c = {8, 0, 0};
     const int prefix = nk - nq;
     if (slices <= 0 || nq <= 0 || prefix <= 0 || nq > kCacheMaxRows) return c;
@@ -181,10 +181,12 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
             c.run_tiles = per;
         }
     }
+    // (what the kernel would refuse is not planned for it: the workspace queries have to know)
+    if (!cache_kernel_takes(slices, nq, nk, head_dim, kv8, max_anc, c)) c.runs = 0;
     return c;
 }
 
-// launches it; FSTA_EUNSUPPORTED where the plan says no or the lists need too much LDS
+// launches it; FSTA_EUNSUPPORTED where the plan says no
 int launch_cache(AttnParams p, int dtype, int out_dtype, int head_dim, bool kv8, bool fast_pv, CachePlan c, void* workspace,
                  size_t workspace_bytes, size_t wanted_bytes, hipStream_t s) {
     if (c.runs < 1) return FSTA_EUNSUPPORTED;
@@ -210,7 +212,6 @@ int launch_cache(AttnParams p, int dtype, int out_dtype, int head_dim, bool kv8,
 extern "C" size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk,
                                                  int32_t head_dim, int32_t dtype, int32_t block_m,
                                                  int32_t max_ancestors, float sm_scale, uint32_t flags) {
-    (void)max_ancestors;
     if (batch <= 0 || heads <= 0 || nq <= 0 || nk <= nq || block_m <= 0) return 0;
     int split_tiles = 0;
     const int64_t slices = (int64_t)batch * heads;
@@ -220,7 +221,7 @@ extern "C" size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, i
         const int splits = plan_key_splits(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, &split_tiles);
         if (splits > 1) bytes = key_split_bytes(splits, slices, nq, head_dim);
     }
-    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, flags, false);
     if (c.runs > 1 && key_split_bytes(c.runs, slices, nq, head_dim) > bytes) bytes = key_split_bytes(c.runs, slices, nq, head_dim);
     return bytes;
 }
@@ -229,7 +230,7 @@ extern "C" int fsta_attention_uses_workspace(int32_t batch, int32_t heads, int32
                                              int32_t dtype, int32_t block_m, int32_t max_ancestors, float sm_scale,
                                              uint32_t flags) {
     if (fsta_attention_workspace_bytes(batch, heads, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, flags) == 0) return 0;
-    const CachePlan c = plan_cache((int64_t)batch * heads, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+    const CachePlan c = plan_cache((int64_t)batch * heads, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, flags, false);
     return c.runs == 1 ? 0 : 1;
 }
 
@@ -311,7 +312,7 @@ extern "C" int fsta_attention_fwd_ws(const void* q, const void* k, const void* v
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (p.plan) {
-        const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, flags, false);
+        const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, flags, false);
         const size_t wanted = c.runs > 1 ? fsta_attention_workspace_bytes(batch, heads, nq, nk, head_dim, dtype, block_m, max_ancestors,
                                                                           sm_scale, flags) : 0;
         const int rc = launch_cache(p, dtype, out_dtype, head_dim, false, (flags & FSTA_FLAG_FAST_PV) != 0, c, workspace, workspace_bytes,
@@ -399,10 +400,9 @@ extern "C" int fsta_attention_fwd_kv8(const void* q, const void* k8, const void*
 
 extern "C" size_t fsta_attention_kv8_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk, int32_t head_dim,
                                                      int32_t dtype, int32_t block_m, int32_t max_ancestors, float sm_scale) {
-    (void)max_ancestors;
     if (batch <= 0 || heads <= 0 || nq <= 0 || nk <= nq || block_m <= 0) return 0;
     const int64_t slices = (int64_t)batch * heads;
-    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, 0, true);
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, 0, true);
     return c.runs > 1 ? key_split_bytes(c.runs, slices, nq, head_dim) : 0;
 }
 
@@ -453,7 +453,7 @@ extern "C" int fsta_attention_fwd_kv8_ws(const void* q, const void* k8, const vo
     p.k_scale = k_scale; p.v_scale = v_scale;
     p.merge_parts = 0; p.dry_run = 0; p.stream_mode = 0;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, sm_scale, 0, true);
+    const CachePlan c = plan_cache(slices, nq, nk, head_dim, dtype, block_m, max_ancestors, sm_scale, 0, true);
     const int rc = launch_cache(p, dtype, out_dtype, head_dim, true, false, c, workspace, workspace_bytes,
                                 c.runs > 1 ? key_split_bytes(c.runs, slices, nq, head_dim) : 0, s);
     if (rc != FSTA_EUNSUPPORTED) return rc;

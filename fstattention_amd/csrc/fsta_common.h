@@ -132,6 +132,8 @@ struct CachePlan {
     int run_tiles;      // prefix tiles per run (no run is empty)
 };
 bool cache_kernel_supported(int dtype, int head_dim, int block_m);
+// whether a launch by that plan fits the kernel's LDS (lists of max_anc slots), grid and 32-bit slice offsets
+bool cache_kernel_takes(int64_t slices, int nq, int nk, int head_dim, bool kv8, int max_anc, const CachePlan& plan);
 int launch_attention_cache(const AttnParams& p, int dtype, int head_dim, bool kv8, bool fast_pv, const CachePlan& plan,
                            hipStream_t stream);
 int launch_attention_mfma16_kv8(const AttnParams& p, int dtype, int head_dim, hipStream_t stream);

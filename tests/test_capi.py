@@ -196,6 +196,15 @@ def test_workspace_planning_is_host_arithmetic():
     assert size(1, 1, 32, 32 + 64, 64, _lib.F16, 32, 16, 0.1, _lib.flag_key_splits(9)) == 2 * 32 * (64 + 1) * 4
     assert size(0, 32, 256, 512, 128, _lib.BF16, 64, 64, 0.1, 0) == 0
     assert size(1, 32, 256, 100, 128, _lib.BF16, 64, 64, 0.1, 0) == 0
+    # a call of one run wants none although other kernels would .. as long as the kernel of that run takes its lists: with
+    # 3200 slots it does not (LDS), nor slices of 4 GiB
+    uses = lambda *a: lib.fsta_attention_uses_workspace(*a)
+    for slots, slices, prefix, used in ((64, 64, 1500, 0), (2700, 64, 1500, 0), (3200, 64, 1500, 1), (100000, 64, 1500, 1)):
+        shape = (1, slices, 64, 64 + prefix, 128, _lib.BF16, 32, slots, 0.1, 0)
+        assert size(*shape) > 0 and uses(*shape) == used, shape
+    kv8_size = lambda *a: lib.fsta_attention_kv8_workspace_bytes(*a)
+    assert kv8_size(1, 8, 64, 64 + 4096, 128, _lib.BF16, 32, 64, 0.1) > 0      # several runs
+    assert kv8_size(1, 8, 64, 64 + 4096, 128, _lib.BF16, 32, 3200, 0.1) == 0   # the kernel without runs
     # the workspace variant validates like the plain one, and wants an aligned workspace
     bad = lib.fsta_attention_fwd_ws(None, None, None, None, None, None, None, None, None, None, 0,
                                     1, 1, 16, 16, 64, 7, 7, 16, 8, 1, 1.0, 0, None, 0, None)

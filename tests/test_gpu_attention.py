@@ -1048,3 +1048,18 @@ def test_cache_kernel_keeps_a_rows_own_value_to_itself(storage, nodes, d, prefix
     from fstattention_amd import _lib
     assert "attn_cache_kernel" in _lib.load().fsta_last_attention_kernel().decode()
     torch.testing.assert_close(o.cpu().double(), want, atol=2e-3, rtol=2e-3, equal_nan=True)
+
+
+@pytest.mark.parametrize("slots,kernel", [(2720, "attn_cache_kernel"), (3200, "attn_mfma16_kernel")])
+def test_lists_too_long_for_the_cache_kernel_keep_their_key_runs(slots, kernel):
+    """Lists on both sides of what the LDS of the kernel for tree and prefix holds, in front of a prefix: the same result."""
+    parent = trees.random_recursive_parents(64, 8, window=16)
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32, max_anc=slots)
+    q, k, v = rand_qkv(1, 24, 64, 64 + 1500, 128, torch.bfloat16, 51)
+    want, _ = dense_oracle(q, k, v, parent, 0.1, prefix=1500)
+    a_idx, l_idx = shift_for_prefix(a_idx, l_idx, 1500)
+    from fstattention_amd import _lib
+    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), 0.1, BLOCK_M=32,
+                      MAX_ANCESTORS=slots, out_dtype=torch.float32)
+    assert kernel in _lib.load().fsta_last_attention_kernel().decode()
+    assert_close(o, want, torch.bfloat16, f"{slots} slots")
