@@ -126,19 +126,29 @@ constexpr CacheCost kCost16[2] = {{2.85f, 2.2f, 0.118f, 0.7f, 2.35f, 5.6f, 6.0f,
                                   {3.5f, 2.9f, 0.276f, 0.0f, 2.9f, 6.4f, 5.6f, 0.21f}};      // head_dim 128
 constexpr CacheCost kCost8[2] = {{3.2f, 2.3f, 0.106f, 0.67f, 2.06f, 3.2f, 4.0f, 0.17f},       // the same on 8-bit K/V
                                  {3.8f, 3.4f, 0.172f, 0.82f, 2.2f, 3.6f, 4.2f, 0.16f}};
-constexpr int kCacheMaxRows = 512;    // longer trees: their own kernels (a workgroup of the cache kernel reads the prefix for 32 rows)
+// Longer trees: 16-bit K/V go to the dense prefix kernel and the tree kernel, which read the prefix once per 128 and 64
+// rows; a workgroup of the cache kernel reads it for 32 rows.
+constexpr int kCacheMaxRows = 512;
+// 8-bit K/V have no other kernel with runs of keys: a workgroup of the tree kernel walks the whole prefix for one block.  It
+// is the faster one only where workgroups fill the GPU more than twice and the prefix is too short to pay for reading it once
+// per 32 rows instead of once per block (bf16, 64 slices, us, tree and cache kernel: 2048 rows in blocks of 128, head_dim
+// 128, behind 100 keys 65.3, 67.9, 700 keys 130, 126; 4096 shallow rows in blocks of 64, head_dim 64, behind 1 key 31.4, 35.6,
+// 100 keys 46.2, 44.7; blocks of 32: 1.0 to 4 times in favour of the cache kernel from one key on.  Elsewhere: 513 rows, 32
+// slices, 8192 keys, head_dim 128: 419, 153).
+constexpr int short_prefix8(int block_m) { return block_m == 128 ? 700 : block_m == 64 ? 100 : 0; }
 constexpr int kGpuCus = 256;
 
 CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, int block_m, int max_anc, float sm_scale,
                      uint32_t flags, bool kv8) {
     CachePlan c = {8, 0, 0};
     const int prefix = nk - nq;
-    if (slices <= 0 || nq <= 0 || prefix <= 0 || nq > kCacheMaxRows) return c;
+    if (slices <= 0 || nq <= 0 || prefix <= 0 || (nq > kCacheMaxRows && !kv8)) return c;
     if ((flags & (FSTA_FLAG_GENERIC | FSTA_FLAG_WIDE_WAVES | FSTA_FLAG_STREAM | FSTA_FLAG_SHARE_TILES)) || !(sm_scale > 0.f) ||
         !cache_kernel_supported(dtype, head_dim, block_m))
         return c;
     const int tiles = (prefix + kKeyTile - 1) / kKeyTile;
     const int64_t groups = (nq + 31) / 32, wgs1 = slices * groups;
+    if (kv8 && nq > kCacheMaxRows && wgs1 > 2 * kGpuCus && prefix < short_prefix8(block_m)) return c;
     if (!kv8) {
         // Enough rows and keys to be bound by the matrix cores: the dense prefix kernel, which shares every tile among 128
         // rows (256 rows, 32 slices, 16384 keys, bf16: 119 us against 139; 8192 keys: 76 against 74).

@@ -77,6 +77,18 @@ def test_prefix_remainders_and_runs(nodes, block_m, d, z, h, prefix):
     run_fp8(parent, block_m, z, h, d, torch.bfloat16 if nodes % 2 else torch.float16, 15, prefix=prefix)
 
 
+@pytest.mark.parametrize("nodes,block_m,d,h,prefix,kernel", [
+    (512, 64, 128, 2, 300, "cache"), (513, 64, 128, 2, 300, "cache"), (700, 32, 64, 30, 33, "cache"), (1500, 128, 64, 3, 2050, "cache"),
+    (1025, 64, 64, 17, 99, "mfma16"), (1025, 64, 64, 17, 100, "cache"), (650, 128, 128, 26, 699, "mfma16"), (650, 128, 128, 26, 700, "cache"),
+    (600, 128, 128, 25, 100, "cache")])
+def test_long_trees_behind_a_prefix(nodes, block_m, d, h, prefix, kernel):
+    """More than 512 rows: both kernels, on both sides of the rule that chooses."""
+    from fstattention_amd import _lib
+    parent = trees.random_recursive_parents(nodes, prefix, window=64)
+    run_fp8(parent, block_m, 1, h, d, torch.bfloat16 if nodes % 2 else torch.float16, 16, prefix=prefix)
+    assert f"attn_{kernel}_kernel" in _lib.load().fsta_last_attention_kernel().decode()
+
+
 def test_per_slice_scales_and_no_scales():
     parent = trees.medusa_parents(n=256, seed=77)
     run_fp8(parent, 64, 2, 4, 128, torch.bfloat16, 11, spread=64.0)
