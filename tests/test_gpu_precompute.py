@@ -179,9 +179,9 @@ def test_lineage_from_parents_on_gpu():
 @pytest.mark.parametrize("children", ["index", "light_first"])
 def test_dfs_order_on_gpu_matches_the_host_order(children):
     cases = [np.array([-1], dtype=np.int64), np.array([-1, -1, -1], dtype=np.int64)]
-    # up to 4096 nodes one workgroup does everything, beyond that six launches over arrays in device memory do
+    # up to 8192 nodes one workgroup does everything, beyond that six launches over arrays in device memory do
     for seed, n, window in [(1, 2, None), (2, 300, None), (3, 1500, 8), (4, 2049, 64), (5, 4096, 200),
-                            (6, 4097, 16), (7, 9000, None)]:
+                            (6, 4097, 16), (7, 9000, None), (8, 8192, 48), (9, 8193, 300), (10, 12000, 8)]:
         parent = trees.random_recursive_parents(n, seed, window)
         parent[::101] = -1                      # forest
         cases.append(parent)

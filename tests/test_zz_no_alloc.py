@@ -2,7 +2,8 @@
 
 Through the C ABI: same parent arrays, results compared bit for bit, two calls in a row with the
 second tree smaller than the first (the library's scratch array keeps the first call's contents).
-Both trees are larger than what the single-workgroup kernel takes, so both calls use the scratch.
+The single-workgroup kernel, which needs no scratch, takes up to 8192 nodes: wherever the scratch is the point, the trees
+are larger than that.
 """
 import numpy as np
 import pytest
@@ -33,7 +34,8 @@ def _order(lib, entry, parent, light_first, workspace):
 def test_static_scratch_entry_point_matches_the_workspace_one():
     lib = _lib.load()
     limit = 16384
-    for n, seed, window, light in ((12000, 5, 64, 1), (5000, 6, None, 0), (limit, 7, 8, 1), (4097, 8, 200, 0), (300, 9, 16, 1)):
+    for n, seed, window, light in ((12000, 5, 64, 1), (8193, 10, None, 0), (5000, 6, None, 0), (limit, 7, 8, 1), (9000, 11, 200, 0),
+                                   (4097, 8, 200, 0), (300, 9, 16, 1)):
         host_parent = trees.random_recursive_parents(n, seed, window)
         parent = torch.from_numpy(host_parent).cuda()
         work = torch.full((_lib.dfs_order_workspace_ints(n),), 0x5A5A5A5A, dtype=torch.int32, device="cuda")
@@ -46,16 +48,17 @@ def test_static_scratch_entry_point_matches_the_workspace_one():
     # beyond the array's size: refused on the host, nothing launched; a malformed tree is flagged as by the other entry point
     assert lib.fsta_dfs_order_static(parent.data_ptr(), limit + 1, 0, 8, 8, 8, None) == _lib.EUNSUPPORTED
     assert b"scratch" in lib.fsta_last_error()
-    bad = torch.from_numpy(trees.random_recursive_parents(6000, 3, 32)).cuda()
-    bad[100] = 5000
-    assert _order(lib, "static", bad, 0, None)[2] & _lib.PRE_BAD_NODE_ID
+    for n in (6000, 12000):
+        bad = torch.from_numpy(trees.random_recursive_parents(n, 3, 32)).cuda()
+        bad[100] = 5000
+        assert _order(lib, "static", bad, 0, None)[2] & _lib.PRE_BAD_NODE_ID
 
 
 def test_status_bits_of_an_earlier_stage_do_not_change_the_order():
     """Stages of a front-end chain may share one status word: a bit another stage left there says
-    nothing about this parent array, in the single-workgroup path (n <= 4096) and in the multi-launch one."""
+    nothing about this parent array, in the single-workgroup path (n <= 8192) and in the multi-launch one."""
     lib = _lib.load()
-    for n in (3000, 6000):
+    for n in (3000, 6000, 8193, 12000):
         host_parent = trees.random_recursive_parents(n, 11, 48)
         parent = torch.from_numpy(host_parent).cuda()
         perm = torch.full((n,), -7, dtype=torch.int64, device="cuda")
@@ -70,11 +73,11 @@ def test_status_bits_of_an_earlier_stage_do_not_change_the_order():
 
 
 def test_static_entry_point_recorded_into_a_graph():
-    """After one call outside capture (which looks the scratch array's address up), two calls -- the larger tree
-    first -- are captured into one HIP graph, replayed several times with eager work in between, and compared
-    with ``fsta_dfs_order`` after every replay."""
+    """After one call outside capture (which looks the scratch array's address up), three calls are captured into one HIP
+    graph, replayed several times with eager work in between, and compared with ``fsta_dfs_order`` after every replay: two
+    that share the scratch, the larger tree first, and one of a tree for the single-workgroup kernel."""
     lib = _lib.load()
-    trees_ = [trees.random_recursive_parents(n, seed, 64) for n, seed in ((9000, 21), (4500, 22))]
+    trees_ = [trees.random_recursive_parents(n, seed, 64) for n, seed in ((12000, 21), (9000, 22), (4500, 23))]
     parents = [torch.from_numpy(t).cuda() for t in trees_]
     want = []
     for p in parents:
