@@ -294,24 +294,41 @@ def test_dense_prefix_kernel_with_peaked_weights(dtype, scale):
     parent = trees.random_recursive_parents(256, 77, window=32)
     run_tree(parent, 64, 1, 4, 128, dtype, 23, prefix=4096, scale=scale)
     run_tree(parent, 128, 2, 2, 64, dtype, 24, prefix=2048, scale=scale)
+    # (few rows: the kernel for tree and prefix takes both; more than 512: the dense kernel, then the tree kernel)
+    parent = trees.random_recursive_parents(700, 78, window=32)
+    run_tree(parent, 64, 1, 2, 128, dtype, 25, prefix=4096, scale=scale, want_kernel="attn_mfma16_kernel")
+    run_tree(parent, 128, 1, 2, 64, dtype, 26, prefix=2050, scale=scale, want_kernel="attn_mfma16_kernel")
 
 
-def test_key_runs_native_output_type_and_workspace_contract():
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block_m,d", [(32, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("prefix,splits", [(300, 3), (1024, 4), (77, 2), (2000, None), (500, 1)])
+def test_key_runs_of_the_tree_kernel(dtype, block_m, d, prefix, splits):
+    """More than 512 rows behind a prefix too short for the dense kernel: runs of keys (or one) in the tree kernel itself."""
+    parent = trees.random_recursive_parents(600, 400 + d + block_m, window=48)
+    run_tree(parent, block_m, 1, 2, d, dtype, 14, prefix=prefix, key_splits=splits, want_kernel="attn_mfma16_kernel")
+
+
+@pytest.mark.parametrize("nodes,kernel", [(256, "attn_cache_kernel"), (600, "attn_mfma16_kernel")])
+def test_key_runs_native_output_type_and_workspace_contract(nodes, kernel):
     """Output in the storage type through the joining kernel; the C entry point with no or too
-    small a workspace runs unsplit; the workspace query is 0 where no split is planned."""
+    small a workspace runs unsplit; the workspace query is 0 where no split is planned.  Up to 512 rows the runs are
+    those of the kernel for tree and prefix, above the dense prefix kernel's."""
     from fstattention_amd import _lib
     from fstattention_amd.attention import _DTYPES, _packed_for
     lib = _lib.load()
     cfg = trees.config(2)
     prefix, m, d, h = 4096, cfg.block_m, cfg.head_dim, 4
-    a_idx, a_mask, l_idx, max_anc = oracle_inputs(cfg.parent, m)
+    parent = cfg.parent if nodes == 256 else trees.random_recursive_parents(nodes, 9, window=32)
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, m)
     nq = a_idx.shape[0] * m
     q, k, v = rand_qkv(1, h, nq, nq + prefix, d, torch.bfloat16, 21)
     scale = 1.0 / math.sqrt(d)
-    want, want_lse = dense_oracle(q, k, v, cfg.parent, scale, prefix=prefix, nq_pad=nq - len(cfg.parent))
+    want, want_lse = dense_oracle(q, k, v, parent, scale, prefix=prefix, nq_pad=nq - nodes)
     a_idx, l_idx = shift_for_prefix(a_idx, l_idx, prefix)
     qd, kd, vd, ad, md, ld = (t.cuda() for t in (q, k, v, a_idx, a_mask, l_idx))
     o, lse = fst_attention(qd, kd, vd, ad, md, ld, scale, BLOCK_M=m, MAX_ANCESTORS=max_anc, return_lse=True)
+    assert kernel in lib.fsta_last_attention_kernel().decode()
     assert o.dtype == torch.bfloat16
     # one rounding to bfloat16 on top of the float32 tolerance
     torch.testing.assert_close(o.cpu().double(), want, atol=2e-3 + 2 ** -8, rtol=2e-3 + 2 ** -8)
@@ -780,18 +797,21 @@ def test_hip_graph_replays_match_eager_calls():
     assert_close(out, want, cfg.dtype, "last replay")
 
 
-def test_hip_graph_replays_of_key_runs_match_eager_calls():
-    """A long shared prefix cut into runs of keys (dense prefix kernel, then the tree part that joins: two launches
-    and a workspace from torch's graph-private pool) captured into a HIP graph; replays on new q and new prefix
-    rows must give the eager results."""
+@pytest.mark.parametrize("nodes,kernel", [(256, "attn_cache_kernel"), (600, "attn_mfma16_kernel")])
+def test_hip_graph_replays_of_key_runs_match_eager_calls(nodes, kernel):
+    """A long shared prefix cut into runs of keys (256 rows: the kernel for tree and prefix, then the join of its runs; 600:
+    the dense prefix kernel, then the tree part that joins; two launches and a workspace from torch's graph-private pool)
+    captured into a HIP graph; replays on new q and new prefix rows must give the eager results."""
+    from fstattention_amd import _lib
     cfg = trees.config(2)
     m, d, prefix = cfg.block_m, cfg.head_dim, 3000
-    lineage, level = trees.lineage_from_parents(cfg.parent)
-    max_anc = trees.required_max_ancestors(cfg.parent, m)
+    parent = cfg.parent if nodes == 256 else trees.random_recursive_parents(nodes, 9, window=32)
+    lineage, level = trees.lineage_from_parents(parent)
+    max_anc = trees.required_max_ancestors(parent, m)
     a_idx, a_mask, l_idx = create_fst_attention_kernel_inputs(lineage.cuda(), level.cuda(), m, max_anc)
     a_idx, l_idx = shift_for_prefix(a_idx, l_idx, prefix)
     scale = 1.0 / math.sqrt(d)
-    q, k, v = (t.cuda() for t in rand_qkv(1, 2, cfg.n_nodes, prefix + cfg.n_nodes, d, cfg.dtype, 41))
+    q, k, v = (t.cuda() for t in rand_qkv(1, 2, nodes, prefix + nodes, d, cfg.dtype, 41))
 
     def step():
         return fst_attention(q, k, v, a_idx, a_mask, l_idx, scale, BLOCK_M=m, MAX_ANCESTORS=max_anc,
@@ -801,6 +821,7 @@ def test_hip_graph_replays_of_key_runs_match_eager_calls():
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(stream):
         step()
+        assert kernel in _lib.load().fsta_last_attention_kernel().decode()
         stream.synchronize()
         with torch.cuda.graph(graph, stream=stream):
             out = step()
@@ -814,7 +835,7 @@ def test_hip_graph_replays_of_key_runs_match_eager_calls():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), f"replay {replay} differs from the eager call"
-    want, _ = dense_oracle(q.cpu(), k.cpu(), v.cpu(), cfg.parent, scale, prefix=prefix)
+    want, _ = dense_oracle(q.cpu(), k.cpu(), v.cpu(), parent, scale, prefix=prefix)
     assert_close(out, want, cfg.dtype, "last replay")
 
 
