@@ -1,7 +1,8 @@
 // Scalar-ALU tree attention kernel: any of f32/f16/bf16, every head_dim and
-// block size the API admits.  It is the float32 path (float32 has no fast matrix
-// core format on gfx950) and a second, independently written implementation the
-// matrix-core kernel is cross-checked against.
+// block size the API admits.  It takes what the matrix-core kernels do not (head_dim
+// 16, float32 at head_dim 32, blocks of 16 rows in 16 bits, ancestor lists beyond
+// their LDS, scales that are not positive) and is the second, independently written
+// implementation they are cross-checked against.
 //
 // One workgroup owns one query block of one (batch, head) slice, as one Triton
 // program does in reference fstattention.py:42-45.  Keys are visited in tiles of

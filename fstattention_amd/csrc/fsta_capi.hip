@@ -112,8 +112,12 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
 // How the cache kernel (32 query rows per workgroup, tree and prefix in one launch) takes a launch: waves per workgroup
 // and runs of prefix tiles (runs = 0: not at all).  Shape and flags only.
 //
-// The number of runs is the one with the shortest predicted time.  The prediction, fitted to 650 timings over 8-256 rows,
-// 8-400 slices and 64-24000 keys (10 % mean error; the run count it picks costs 2 % over the best one):
+// The number of runs is the one with the shortest predicted time.  Over 45000 timings of 8500 shapes (8-512 rows, 8 bits
+// -1024, 8-400 slices, 64-24000 keys, every candidate forced) the prediction is off by 10-12 % on average with 16-bit K/V and
+// by 15-23 % with 8-bit (too long for fp16, which needs no second weight half); the run count it picks costs 3.4 % over the
+// best candidate on average, 10 % at the ninetieth percentile.  Where it is wrong: 64-127 workgroups of one row group behind
+// more than 1000 keys (one run, 20-27 % over the best on average, 67 % at worst: the bytes are priced at the whole GPU's rate,
+// which half of the CUs do not draw).  The prediction:
 //   1.6 (launch) + rounds of workgroups * start_end + the larger of
 //     workgroups on the fullest CU * tiles * tile   (a CU's matrix cores, L2 and LDS)      [us]
 //     rounds * tiles per wave * wave_tile           (one wave's chain)

@@ -1,6 +1,7 @@
-// PyTorch operator registration of the two entry points of the path (host code only, no kernels):
-//   torch.ops.fsta.attention_fwd(...)  ->  fsta_attention_fwd_ws / fsta_attention_fwd_kv8 of libfsta.so
+// PyTorch operator registration of the entry points of the path (host code only, no kernels):
+//   torch.ops.fsta.attention_fwd(...)  ->  fsta_attention_fwd_ws / fsta_attention_fwd_kv8_ws of libfsta.so
 //   torch.ops.fsta.precompute(...)     ->  fsta_precompute (reference utils.py:104-129)
+//   torch.ops.fsta.quantize_kv(...)    ->  fsta_quantize_fp8
 // on torch's current HIP stream of the tensors' device.  It does in C++ what the operator wrapper of
 // reference fstattention.py:153-181 does in Python (shape checks, allocation of o and L, launch), so
 // that an eager caller pays the dispatcher and one allocation per call instead of a page of Python.
