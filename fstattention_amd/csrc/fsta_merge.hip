@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_splits_kernel(
         for (int i = 0; i < 4; ++i) acc[i] *= old;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            if (s0 + u >= splits) break;        // (the same in every lane; a repeated infinity under weight 0 would be a NaN)
+            if (s0 + u >= splits) x[u] = float4{0.f, 0.f, 0.f, 0.f};      // (a repeated infinity under weight 0 would be a NaN)
             const float w = exp2f(l[u] - safe);
             acc[0] += w * x[u].x; acc[1] += w * x[u].y; acc[2] += w * x[u].z; acc[3] += w * x[u].w;
             sum += w;
