@@ -168,6 +168,9 @@ def _packed_for(ancestor_idx: torch.Tensor, ancestor_mask, leaf_idx: torch.Tenso
     return packed
 
 
+# torch.compile follows Python code up to the first C function it does not know
+_tracing = torch.compiler.is_dynamo_compiling
+
 _FP8 = torch.float8_e4m3fn
 _FP8_MAX = 448.0
 
@@ -181,10 +184,8 @@ def quantize_kv_fp8(k: torch.Tensor, v: torch.Tensor):
     traced, fake, batched by ``vmap`` --, differentiated in either direction) go through the same steps as tensor
     operations.  Those give the kernel's bytes on the GPU; on the host, where torch divides by 448 instead of multiplying by
     the rounded 1/448, a scale may differ by one unit in the last place."""
-    if k.is_cuda and not torch.compiler.is_compiling() and (_CALLS or _calls()).plain_tensors(k, v) and k.dim() == 4 and \
-            v.device == k.device and v.shape == k.shape and v.dtype == k.dtype and k.dtype in _DTYPES and \
-            k.shape[2] * k.shape[3] % 16 == 0 and k.numel() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0:
-        return (_OPS or _ops()).quantize_kv(k, v)
+    if not _tracing() and (_CALLS or k.is_cuda) and (_CALLS or _calls()).quantizes(k, v):
+        return _OPS.quantize_kv(k, v)
 
     def one(t):
         amax = t.float().abs().amax(dim=(2, 3))
@@ -308,7 +309,7 @@ def shift_for_prefix(ancestor_idx: torch.Tensor, leaf_idx: torch.Tensor, prefix:
     packed inputs with the shift noted, so that they stay valid for the shifted tensors.
     """
     shifted = NotImplemented
-    if ancestor_idx.is_cuda and not torch.compiler.is_compiling():      # one launch for both
+    if not _tracing() and (_CALLS or ancestor_idx.is_cuda):      # one launch for both
         shifted = (_CALLS or _calls()).shift_index(ancestor_idx, leaf_idx, prefix)
     if shifted is NotImplemented:       # (on the host, other integer types, traced)
         shifted = (torch.where(ancestor_idx >= 0, ancestor_idx + prefix, ancestor_idx),

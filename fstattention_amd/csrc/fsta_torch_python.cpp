@@ -110,6 +110,19 @@ PyObject* recall(PyObject* mask_obj, const at::Tensor& mask, const at::Tensor& a
     return PyTuple_GET_ITEM(entry, 2);
 }
 
+// Profilers and other observers see a call under the name of the registered operator
+__attribute__((noinline)) void report(c10::optional<at::RecordFunction>& seen, at::StepCallbacks&& callbacks, const at::Tensor& q,
+                                      const at::Tensor& k, const at::Tensor& v, const at::Tensor& a_idx, const Packed& p,
+                                      const at::Tensor& l_idx) {
+    seen.emplace(std::move(callbacks));
+    if (seen->needsInputs()) {
+        const c10::IValue inputs[] = {q, k, v, a_idx, *p.bits, *p.count, l_idx};
+        seen->before("fsta::attention_fwd", c10::ArrayRef<const c10::IValue>(inputs, 7));
+    } else {
+        seen->before("fsta::attention_fwd");
+    }
+}
+
 // attention(q, k, v, ancestor_idx, ancestor_mask, leaf_idx, sm_scale, BLOCK_M, MAX_ANCESTORS, out_dtype, return_lse, flags,
 //           k_scale, v_scale): attention.fst_attention with its switches as FSTA_FLAG_* bits
 PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -159,17 +172,9 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
             (i ? v_scale : k_scale) = *s;
         }
     try {
-        // profilers and other observers see the call under the name of the registered operator
         c10::optional<at::RecordFunction> seen;
-        if (auto callbacks = at::getStepCallbacksUnlessEmpty(at::RecordScope::FUNCTION)) {
-            seen.emplace(std::move(*callbacks));
-            if (seen->needsInputs()) {
-                const c10::IValue inputs[] = {*q, *k, *v, *a_idx, *p.bits, *p.count, *l_idx};
-                seen->before("fsta::attention_fwd", c10::ArrayRef<const c10::IValue>(inputs, 7));
-            } else {
-                seen->before("fsta::attention_fwd");
-            }
-        }
+        if (auto callbacks = at::getStepCallbacksUnlessEmpty(at::RecordScope::FUNCTION))
+            report(seen, std::move(*callbacks), *q, *k, *v, *a_idx, p, *l_idx);
         const auto out = fsta_torch::attention_fwd(*q, *k, *v, *a_idx, *p.bits, *p.count, *l_idx,
                                                    p.plan ? c10::optional<at::Tensor>(*p.plan) : c10::nullopt, p.key_shift, sm_scale,
                                                    block_m, max_anc, out_code, return_lse, flags, k_scale, v_scale);
@@ -369,17 +374,23 @@ PyObject* shift_index(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
-// plain_tensors(a, b): True if an operator whose only implementation is a kernel may take both: ordinary GPU tensors that
-// nobody transforms, traces below the dispatcher or differentiates, in either direction.  (A mode that watches calls from
-// Python, such as a default device, sees the operator as any other.)
-PyObject* plain_tensors(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+// quantizes(k, v): True if the operator for the 8-bit storage, whose only implementation is a kernel, takes both: ordinary GPU
+// tensors of one shape and type, in slices of whole 16-byte pieces, that nobody transforms, traces below the dispatcher or
+// differentiates, in either direction.  (A mode that watches calls from Python, such as a default device, sees the operator.)
+PyObject* quantizes(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK_TYPE(n_args == 2, "plain_tensors takes 2 arguments");
+    TORCH_CHECK_TYPE(n_args == 2, "quantizes takes 2 arguments");
     if (!plain_dispatch()) Py_RETURN_FALSE;
+    const at::Tensor* t[2];
     for (int i = 0; i < 2; ++i) {
-        const at::Tensor* t = gpu_tensor(args[i]);
-        if (!t || (c10::GradMode::is_enabled() && wants_grad(*t)) || t->_fw_grad(0).defined()) Py_RETURN_FALSE;
+        t[i] = gpu_tensor(args[i]);
+        if (!t[i] || (c10::GradMode::is_enabled() && wants_grad(*t[i])) || t[i]->_fw_grad(0).defined()) Py_RETURN_FALSE;
     }
+    const at::Tensor &k = *t[0], &v = *t[1];
+    if (k.dim() != 4 || v.sizes() != k.sizes() || v.device() != k.device() || v.scalar_type() != k.scalar_type() ||
+        fsta_torch::dtype_code(k.scalar_type()) < 0 || k.numel() == 0 || k.size(2) * k.size(3) % 16 != 0 ||
+        (uintptr_t)k.data_ptr() % 16 != 0 || (uintptr_t)v.data_ptr() % 16 != 0)
+        Py_RETURN_FALSE;
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -403,7 +414,7 @@ PyMethodDef kMethods[] = {
     FSTA_FASTCALL(inputs_from_parents),
     FSTA_FASTCALL(medusa_parents),
     FSTA_FASTCALL(shift_index),
-    FSTA_FASTCALL(plain_tensors),
+    FSTA_FASTCALL(quantizes),
     {"setup", &setup, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -86,7 +86,7 @@ def test_quantize_under_transforms_matches_the_kernel():
     assert quantize_kv_fp8(x, v[0].float())[2].requires_grad
     with torch.inference_mode():      # the usual way to serve: the kernel
         _same_bytes(quantize_kv_fp8(k[0], v[0]), want[0])
-        assert attention_module._CALLS.plain_tensors(k, v)
+        assert attention_module._CALLS.quantizes(k[0], v[0])
 
 
 @pytest.mark.gpu
@@ -105,7 +105,7 @@ def test_quantize_as_tensor_operations_gives_the_same_bytes(dtype):
     assert torch.ops.fsta.quantize_kv.default not in seen
     _same_bytes(quantize_kv_fp8(k, v), steps)
     with torch.device("cuda"):      # (a mode that watches calls from Python: the kernel)
-        assert attention_module._CALLS.plain_tensors(k, v)
+        assert attention_module._CALLS.quantizes(k, v)
         _same_bytes(quantize_kv_fp8(k, v), steps)
 
 
