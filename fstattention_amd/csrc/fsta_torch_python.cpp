@@ -300,6 +300,11 @@ PyObject* inputs_from_parents(PyObject*, PyObject* const* args, Py_ssize_t n_arg
     TORCH_CHECK_VALUE(block_m > 0 && block_m <= INT32_MAX && max_anc > 0 && max_anc <= INT32_MAX && width > 0,
                       "block_m, max_ancestors and width must be positive");
     const OnStream on(parent);
+    if (check) {      // (before anything is recorded: a replay would report into memory that has gone to others)
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        TORCH_CHECK(hipStreamIsCapturing(on.stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone,
+                    "kernel_inputs_from_parents_gpu: check=True waits for the GPU, which a stream that is being captured does not");
+    }
     const int64_t nb = (n + block_m - 1) / block_m;
     at::Tensor a_idx = fresh({nb, max_anc}, at::kLong, parent), l_idx = fresh({nb, block_m}, at::kLong, parent), a_mask, lineage, level, plan;
     if (want_mask) a_mask = fresh({nb, block_m, max_anc}, at::kBool, parent);

@@ -452,3 +452,24 @@ def test_shift_for_prefix_on_device_and_host_tensors():
     for x, y in ((a, b), (a.cuda(), b.cuda()), (a.cuda().t(), b.cuda()), (a.cuda()[:0], b.cuda())):
         for got, src in zip(shift_for_prefix(x, y, 1000), (x, y)):
             assert torch.equal(got, torch.where(src >= 0, src + 1000, src))
+
+
+def test_kernel_inputs_from_parents_refuses_to_wait_inside_a_capture():
+    """``check=True`` waits for words the kernel writes into host memory.  Inside a capture it raises before anything is
+    recorded; the capture goes on and its replay gives what ``check=False`` recorded."""
+    parent = torch.from_numpy(trees.random_recursive_parents(200, 4, 16)).cuda()
+    want = kernel_inputs_from_parents_gpu(parent, 64, 160, 100)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        kernel_inputs_from_parents_gpu(parent, 64, 160, 100, check=False)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            with pytest.raises(RuntimeError, match="captured"):
+                kernel_inputs_from_parents_gpu(parent, 64, 160, 100)
+            got = kernel_inputs_from_parents_gpu(parent, 64, 160, 100, check=False)
+    for _ in range(2):
+        got[0].fill_(-7)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2]) and int(got[3].item()) == 0
