@@ -263,7 +263,9 @@ extern "C" int fsta_quantize_fp8(const void* a, const void* b, void* a8, void* b
     if (misaligned(a_scale, 4) || misaligned(b_scale, 4) || misaligned(workspace, 4))
         return fail(FSTA_EINVAL, "fsta_quantize_fp8: scales and workspace must be 4-byte aligned");
     const int64_t pieces = pieces_of(elements);
-    if (2 * slices * pieces > 0x7fffffff)
+    // (a grid ends at 2^32 threads)
+    if (slices > 0x7fffffff || pieces > 0x7fffffff ||
+        2.0 * (double)slices * (one_launch(elements, dtype) ? (double)kOneThreads : (double)pieces * kThreads) >= 4294967296.0)
         return fail(FSTA_EUNSUPPORTED, "fsta_quantize_fp8: %lld slices of %lld elements", (long long)slices, (long long)elements);
     const size_t need = fsta_quantize_workspace_bytes(slices, elements, dtype);
     if (need && (!workspace || workspace_bytes < need))

@@ -394,6 +394,7 @@ PyObject* quantizes(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor &k = *t[0], &v = *t[1];
     if (k.dim() != 4 || v.sizes() != k.sizes() || v.device() != k.device() || v.scalar_type() != k.scalar_type() ||
         fsta_torch::dtype_code(k.scalar_type()) < 0 || k.numel() == 0 || k.size(2) * k.size(3) % 16 != 0 ||
+        k.size(0) * k.size(1) > (int64_t)1 << 20 ||      // (a workgroup of 1024 threads per slice of both: a grid ends at 2^32)
         (uintptr_t)k.data_ptr() % 16 != 0 || (uintptr_t)v.data_ptr() % 16 != 0)
         Py_RETURN_FALSE;
     Py_RETURN_TRUE;

@@ -109,6 +109,18 @@ def test_quantize_as_tensor_operations_gives_the_same_bytes(dtype):
         _same_bytes(quantize_kv_fp8(k, v), steps)
 
 
+@pytest.mark.gpu
+def test_quantize_of_more_slices_than_a_grid_holds():
+    g = torch.Generator(device="cuda").manual_seed(6)
+    k = torch.randn((1 << 21, 1, 1, 16), generator=g, device="cuda").to(torch.bfloat16)
+    part = [k[:1 << 20].contiguous(), k[1 << 20:].contiguous()]
+    assert not attention_module._calls().quantizes(k, k) and attention_module._calls().quantizes(*part)
+    k8, v8, k_scale, v_scale = quantize_kv_fp8(k, k)      # tensor operations
+    a8, b8, a_scale, b_scale = quantize_kv_fp8(*part)     # the kernel
+    _same_bytes((k8, k_scale), (torch.cat([a8.view(torch.uint8), b8.view(torch.uint8)]).view(k8.dtype), torch.cat([a_scale, b_scale])))
+    _same_bytes((v8, v_scale), (k8, k_scale))
+
+
 def test_shift_is_traceable_and_needs_no_library_on_the_host(monkeypatch):
     a_idx = torch.arange(12).view(2, 6) - 3
     l_idx = torch.arange(8).view(2, 4) - 1

@@ -166,6 +166,16 @@ def test_tree_builder_rejects_bad_arguments_before_any_gpu_work():
     assert ws(8, _lib.F64, 0, 10, 5, 8, 8, None, 0, None) == _lib.EINVAL      # small problems: the checks of fsta_medusa_tree
 
 
+def test_quantize_refuses_grids_that_do_not_exist():
+    lib = _lib.load()
+    call = lambda slices, elements, work=1 << 60: lib.fsta_quantize_fp8(16, 16, 16, 16, 16, 16, slices, elements, _lib.BF16, 16, work, None)
+    assert call(1 << 21, 16) == _lib.EUNSUPPORTED                    # 2 x 2^21 workgroups of 1024 threads
+    assert call(1 << 20, 1 << 17) == _lib.EUNSUPPORTED               # 2 x 2^20 x 16 workgroups of 256
+    assert call(1, 1 << 50) == _lib.EUNSUPPORTED
+    assert call(1 << 21, 24) == _lib.EINVAL                          # not whole 16-byte pieces
+    assert call(1, 1 << 17, 4) == _lib.EINVAL and b"workspace" in lib.fsta_last_error()
+
+
 def test_workspace_planning_is_host_arithmetic():
     """How a shared prefix is cut into runs of keys depends on the shape and flags only."""
     lib = _lib.load()
