@@ -180,7 +180,7 @@ def quantize_kv_fp8(k: torch.Tensor, v: torch.Tensor):
     ``float8_e4m3fn`` tensors and one float32 scale per (batch, head) slice (``[Z*H]``) chosen so that
     the slice's largest magnitude maps to the format's largest value (448).  ``k8 * k_scale`` is the K
     the kernel computes with.  On the GPU one or two launches of a kernel of the library; tensors it does not take (on
-    the host, float64, of different shapes, slices that are no multiple of 16 elements, without memory of their own --
+    the host, float64, of different shapes, slices that are no multiple of 16 elements or more than 2**20 of them, without memory of their own --
     traced, fake, batched by ``vmap`` --, differentiated in either direction) go through the same steps as tensor
     operations.  Those give the kernel's bytes on the GPU; on the host, where torch divides by 448 instead of multiplying by
     the rounded 1/448, a scale may differ by one unit in the last place."""
