@@ -595,7 +595,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
         T* dst = static_cast<T*>(p.o) + out_row * D + piece0 * 4;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            const u32x2 packed = {MM::pack(acc[i][0], acc[i][1]), MM::pack(acc[i][2], acc[i][3])};
+            const u32x2 packed = {MM::pack_out(acc[i][0], acc[i][1]), MM::pack_out(acc[i][2], acc[i][3])};
             *reinterpret_cast<u32x2*>(dst + 4 * i) = packed;
         }
     }

@@ -474,7 +474,7 @@ __global__ __launch_bounds__(M * 2 * key_split_for(M), 2) void attn_mfma_kernel(
                 if (p.out_f32) {
                     *reinterpret_cast<float4*>(static_cast<float*>(p.o) + base + d) = val;
                 } else {
-                    const u32x2 packed = {MM::pack(val.x, val.y), MM::pack(val.z, val.w)};
+                    const u32x2 packed = {MM::pack_out(val.x, val.y), MM::pack_out(val.z, val.w)};
                     *reinterpret_cast<u32x2*>(static_cast<T*>(p.o) + base + d) = packed;
                 }
             }

@@ -886,7 +886,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
             for (int i = 0; i < kTilesHere; ++i) {
                 // accumulator rows 4g .. 4g+3 of a tile are 4 consecutive head dims
                 const f32x4& acc = vals[i];
-                const u32x2 packed = {MM::pack(acc[0] * inv, acc[1] * inv), MM::pack(acc[2] * inv, acc[3] * inv)};
+                const u32x2 packed = {MM::pack_out(acc[0] * inv, acc[1] * inv), MM::pack_out(acc[2] * inv, acc[3] * inv)};
                 *reinterpret_cast<u32x2*>(stage + ql * kStageStride + (16 * i + 4 * g) * 2) = packed;
             }
             __builtin_amdgcn_wave_barrier();

@@ -590,8 +590,8 @@ __global__ __launch_bounds__(M * 4, 4) void attn_stream_kernel(AttnParams p, int
                     for (int a = 0; a < kOTiles / 2; ++a) {
                         const f32x4& x = o[2 * a];
                         const f32x4& y = o[2 * a + 1];
-                        const uint32_t x0 = MM::pack(x[0] * inv, x[1] * inv), x1 = MM::pack(x[2] * inv, x[3] * inv);
-                        const uint32_t y0 = MM::pack(y[0] * inv, y[1] * inv), y1 = MM::pack(y[2] * inv, y[3] * inv);
+                        const uint32_t x0 = MM::pack_out(x[0] * inv, x[1] * inv), x1 = MM::pack_out(x[2] * inv, x[3] * inv);
+                        const uint32_t y0 = MM::pack_out(y[0] * inv, y[1] * inv), y1 = MM::pack_out(y[2] * inv, y[3] * inv);
                         const u32x2 s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
                         const u32x2 s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
                         const uint32_t a0 = s0[0], b0 = s0[1], a1 = s1[0], b1 = s1[1];
