@@ -155,13 +155,26 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
     const int slice_bytes = (int)((uint32_t)p.nk * (uint32_t)kRowBytes);
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kb), 0, slice_bytes, kRawBuffer);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vb), 0, slice_bytes, kRawBuffer);
+    // Row groups that walk a run in step ask for the same keys at the same time: 256 workgroups of eight groups have 4 MB of
+    // distinct bytes on their way, which at 2 us to HBM and back is 2.1 TB/s (a probe with nothing but such transfers; pairs:
+    // 5.5).  So every other group takes the rounds of a run (a tile per wave) two by two in the other order: twice the bytes on
+    // their way, and what one group fetched from memory its neighbour finds in L2 a round later.  Measured with K and V in HBM,
+    // as a step through a model's layers finds them (32 slices, bf16, D 128): 256 rows behind 600, 1100, 6000 keys 12.0 ->
+    // 10.3, 16.3 -> 14.6, 54.0 -> 51.7 us, 130 rows, 1100 keys 16.0 -> 14.4; with K and V in the Infinity Cache, where the way is
+    // short, 0-3 % slower.  Two to four groups have enough on their way (128 rows, 2000 keys: 4 % slower, 61 rows: 7 %); whole
+    // runs or four rounds in other orders bring more at once and overfill the L2; 8-bit tiles are half as large and their
+    // arithmetic is longer than the way (no gain).
+    const bool swapped = !KV8 && gr.chunks >= 5 && (chunk & 1);
+    const int pairs_end = n_pfx / (2 * kWaves) * (2 * kWaves);
+    auto prefix_tile = [&](int t) { return first_tile + (swapped && t < pairs_end ? t ^ kWaves : t); };
     int n_anc_tiles = 0;                     // the list is [prefix tiles | ancestor tiles | the rows' own keys]
     auto issue = [&](int t, int slot) {
         unsigned char* dst = ring + slot * 2 * kHalf;
-        if (t < n_pfx && (first_tile + t + 1) * kTileN <= p.prefix) {
+        const int pt = prefix_tile(t);
+        if (t < n_pfx && (pt + 1) * kTileN <= p.prefix) {
             // 32 consecutive rows: one uniform offset, lane offsets that never change.  Buffer addressing takes both as they
             // are (a flat address is 64-bit vector arithmetic per transfer: 8192 keys in 8 bits 35.3 us, 33.9 this way).
-            const uint32_t tile_off = (uint32_t)(first_tile + t) * (uint32_t)kHalf;
+            const uint32_t tile_off = (uint32_t)pt * (uint32_t)kHalf;
 #pragma unroll
             for (int i = 0; i < 2 * kDma; ++i)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(i < kDma ? k_rsrc : v_rsrc, (void __attribute__((address_space(3)))*)(dst + i * 1024), 16,
@@ -171,7 +184,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
             int rows[kDma];
             if (t < n_pfx) {
 #pragma unroll
-                for (int i = 0; i < kDma; ++i) rows[i] = min((first_tile + t) * kTileN + i * kRowsPerDma + dma_row, p.prefix - 1);
+                for (int i = 0; i < kDma; ++i) rows[i] = min(pt * kTileN + i * kRowsPerDma + dma_row, p.prefix - 1);
             } else {
                 const int ta = t - n_pfx;
                 const uint32_t keys = lds_addr(ta < n_anc_tiles ? plan_s + kPlanHeaderWords + ta * kTileN : group_s) + dma_row * 4;
@@ -367,8 +380,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
         f32x16 s = scores();
         // mask: none for whole prefix tiles (uniform branch)
         uint32_t word = 0xffffffffu;
-        if (t >= n_pfx || (first_tile + t + 1) * kTileN > p.prefix) {
-            if (t < n_pfx) word = (1u << (p.prefix - (first_tile + t) * kTileN)) - 1u;
+        const int pt = prefix_tile(t);
+        if (t >= n_pfx || (pt + 1) * kTileN > p.prefix) {
+            if (t < n_pfx) word = (1u << (p.prefix - pt * kTileN)) - 1u;
             else word = group_s[kTileN + (t - n_pfx) * kTileN + ql];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {

@@ -284,6 +284,19 @@ def test_cache_kernel_edges(dtype, nodes, block_m, d, z, h, prefix, splits):
              want_kernel="attn_cache_kernel")
 
 
+@pytest.mark.parametrize("nodes,d,h,prefix,splits", [
+    (160, 128, 2, 511, 1),                  # five row groups, eight waves: a pair of rounds is 512 keys; one key short of it
+    (160, 64, 2, 512, 1),
+    (288, 128, 1, 513, 1),                  # nine row groups, one key more
+    (288, 64, 2, 1200, 1),                  # two pairs of rounds and a rest
+    (256, 128, 2, 1700, 3),                 # 18 tiles a run: a pair and two tiles; the last run one tile shorter
+    (160, 128, 60, 257, 1)])                # more workgroups than CUs: four waves, a pair is 256 keys
+def test_cache_kernel_row_groups_in_different_order(nodes, d, h, prefix, splits):
+    """Five and more row groups: every other one takes the rounds of a run two by two in the other order."""
+    parent = trees.random_recursive_parents(nodes, nodes + prefix, window=24)
+    run_tree(parent, 32, 1, h, d, torch.bfloat16, 6, prefix=prefix, key_splits=splits, want_kernel="attn_cache_kernel")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("scale", [0.3, 1.0])
 def test_dense_prefix_kernel_with_peaked_weights(dtype, scale):
