@@ -7,7 +7,11 @@
 // them again (what the 256 MB Infinity Cache still holds does not come from HBM a second time), joins the maxima of its
 // slice (at most a few hundred words) and writes the bytes.  The second reading and the bytes go past the caches, so that
 // they do not drive out what is still to be read (K and V of 32 heads x 8192 keys x 128, bf16: 58.0 -> 53.0 us by the
-// stores, 50.8 with the loads and pieces of half the size).
+// stores, 50.8 with the loads and pieces of half the size).  Pieces are 16 KB, one unit of 16 elements for each of 512
+// threads: 48.6 us (256 threads with two units 50.6, 512 with two 50.4, 256 with one 49.6, 1024 with one 51.8).  Both launches
+// deal the same pieces to the same workgroup numbers, hence XCDs: with pieces of another size in the second one its reading
+// misses what the first left in the XCD's L2 (8 heads, 33 MB: 12.7 us against 16.1).  Several pieces per workgroup with the
+// next one's loads in flight: 53 to 57 us (half the waves by their registers).
 #include "fsta_common.h"
 
 namespace fsta {
@@ -16,8 +20,7 @@ namespace {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kFp8Max = 448.f;
-constexpr int kThreads = 256;            // two launches: threads per piece
-constexpr int kUnits = 2;                // units of 16 elements per thread and piece
+constexpr int kThreads = 512;            // two launches: threads per piece, a unit of 16 elements each
 constexpr int kOneThreads = 1024;        // one launch: threads per slice
 constexpr int kUnitElems = 16;
 
@@ -96,30 +99,37 @@ __device__ __forceinline__ Scale make_scale(float amax) {
     return sc;
 }
 // x / s, correctly rounded: with inv = 1/s correctly rounded, one residual step on x * inv gives the rounded quotient
-// (Markstein); 3 instructions in place of the ten of a full division.  The sign of a zero is x's.
+// (Markstein); 3 instructions in place of the ten of a full division.  A zero loses its sign.
 __device__ __forceinline__ float divide(float x, const Scale& sc) {
     const float q0 = x * sc.inv;
-    const float q = __builtin_fmaf(__builtin_fmaf(-q0, sc.s, x), sc.inv, q0);
-    return __builtin_copysignf(q, x);
+    return __builtin_fmaf(__builtin_fmaf(-q0, sc.s, x), sc.inv, q0);
+}
+// The signs of elements 4w .. 4w+3 in bit 7 of their bytes (the scale is positive: they are the bytes' signs, zeros' and
+// NaNs' too; two instructions for four elements instead of one each).
+template <typename T> __device__ __forceinline__ uint32_t signs(const Unit<T>& u, int w) {
+    if constexpr (sizeof(T) == 4) {
+        const uint32_t a = u.w[w][0], b = u.w[w][1], c = u.w[w][2], d = u.w[w][3];
+        return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d, c, 0x07030c0cu), __builtin_amdgcn_perm(b, a, 0x0c0c0703u), 0x07060100u) &
+               0x80808080u;
+    } else {
+        const uint32_t a = u.w[w / 2][2 * (w % 2)], b = u.w[w / 2][2 * (w % 2) + 1];
+        return __builtin_amdgcn_perm(b, a, 0x07050301u) & 0x80808080u;
+    }
 }
 // PAST: around the caches
-template <bool PAST, typename T> __device__ __forceinline__ void store_unit(const Unit<T>& u, const Scale& sc, uint8_t* dst) {
+template <bool PAST, typename T>
+__device__ __forceinline__ void store_unit(const Unit<T>& u, const Scale& sc, const T* src, uint8_t* dst) {
+    if (!sc.plain) {      // (rare, and kept short: element by element from memory)
+#pragma unroll 1
+        for (int i = 0; i < kUnitElems; ++i) dst[i] = (uint8_t)fp8_any(to_float(src[i]) / sc.s);
+        return;
+    }
     u32x4 out;
-    if (sc.plain) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            int pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w), sc), divide(unit_value(u, 4 * w + 1), sc), 0, false);
-            pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w + 2), sc), divide(unit_value(u, 4 * w + 3), sc), pk, true);
-            out[w] = (uint32_t)pk;
-        }
-    } else {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            uint32_t pk = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= fp8_any(unit_value(u, 4 * w + e) / sc.s) << (8 * e);
-            out[w] = pk;
-        }
+    for (int w = 0; w < 4; ++w) {
+        int pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w), sc), divide(unit_value(u, 4 * w + 1), sc), 0, false);
+        pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w + 2), sc), divide(unit_value(u, 4 * w + 3), sc), pk, true);
+        out[w] = ((uint32_t)pk & 0x7f7f7f7fu) | signs(u, w);
     }
     if constexpr (PAST) __builtin_nontemporal_store(out, reinterpret_cast<u32x4*>(dst));
     else *reinterpret_cast<u32x4*>(dst) = out;
@@ -164,11 +174,14 @@ __global__ __launch_bounds__(kOneThreads) void quantize_slice_kernel(QuantArgs a
     uint8_t* dst = (tensor ? a.dst[1] : a.dst[0]) + (size_t)slice * a.elems;
 #pragma unroll
     for (int i = 0; i < N; ++i)
-        if (tid + i * kOneThreads < units) store_unit<false>(u[i], sc, dst + (size_t)(tid + i * kOneThreads) * kUnitElems);
+        if (tid + i * kOneThreads < units) {
+            const size_t at = (size_t)(tid + i * kOneThreads) * kUnitElems;
+            store_unit<false>(u[i], sc, src + at, dst + at);
+        }
     if (tid == 0) (tensor ? a.scale[1] : a.scale[0])[slice] = sc.s;
 }
 
-// Workgroup -> (tensor, slice, piece); the piece's units of this thread, kThreads apart.
+// Workgroup -> (tensor, slice, piece), thread -> unit.
 template <typename T, bool WRITE>
 __global__ __launch_bounds__(kThreads) void quantize_pieces_kernel(QuantArgs a) {
     __shared__ uint32_t wave_mx[kThreads / 64];
@@ -177,19 +190,15 @@ __global__ __launch_bounds__(kThreads) void quantize_pieces_kernel(QuantArgs a) 
     const int tensor = row >= (unsigned)a.slices;
     const int slice = (int)row - tensor * a.slices, tid = threadIdx.x;
     const T* src = static_cast<const T*>(tensor ? a.src[1] : a.src[0]) + (size_t)slice * a.elems;
-    const int64_t units = a.elems / kUnitElems, first = (int64_t)piece * (kThreads * kUnits) + tid;
-    Unit<T> u[kUnits];
-#pragma unroll
-    for (int i = 0; i < kUnits; ++i)
-        if (first + i * kThreads < units) u[i] = load_unit<WRITE>(src + (first + i * kThreads) * kUnitElems);
+    const int64_t at = ((int64_t)piece * kThreads + tid) * kUnitElems;
+    Unit<T> u;
     uint32_t mx = 0;
-    if constexpr (!WRITE) {
-#pragma unroll
-        for (int i = 0; i < kUnits; ++i)
-            if (first + i * kThreads < units) mx = max(mx, unit_max(u[i]));
-    } else {
-        for (int i = tid; i < a.pieces; i += kThreads) mx = max(mx, a.part[(size_t)row * a.pieces + i]);
+    if (at < a.elems) {
+        u = load_unit<WRITE>(src + at);
+        if constexpr (!WRITE) mx = unit_max(u);
     }
+    if constexpr (WRITE)
+        for (int i = tid; i < a.pieces; i += kThreads) mx = max(mx, a.part[(size_t)row * a.pieces + i]);
     mx = wave_max(mx);
     if ((tid & 63) == 0) wave_mx[tid >> 6] = mx;
     __syncthreads();
@@ -200,9 +209,7 @@ __global__ __launch_bounds__(kThreads) void quantize_pieces_kernel(QuantArgs a) 
     } else {
         const Scale sc = make_scale(from_bits<T>(mx));
         uint8_t* dst = (tensor ? a.dst[1] : a.dst[0]) + (size_t)slice * a.elems;
-#pragma unroll
-        for (int i = 0; i < kUnits; ++i)
-            if (first + i * kThreads < units) store_unit<true>(u[i], sc, dst + (first + i * kThreads) * kUnitElems);
+        if (at < a.elems) store_unit<true>(u, sc, src + at, dst + at);
         if (tid == 0 && piece == 0) (tensor ? a.scale[1] : a.scale[0])[slice] = sc.s;
     }
 }
@@ -212,7 +219,7 @@ __global__ __launch_bounds__(kThreads) void quantize_pieces_kernel(QuantArgs a) 
 template <typename T> constexpr int one_launch_units() { return 64 / (4 * Unit<T>::kWords) < 4 ? 64 / (4 * Unit<T>::kWords) : 4; }
 
 int64_t pieces_of(int64_t elems) {
-    const int64_t per = (int64_t)kThreads * kUnits * kUnitElems;
+    const int64_t per = (int64_t)kThreads * kUnitElems;
     return (elems + per - 1) / per;
 }
 
