@@ -112,24 +112,26 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
 // How the cache kernel (32 query rows per workgroup, tree and prefix in one launch) takes a launch: waves per workgroup
 // and runs of prefix tiles (runs = 0: not at all).  Shape and flags only.
 //
-// The number of runs is the one with the shortest predicted time.  Over 45000 timings of 8500 shapes (8-512 rows, 8 bits
-// -1024, 8-400 slices, 64-24000 keys, every candidate forced) the prediction is off by 10-12 % on average with 16-bit K/V and
-// by 15-23 % with 8-bit (too long for fp16, which needs no second weight half); the run count it picks costs 3.4 % over the
-// best candidate on average, 10 % at the ninetieth percentile.  Where it is wrong: 64-127 workgroups of one row group behind
-// more than 1000 keys (one run, 20-27 % over the best on average, 67 % at worst: the bytes are priced at the whole GPU's rate,
-// which half of the CUs do not draw).  The prediction:
+// The number of runs is the one with the shortest predicted time.  The constants are those that choose best, not those that
+// predict best: fitted to the choice over 91000 timings of 14000 shapes (8-256 rows, 8-512 slices, 64-32768 keys, K and V of
+// three calls in turn), the run count they pick costs 0.6 % over the best candidate on average, 2.2 % at the ninetieth
+// percentile, 25 % at worst (shapes held out of the fit: the same; 45000 older timings with up to 1024 rows: 1.1, 4, 58 %),
+// where a prediction without `cu_rate` and the products' type, fitted to the times, cost 2.2, 8 and 66 % (84 slices of
+// 32 rows behind 12055 keys, D 64: 73 us in one run, 45 in three; 64 slices of 49 rows, 32694 keys: 173, 105).
 //   1.6 (launch) + rounds of workgroups * start_end + the larger of
 //     workgroups on the fullest CU * tiles * tile   (a CU's matrix cores, L2 and LDS)      [us]
 //     rounds * tiles per wave * wave_tile           (one wave's chain)
-//   but no less than the prefix read once at `tb` TB/s (rereading by the other row groups: a fraction `again` each),
+//       both times f16 for float16, which needs no second weight half,
+//   but no less than start_end + the prefix read once at `tb1` or, with several row groups, `tb` TB/s (rereading by the other
+//   groups: a fraction `again` each), and no faster than `cu_rate` B/ns for each CU that has a workgroup,
 //   + for more than one run `join` and the float32 parts, written and read once at `join_tb` TB/s.
 struct CacheCost {
-    float start_end8, start_end4, tile, wave_tile, join, join_tb, tb, again;
+    float start_end8, start_end4, tile, wave_tile, f16, join, join_tb, tb1, tb, again, cu_rate;
 };
-constexpr CacheCost kCost16[2] = {{2.85f, 2.2f, 0.118f, 0.7f, 2.35f, 5.6f, 6.0f, 0.36f},      // head_dim 64
-                                  {3.5f, 2.9f, 0.276f, 0.0f, 2.9f, 6.4f, 5.6f, 0.21f}};      // head_dim 128
-constexpr CacheCost kCost8[2] = {{3.2f, 2.3f, 0.106f, 0.67f, 2.06f, 3.2f, 4.0f, 0.17f},       // the same on 8-bit K/V
-                                 {3.8f, 3.4f, 0.172f, 0.82f, 2.2f, 3.6f, 4.2f, 0.16f}};
+constexpr CacheCost kCost16[2] = {{2.71f, 2.42f, 0.0481f, 1.1f, 1.06f, 2.84f, 2.83f, 9.67f, 8.05f, 0.34f, 50.2f},       // head_dim 64
+                                  {4.11f, 0.236f, 0.346f, 0.555f, 1.04f, 1.56f, 1.27f, 9.0f, 11.5f, 0.64f, 46.3f}};      // head_dim 128
+constexpr CacheCost kCost8[2] = {{2.42f, 3.46f, 0.112f, 0.602f, 1.01f, 2.39f, 16.8f, 6.09f, 4.28f, 0.08f, 33.7f},        // the same on 8-bit K/V
+                                 {2.76f, 5.56f, 0.208f, 0.628f, 1.16f, 3.14f, 15.4f, 8.89f, 6.05f, 0.412f, 66.8f}};
 // Longer trees: 16-bit K/V go to the dense prefix kernel and the tree kernel, which read the prefix once per 128 and 64
 // rows; a workgroup of the cache kernel reads it for 32 rows.
 constexpr int kCacheMaxRows = 512;
@@ -165,9 +167,10 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
     const int forced = (int)((flags >> 8) & 0xffu);
     const CacheCost& k = (kv8 ? kCost8 : kCost16)[head_dim == 128 ? 1 : 0];
     const double bytes = (double)slices * prefix * head_dim * (kv8 ? 2.0 : 4.0) * 1e-6;      // prefix K and V, MB
+    const double product = dtype == FSTA_F16 ? k.f16 : 1.0;
     double best = 0.0;
     // candidates: one run, the counts that fill the CUs once, twice, .., and those whose runs are one, two, .. tiles for
-    // each of eight waves, if they promise a tenth, the prediction's error (few slices: 46 rows, 8 slices, 1955 keys fill
+    // each of eight waves, if they promise a tenth (few slices: 46 rows, 8 slices, 1955 keys fill
     // 16 CUs in one run, 15.0 us, 9.3 in eight); a run has work for half of a workgroup's waves
     for (int i = 0; i <= 8; ++i) {
         const int64_t fill = i == 0 ? 1 : i <= 4 ? (int64_t)kGpuCus * i / wgs1 : (tiles + 8 * (i - 4) - 1) / (8 * (i - 4));
@@ -184,8 +187,11 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
         const double t_tiles = per + 3.0;                        // (a few ancestor tiles and the own rows)
         const double chain = rounds * (double)((per + 3 + waves - 1) / waves) * k.wave_tile;
         const double work = on_cu * t_tiles * k.tile;
-        double t = 1.6 + rounds * (waves == 8 ? k.start_end8 : k.start_end4) + (chain > work ? chain : work);
-        const double mem = 1.6 + k.start_end8 + bytes / k.tb * (1.0 + k.again * (double)(groups - 1));
+        double t = 1.6 + rounds * (waves == 8 ? k.start_end8 : k.start_end4) + (chain > work ? chain : work) * product;
+        const double cus = wgs < kGpuCus ? (double)wgs : (double)kGpuCus;
+        const double together = (1.0 + k.again * (double)(groups - 1)) / (groups == 1 ? k.tb1 : k.tb);
+        const double each = (double)groups / (cus * k.cu_rate * 1e-3);
+        const double mem = 1.6 + k.start_end8 + bytes * (together > each ? together : each);
         if (mem > t) t = mem;
         if (runs > 1) t += k.join + 2.0 * runs * (double)slices * nq * head_dim * 4e-6 / k.join_tb;
         if (c.runs == 0 || t < (i <= 4 ? best : 0.9 * best)) {
