@@ -246,24 +246,32 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
     const int q_row = lane / kCpr, q_slot = lane % kCpr;           // Q rows are 16-bit
     const int dma_row = lane / kKvCpr, dma_slot = lane % kKvCpr;   // K/V rows as stored
     constexpr int kQRowsPerDma = 64 / kCpr;
-    constexpr int kQDma = 16 / kQRowsPerDma;
+    // The two waves of a row group that share its tiles fetch half of its Q rows each and read all of them (one barrier
+    // more): half the Q transfers in the burst a launch starts with, and one ring slot more for the first tiles (1024 deep rows,
+    // 32 slices, D 128: 12.07 -> 11.89 us; 1500 deep rows, 80 slices: 37.4 -> 36.1; 2048 rows of window 64, 64 slices: 43.7 -> 42.7).
+    // (Q straight into registers, 64 bytes of a row per instruction: 12.9, 45.9 us for the first and the last.)
+    constexpr bool kQShared = KS == 2 && 16 / kQRowsPerDma >= 2;
+    constexpr int kQDma = 16 / kQRowsPerDma / (kQShared ? 2 : 1);
     static_assert(kQDma >= 1, "a transfer covers at most the wave's 16 rows");
+    constexpr int kQCopies = kQShared ? kQGroups : kWaves;
+    const int q_at = kQShared ? qgroup : wave;
     // (a small grid has LDS to spare: Q then gets an area of its own behind the plan, the
     // whole ring is free from the start and the fragments are read after the ancestor tiles have
     // been requested instead of in front of the first barrier)
     // (8-bit K/V: Q waits in the widened tiles, which are first written behind the first barrier)
-    T* qstage = early_leaf ? reinterpret_cast<T*>(group_s + kLeafTiles * group_words) + wave * 16 * D
+    T* qstage = early_leaf ? reinterpret_cast<T*>(group_s + kLeafTiles * group_words) + q_at * 16 * D
                 : KV8      ? ring + wave * 16 * D
-                           : ring + (size_t)stages * 2 * kTileElems - (kWaves - wave) * 16 * D;
+                           : ring + (size_t)stages * 2 * kTileElems - (kQCopies - q_at) * 16 * D;
     static_assert(!KV8 || kWaves * 16 <= 4 * kTileN, "Q must fit into the two widened tiles");
 #pragma unroll
     for (int i = 0; i < kQDma; ++i) {
-        const int r = i * kQRowsPerDma + q_row;
+        const int n = kQShared ? split * kQDma + i : i;
+        const int r = n * kQRowsPerDma + q_row;
         const int grow = min(row_base + qgroup * 16 + r, p.nq - 1);
         const uint32_t off = (uint32_t)grow * (uint32_t)(D * sizeof(T)) + (uint32_t)k_chunk<D>(r, q_slot) * 16u;
         __builtin_amdgcn_global_load_lds(
             (const void __attribute__((address_space(1)))*)(reinterpret_cast<const char*>(qb) + (size_t)off),
-            (void __attribute__((address_space(3)))*)(qstage + i * 512), 16, 0, kStreamOnce);
+            (void __attribute__((address_space(3)))*)(qstage + n * 512), 16, 0, kStreamOnce);
     }
 
     // ---- gather: HBM -> LDS, 16 bytes per lane, no registers in between --------
@@ -340,6 +348,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
     Frag qf[kSteps];
     auto read_q = [&](int tiles_issued_since) {
         wait_tiles_outstanding<kDmaPerWave>(gathers ? tiles_issued_since : 0);
+        if constexpr (kQShared) ring_barrier();      // the other wave's half has landed
         u32x4 qraw[kSteps];
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
@@ -544,7 +553,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
     }
     if (!early_leaf) {
         // (Q is parked in the last ring slots -- 8-bit K/V: in the widened tiles, the whole staging ring is free)
-        constexpr int kQSlots = KV8 ? 0 : (kWaves * 16 + 2 * kTileN - 1) / (2 * kTileN);
+        constexpr int kQSlots = KV8 ? 0 : (kQCopies * 16 + 2 * kTileN - 1) / (2 * kTileN);
         refill_to(consumed + stages - kQSlots);
         read_q(issued - consumed);
         ring_barrier();   // everybody has read its Q rows: their slots are free
