@@ -74,6 +74,19 @@ __device__ __forceinline__ void flush_rows(const unsigned char* stage, int strid
     }
 }
 
+// Instantiations that run at eight waves per SIMD: head_dim 64 in workgroups of eight waves (blocks of 128 rows, or of 64 with
+// two waves per row group) fits 64 registers, and four of these workgroups share a CU's LDS instead of three (500 deep rows in
+// blocks of 128, 256 slices: 21.8 -> 19.9 us; 3000 rows in blocks of 64, 84 slices 54.4 -> 50.5; 500 rows in blocks of 64, 160
+// slices 16.2 -> 15.3).  Others are held back by their registers (head_dim 128) or the LDS of their workgroups.
+template <int D, int M, int KS, bool RUNS, bool KV8> constexpr bool eight_waves_per_simd() {
+    return D == 64 && M / 16 * KS == 8 && !RUNS && !KV8;
+}
+// Tiles in the ring where the whole list fits: six of 8 KB for blocks of 128 rows at head_dim 64 (four leaf tiles and two of
+// ancestors: the trees of the reference's benchmark), everything requested at the start, three workgroups per CU; longer
+// lists walk a ring of kMaxStages tiles, four workgroups per CU (the benchmark's tree of 65536 nodes: 1060 us against 1100
+// in a ring of four; 500 deep rows: 24.9 us against 19.9 in a ring of four).
+template <int D, int M> constexpr int ring_stages() { return D == 64 && M == 128 ? 6 : kMaxStages; }
+
 // KS > 0: waves that share one group of 16 query rows, each taking every KS-th tile with its own
 // running softmax (merged through LDS at the end).  KS = -2: two waves share a group of rows by
 // the head dimension instead: both walk every tile and form the same weights, each accumulates
@@ -89,7 +102,7 @@ __device__ __forceinline__ void flush_rows(const unsigned char* stage, int strid
 // one step ahead of its use, and the products run on those as they do for 16-bit K/V.  Widening a
 // tile once per workgroup costs an eighth of widening the fragments in every wave.
 template <bool BF16, int D, int M, bool SPLIT, int KS, bool RUNS, bool KV8 = false>
-__global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_kernel(AttnParams p, int stages, int early_leaf, int sub_shift) {
+__global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), (eight_waves_per_simd<D, M, KS, RUNS, KV8>() ? 8 : 4)) void attn_mfma16_kernel(AttnParams p, int stages, int early_leaf, int sub_shift) {
     using MM = Mma<BF16>;
     using T = typename MM::elem;
     using T2 = typename MM::elem2;
@@ -347,7 +360,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
     // tiles requested above were issued after the Q rows.
     Frag qf[kSteps];
     auto read_q = [&](int tiles_issued_since) {
-        wait_tiles_outstanding<kDmaPerWave>(gathers ? tiles_issued_since : 0);
+        wait_tiles_outstanding<kDmaPerWave, KV8 ? kMaxStages : ring_stages<D, M>()>(gathers ? tiles_issued_since : 0);
         if constexpr (kQShared) ring_barrier();      // the other wave's half has landed
         u32x4 qraw[kSteps];
 #pragma unroll
@@ -499,14 +512,14 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
             // this step.  A staging slot is free again once its tile has been widened by everyone,
             // i.e. behind the barrier after that: the slots of tiles up to `consumed` here.
             if (widened == consumed) {   // first step: nothing widened yet
-                wait_tiles_outstanding<kDmaPerWave>(max(issued - consumed - 1, 0));
+                wait_tiles_outstanding<kDmaPerWave, KV8 ? kMaxStages : ring_stages<D, M>()>(max(issued - consumed - 1, 0));
                 ring_barrier();
                 widen(consumed);
                 widened = consumed + 1;
             }
             const bool more = consumed + 1 < total_tiles;
             if (more && issued < consumed + 2) refill_to(consumed + 2);   // (a ring of one slot)
-            if (more) wait_tiles_outstanding<kDmaPerWave>(max(issued - consumed - 2, 0));
+            if (more) wait_tiles_outstanding<kDmaPerWave, KV8 ? kMaxStages : ring_stages<D, M>()>(max(issued - consumed - 2, 0));
             ring_barrier();
             refill_to(consumed + 1 + stages);
             if (more) {
@@ -530,7 +543,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
             ring_barrier();
             refill();
         }
-        wait_tiles_outstanding<kDmaPerWave>(max(issued - consumed - n, 0));
+        wait_tiles_outstanding<kDmaPerWave, KV8 ? kMaxStages : ring_stages<D, M>()>(max(issued - consumed - n, 0));
         ring_barrier();
         refill();
     };
@@ -822,6 +835,15 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
     // per lane; columns go in passes of at most 2*D bytes per row.
     constexpr int kStageStride = D * 2 + 16;     // bytes per staged row (padded against bank conflicts)
     const int first_row = row_base + qgroup * 16;
+    // The lane's place.  Where no register is to spare it is derived again behind an opaque move instead of kept from the
+    // start-up through the whole kernel.
+    constexpr bool kDerive = eight_waves_per_simd<D, M, KS, RUNS, KV8>();
+    int out_lane = lane;
+    if constexpr (kDerive) {
+        out_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(out_lane));
+    }
+    const int out_ql = kDerive ? out_lane & 15 : +ql, out_g = kDerive ? out_lane >> 4 : +g;
     // (with key runs: a partial result in the workspace, unless this launch is the one that joins the parts)
     const bool join = RUNS && p.merge_parts > 0;
     const bool partial = RUNS && !join;
@@ -837,7 +859,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
         float lse_val = l_tot > 0.f ? m_i + log2f(l_tot) : -INFINITY;
         // the row number is derived again from an opaque copy: kept from the start-up it
         // would occupy a register pair through the whole kernel
-        int rib = row_in_block;
+        int rib = kDerive ? qgroup * 16 + out_ql : +row_in_block;
         asm volatile("" : "+v"(rib));
         const int row = row_base + rib;
         if constexpr (RUNS) {
@@ -859,7 +881,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
                 for (int pp = 1; pp <= p.merge_parts; ++pp) {
                     const float w = __builtin_amdgcn_exp2f(p.part_lse[pp * part_rows + mine] - mx_safe);
                     wsum += w;
-                    const float* src = p.part_o + (pp * part_rows + mine) * D + col0 + 4 * g;
+                    const float* src = p.part_o + (pp * part_rows + mine) * D + col0 + 4 * out_g;
 #pragma unroll
                     for (int i = 0; i < kTilesHere; ++i) {
                         const f32x4 x = *reinterpret_cast<const f32x4*>(src + 16 * i);
@@ -871,7 +893,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
                 lse_val = wsum > 0.f ? mx + log2f(wsum) : -INFINITY;
             }
         }
-        if (write_lse && row < p.nq && lse_out && g == 0) lse_out[(size_t)hz_out * p.nq + row] = lse_val;
+        if (write_lse && row < p.nq && lse_out && out_g == 0) lse_out[(size_t)hz_out * p.nq + row] = lse_val;
         const int rows_valid = p.nq - first_row;
         if (out_f32) {
             constexpr int kPass = kTilesHere < D / 32 ? kTilesHere : D / 32;   // tiles per pass
@@ -882,11 +904,11 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
                 for (int i = 0; i < kPass; ++i) {
                     const f32x4& acc = vals[h * kPass + i];
                     const f32x4 val = {acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-                    *reinterpret_cast<f32x4*>(stage + ql * kStageStride + (16 * i + 4 * g) * 4) = val;
+                    *reinterpret_cast<f32x4*>(stage + out_ql * kStageStride + (16 * i + 4 * out_g) * 4) = val;
                 }
                 __builtin_amdgcn_wave_barrier();
                 flush_rows<kPass * 64>(stage, kStageStride, reinterpret_cast<unsigned char*>(ob + h * kPass * 16),
-                                       (size_t)D * 4, lane, rows_valid);
+                                       (size_t)D * 4, out_lane, rows_valid);
                 __builtin_amdgcn_wave_barrier();
             }
         } else {
@@ -896,10 +918,10 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
                 // accumulator rows 4g .. 4g+3 of a tile are 4 consecutive head dims
                 const f32x4& acc = vals[i];
                 const u32x2 packed = {MM::pack_out(acc[0] * inv, acc[1] * inv), MM::pack_out(acc[2] * inv, acc[3] * inv)};
-                *reinterpret_cast<u32x2*>(stage + ql * kStageStride + (16 * i + 4 * g) * 2) = packed;
+                *reinterpret_cast<u32x2*>(stage + out_ql * kStageStride + (16 * i + 4 * out_g) * 2) = packed;
             }
             __builtin_amdgcn_wave_barrier();
-            flush_rows<kTilesHere * 32>(stage, kStageStride, reinterpret_cast<unsigned char*>(ob), (size_t)D * 2, lane,
+            flush_rows<kTilesHere * 32>(stage, kStageStride, reinterpret_cast<unsigned char*>(ob), (size_t)D * 2, out_lane,
                                         rows_valid);
         }
     };
@@ -918,26 +940,26 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
         __syncthreads();   // the ring is free: every tile has been consumed
         float* give = reinterpret_cast<float*>(smem) + (size_t)(qgroup * 2 + split) * kXchFloats;
         const float* take = reinterpret_cast<float*>(smem) + (size_t)(qgroup * 2 + (1 - split)) * kXchFloats;
-        give[lane] = m_i;
-        give[64 + lane] = l_i;
+        give[out_lane] = m_i;
+        give[64 + out_lane] = l_i;
         f32x4 keep[kH];
         if (split == 0) {
 #pragma unroll
             for (int i = 0; i < kH; ++i) {
                 keep[i] = o[i];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) give[(2 + 4 * i + r) * 64 + lane] = o[kH + i][r];
+                for (int r = 0; r < 4; ++r) give[(2 + 4 * i + r) * 64 + out_lane] = o[kH + i][r];
             }
         } else {
 #pragma unroll
             for (int i = 0; i < kH; ++i) {
                 keep[i] = o[kH + i];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) give[(2 + 4 * i + r) * 64 + lane] = o[i][r];
+                for (int r = 0; r < 4; ++r) give[(2 + 4 * i + r) * 64 + out_lane] = o[i][r];
             }
         }
         __syncthreads();
-        const float m_b = take[lane], l_b = take[64 + lane];
+        const float m_b = take[out_lane], l_b = take[64 + out_lane];
         const float m_new = fmaxf(m_i, m_b);
         const float m_safe = m_new == -INFINITY ? 0.f : m_new;
         const float a_own = __builtin_amdgcn_exp2f(m_i - m_safe);
@@ -947,7 +969,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), 4) void attn_mfma16_ke
 #pragma unroll
         for (int i = 0; i < kH; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) keep[i][r] = keep[i][r] * a_own + take[(2 + 4 * i + r) * 64 + lane] * a_oth;
+            for (int r = 0; r < 4; ++r) keep[i][r] = keep[i][r] * a_own + take[(2 + 4 * i + r) * 64 + out_lane] * a_oth;
         unsigned char* stage = smem + (size_t)kQGroups * 2 * kXchFloats * 4 + (size_t)wave * 16 * kStageStride;
         finish(keep, split * (D / 2), stage, split == 0);
     }
@@ -967,7 +989,7 @@ template <bool BF16, int D, int M, bool SPLIT, int KS>
 int launch_ks(const AttnParams& p, int sub_shift, hipStream_t stream) {
     // ring depth: everything in flight at once for short tile lists, else the limit
     const int tiles = M / 32 + anc_tile_capacity(p.max_anc) + (p.prefix + kTileN - 1) / kTileN;
-    int stages = tiles < 2 ? 2 : (tiles > kMaxStages ? kMaxStages : tiles);
+    int stages = tiles < 2 ? 2 : (tiles <= ring_stages<D, M>() ? tiles : kMaxStages);
     size_t lds = mfma16_lds_bytes<D, M>(p.max_anc, stages);
     while (lds > 160 * 1024 && stages > 2) lds = mfma16_lds_bytes<D, M>(p.max_anc, --stages);
     // the kernel's start-up parks Q in the last ring slots and requests up to two leaf tiles

@@ -96,14 +96,16 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // Waits until at most `tiles` tiles' worth of this wave's global->LDS transfers
-// (kPerTile instructions each, retired in order) are still outstanding.
-template <int kPerTile> __device__ __forceinline__ void wait_tiles_outstanding(int tiles) {
-    static_assert((kMaxStages - 1) * kPerTile < 64, "ring too deep for vmcnt");
+// (kPerTile instructions each, retired in order) are still outstanding; kStages: the deepest ring.
+template <int kPerTile, int kStages = kMaxStages> __device__ __forceinline__ void wait_tiles_outstanding(int tiles) {
+    static_assert(kStages <= 6 && (kStages - 1) * kPerTile < 64, "ring too deep for vmcnt");
     switch (tiles) {
         case 0: wait_vmcnt<0>(); break;
         case 1: wait_vmcnt<kPerTile>(); break;
         case 2: wait_vmcnt<2 * kPerTile>(); break;
-        default: wait_vmcnt<3 * kPerTile>(); break;
+        case 3: wait_vmcnt<3 * kPerTile>(); break;
+        case 4: if constexpr (kStages > 4) { wait_vmcnt<4 * kPerTile>(); break; }
+        default: wait_vmcnt<(kStages > 4 ? 5 : 3) * kPerTile>(); break;
     }
 }
 

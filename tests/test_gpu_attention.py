@@ -397,6 +397,18 @@ def test_two_tiles_per_step_with_peaked_weights(dtype, scale):
     run_tree(parent, 128, 1, 3, 64, dtype, 32, scale=scale, want_kernel="-2")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("ancestors", [20, 32, 64, 90])
+def test_blocks_of_128_rows_with_the_whole_list_in_the_ring(dtype, ancestors):
+    """head_dim 64, enough workgroups that no block is halved: lists of five and six tiles have a ring as long as
+    the list, longer ones walk a ring of four."""
+    n = 300                                                      # a ragged last block
+    parent = np.arange(-1, n - 1, dtype=np.int64) % ancestors     # a chain of that many nodes, all others its children
+    parent[0] = -1
+    parent[1:ancestors] = np.arange(ancestors - 1)
+    run_tree(parent, 128, 2, 24, 64, dtype, 8, native_out=True, want_kernel=", 64, 128, ")
+
+
 def test_reference_test_shape_with_and_without_prefix():
     # the reference's own test: Z=2 H=2 N_CTX=2048 D=64 fp16, tree of 2044 nodes,
     # blocks of 128, 64 ancestors, sm_scale 0.5, inputs N(0, 0.5^2), prefix 0 or 2048
