@@ -5,6 +5,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/fsta.h"
 
@@ -68,6 +69,22 @@ struct AttnParams {
     const float* k_scale;
     const float* v_scale;
 };
+
+// Sum over the lanes up to and including this one (all 64 active): four shifts within rows of 16 lanes, then the rows' totals
+// to the rows behind them.  Six register-to-register steps; by __shfl_up, whose every step is a round trip through the LDS
+// unit, such a sum took 0.3 us of the single-workgroup kernels' chains.
+__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t x) {
+    auto from = [](uint32_t v, auto ctrl, auto rows) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    };
+    x += from(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr:1, 2, 4, 8
+    x += from(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    x += from(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    x += from(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    x += from(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15 into rows 1 and 3
+    x += from(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2 and 3
+    return x;
+}
 
 // true when a non-null pointer is not a multiple of `bytes` (null pointers are judged elsewhere)
 inline bool misaligned(const void* ptr, unsigned bytes) { return reinterpret_cast<uintptr_t>(ptr) % bytes != 0; }

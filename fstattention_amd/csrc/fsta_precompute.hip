@@ -41,12 +41,7 @@ __device__ __forceinline__ void rank_ancestors(const uint32_t* bitmap, uint32_t*
     const int w_end = min(w_begin + per_lane, n_words);
     uint32_t local = 0u;
     for (int w = w_begin; w < w_end; ++w) local += __popc(bitmap[w]);
-    uint32_t incl = local;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t up = __shfl_up(incl, d, 64);
-        if (tid >= d) incl += up;
-    }
+    const uint32_t incl = wave_prefix_sum(local);
     uint32_t run = incl - local;
     for (int w = w_begin; w < w_end; ++w) { rank_base[w] = run; run += __popc(bitmap[w]); }
     if (tid == 63) misc[2] = incl;

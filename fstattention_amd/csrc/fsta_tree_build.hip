@@ -11,8 +11,8 @@
 // of a path is the path without its last rank.
 //
 //   1. scores of all candidates into LDS
-//   2. the (n-1)-th largest score by radix selection on the bit patterns (up to 8 passes of 8 bits,
-//      ending as soon as the candidates left all belong to the kept ones; non-negative doubles
+//   2. the (n-1)-th largest score by radix selection on the bit patterns (passes of 8 bits behind a first one over the
+//      leading 16, ending as soon as the candidates left all belong to the kept ones; non-negative doubles
 //      order like their bit patterns)
 //   3. "kept" flags (above the threshold, or equal to it and among the first ties), numbered by
 //      a prefix sum over the candidate index
@@ -21,6 +21,9 @@
 // level is never stored: the (n-1)-th largest score of the shorter paths bounds the threshold from
 // below, the last level is scored on the fly against that bound, and steps 2-4 run over the short
 // list of paths that reach it (same result, a tenth of the keys; 18.5 -> 13.3 us for that shape).
+// One workgroup, nothing busy: what it takes is its chain of LDS round trips and barriers.  Sums over a wave by register moves
+// instead of LDS permutes: 13.9 -> 12.5 us for that shape and 255 paths; a first pass over a window of 16 leading bits, the next
+// histogram cleared beside the sum, and one list request per four candidates: 12.5 -> 10.9.
 #include "fsta_common.h"
 
 namespace fsta {
@@ -44,8 +47,8 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
     extern __shared__ __attribute__((aligned(16))) unsigned char build_s[];
     uint64_t* key_s = reinterpret_cast<uint64_t*>(build_s);                    // [n_cand] score bits, later node ids
     double* prob_s = reinterpret_cast<double*>(key_s + n_cand);                // [depths * topk]
-    uint32_t* hist_s = reinterpret_cast<uint32_t*>(prob_s + depths * topk);    // [256] bytes; later counts per (row, wave)
-    uint32_t* misc_s = hist_s + 256;   // [0] chosen byte, [1] candidates still wanted, [2] selection finished, [3] length of the short list
+    uint32_t* hist_s = reinterpret_cast<uint32_t*>(prob_s + depths * topk);    // two histograms of [256]; later counts per (row, wave)
+    uint32_t* misc_s = hist_s + 512;   // [0] chosen byte, [1] candidates still wanted, [2] selection finished, [3] length of the short list
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -56,30 +59,37 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
         return;
     }
     for (int e = tid; e < depths * topk; e += kBuildThreads) prob_s[e] = (double)probs[e];
+    if (tid < 512) hist_s[tid] = 0u;
     __syncthreads();
 
     // select(src, count, k): the k-th largest of src[0 .. count) and how many of the keys equal to it belong to the k
     // largest, by radix selection, 8 bits per pass from the top (non-negative doubles order like their bit
     // patterns); a pass ends the search as soon as every key left is wanted.
+    // What bounds it is the chain of a pass: counts, barrier, one wave's sum over the histogram, barrier (the histogram of the
+    // next pass is cleared beside that sum).  The leading byte of a product of probabilities says next to nothing, so the first
+    // pass takes the leading 16 bits against a window of 256 values that ends at 1.0 (scores down to 2^-16 in sixteenths of a
+    // power of two), whose first and last bin take what lies outside; only a search that ends up there starts over by bytes.
     uint64_t threshold = 0ull;
     uint32_t want = 0u;
+    int buf = 0;                                  // the histogram that is clear
+    constexpr int kWindow = 0x3ff0 - 255;         // leading 16 bits of the window's first value; those of 1.0 are its last
     auto select = [&](const uint64_t* src, int count, uint32_t k) {
         const int src_rows = (count + kBuildThreads - 1) / kBuildThreads;
-        uint64_t prefix = 0ull;        // the bytes of the threshold found so far (in place, lower bytes zero)
+        uint64_t prefix = 0ull;        // the bits of the threshold found so far (in place, lower ones zero)
         uint32_t left = k;
-        if (tid < 3) misc_s[tid] = 0u;
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            if (tid < 256) hist_s[tid] = 0u;
-            __syncthreads();
-            const uint64_t high_mask = shift == 56 ? 0ull : ~0ull << (shift + 8);
+        bool window = true;
+        int shift = 48;
+        while (true) {
+            uint32_t* const hist = hist_s + buf * 256;
+            const uint64_t high_mask = window || shift == 56 ? 0ull : ~0ull << (shift + 8);
 #pragma unroll 1
             for (int r = 0; r < src_rows; ++r) {
                 const int c = tid + r * kBuildThreads;
                 const uint64_t key = c < count ? src[c] : 0ull;
                 const bool in = c < count && (key & high_mask) == prefix;
-                const uint32_t bin = (uint32_t)(key >> shift) & 255u;
-                // The leading bytes of the scores are nearly all alike: 64 atomics of a wave would queue
-                // on one or two words.  For up to two byte values one lane counts for all lanes that
+                const uint32_t bin = window ? (uint32_t)min(max((int)(key >> 48) - kWindow, 0), 255) : (uint32_t)(key >> shift) & 255u;
+                // Scores may be nearly all alike in the bits looked at: 64 atomics of a wave would queue
+                // on one or two words.  For up to two values one lane counts for all lanes that
                 // hold it; what is left after that is spread over many words and goes lane by lane.
                 uint64_t voters = __ballot(in);
 #pragma unroll
@@ -88,43 +98,54 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
                         const int leader = __ffsll((long long)voters) - 1;
                         const uint32_t first = __builtin_amdgcn_readlane(bin, leader);
                         const uint64_t same = __ballot(in && bin == first);
-                        if (lane == leader) atomicAdd(&hist_s[first], (uint32_t)__popcll(same));
+                        if (lane == leader) atomicAdd(&hist[first], (uint32_t)__popcll(same));
                         voters &= ~same;
                     }
                 }
-                if ((voters >> lane) & 1ull) atomicAdd(&hist_s[bin], 1u);
+                if ((voters >> lane) & 1ull) atomicAdd(&hist[bin], 1u);
             }
             __syncthreads();
+            buf ^= 1;
             if (tid < 64) {
                 // lane l owns bins 255 - 4l .. 252 - 4l; counts accumulate from the largest byte down
                 uint32_t mine[4], local = 0u;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) { mine[b] = hist_s[255 - 4 * tid - b]; local += mine[b]; }
-                uint32_t incl = local;
-#pragma unroll
-                for (int dlt = 1; dlt < 64; dlt <<= 1) {
-                    const uint32_t up = __shfl_up(incl, dlt, 64);
-                    if (tid >= dlt) incl += up;
-                }
+                for (int b = 0; b < 4; ++b) { mine[b] = hist[255 - 4 * tid - b]; local += mine[b]; }
+                const uint32_t incl = wave_prefix_sum(local);
                 uint32_t before = incl - local;       // candidates in larger bins
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     if (before < left && left <= before + mine[b]) {
                         misc_s[0] = (uint32_t)(255 - 4 * tid - b);
                         misc_s[1] = left - before;
-                        // every candidate of this byte value is wanted: the lower bytes need no look
-                        if (left - before == mine[b]) misc_s[2] = 1u;
+                        // every candidate of this byte value is wanted: the lower bits need no look
+                        misc_s[2] = left - before == mine[b] ? 1u : 0u;
                     }
                     before += mine[b];
                 }
+            } else if (tid >= 256 && tid < 512) {
+                hist_s[buf * 256 + tid - 256] = 0u;
             }
             __syncthreads();
-            prefix |= (uint64_t)misc_s[0] << shift;
-            left = misc_s[1];
-            // (uniform: everyone reads the flag between the same two barriers)
-            if (misc_s[2] != 0u) break;   // threshold = the prefix with zero lower bytes, all `left` candidates from it up
+            // (uniform: everyone reads the words between the same two barriers)
+            const uint32_t digit = misc_s[0];
+            const bool done = misc_s[2] != 0u;   // threshold = the prefix with zero lower bits, all `left` candidates from it up
+            if (window) {
+                window = false;
+                if (done || (digit > 0u && digit < 255u)) {
+                    prefix = digit > 0u ? (uint64_t)(kWindow + (int)digit) << 48 : 0ull;
+                    left = misc_s[1];
+                    shift = 40;
+                } else {
+                    shift = 56;
+                }
+            } else {
+                prefix |= (uint64_t)digit << shift;
+                left = misc_s[1];
+                shift -= 8;
+            }
+            if (done || shift < 0) break;
         }
-        __syncthreads();   // (the next search clears the words read above)
         threshold = prefix;
         want = left;
     };
@@ -173,33 +194,60 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
             if (tid == 0) misc_s[3] = 0u;
             __syncthreads();
             const uint64_t lanes_below = (1ull << lane) - 1ull;
-            auto list = [&](bool take, uint64_t key, int index) {      // (called by whole waves)
-                const uint64_t takers = __ballot(take);
-                if (takers == 0ull) return;
+            // (four candidates per thread at a time: one request for places in the list per wave, whose round trip is the chain)
+            constexpr int kListed = 4;
+            auto list = [&](const bool (&take)[kListed], const uint64_t (&key)[kListed], const int (&index)[kListed]) {   // (by whole waves)
+                uint64_t takers[kListed];
+                uint32_t n = 0u;
+#pragma unroll
+                for (int i = 0; i < kListed; ++i) {
+                    takers[i] = __ballot(take[i]);
+                    n += (uint32_t)__popcll(takers[i]);
+                }
+                if (n == 0u) return;
                 uint32_t base = 0u;
-                if (lane == 0) base = atomicAdd(&misc_s[3], (uint32_t)__popcll(takers));
+                if (lane == 0) base = atomicAdd(&misc_s[3], n);
                 base = __builtin_amdgcn_readfirstlane(base);
-                const uint32_t pos = base + (uint32_t)__popcll(takers & lanes_below);
-                if (take && pos < (uint32_t)kBuildShort) {
-                    skey_s[pos] = key;
-                    sidx_s[pos] = (uint32_t)index;
+#pragma unroll
+                for (int i = 0; i < kListed; ++i) {
+                    const uint32_t pos = base + (uint32_t)__popcll(takers[i] & lanes_below);
+                    if (take[i] && pos < (uint32_t)kBuildShort) {
+                        skey_s[pos] = key[i];
+                        sidx_s[pos] = (uint32_t)index[i];
+                    }
+                    base += (uint32_t)__popcll(takers[i]);
                 }
             };
 #pragma unroll 1
-            for (int c0 = 0; c0 < n_head; c0 += kBuildThreads) {
-                const int c = c0 + tid;
-                const uint64_t key = c < n_head ? key_s[c] : 0ull;
-                list(c < n_head && key >= bound, key, c);
+            for (int c0 = 0; c0 < n_head; c0 += kListed * kBuildThreads) {
+                bool take[kListed];
+                uint64_t key[kListed];
+                int index[kListed];
+#pragma unroll
+                for (int i = 0; i < kListed; ++i) {
+                    index[i] = c0 + i * kBuildThreads + tid;
+                    key[i] = key_s[min(index[i], n_head - 1)];
+                    take[i] = index[i] < n_head && key[i] >= bound;
+                }
+                list(take, key, index);
             }
 #pragma unroll 1
-            for (int v0 = 0; v0 < last; v0 += kBuildThreads) {
-                const int v = v0 + tid;
-                const bool valid = v < last;
-                const uint32_t q = __umulhi((uint32_t)(valid ? v : 0), magic);
-                const uint32_t r = (uint32_t)(valid ? v : 0) - q * (uint32_t)topk;
-                const double head = __longlong_as_double((long long)key_s[prev_start + q]);
-                const uint64_t key = (uint64_t)__double_as_longlong(head * prob_s[lvl * topk + r]);
-                list(valid && key >= bound, key, n_head + v);
+            for (int v0 = 0; v0 < last; v0 += kListed * kBuildThreads) {
+                bool take[kListed];
+                uint64_t key[kListed];
+                int index[kListed];
+#pragma unroll
+                for (int i = 0; i < kListed; ++i) {
+                    const int v = v0 + i * kBuildThreads + tid;
+                    const uint32_t at = (uint32_t)min(v, last - 1);
+                    const uint32_t q = __umulhi(at, magic);
+                    const uint32_t r = at - q * (uint32_t)topk;
+                    const double head = __longlong_as_double((long long)key_s[prev_start + q]);
+                    key[i] = (uint64_t)__double_as_longlong(head * prob_s[lvl * topk + r]);
+                    take[i] = v < last && key[i] >= bound;
+                    index[i] = n_head + v;
+                }
+                list(take, key, index);
             }
             __syncthreads();
             const int n_short = (int)misc_s[3];
@@ -219,12 +267,7 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
                         uint32_t mine[8], local = 0u;
 #pragma unroll
                         for (int i = 0; i < 8; ++i) { mine[i] = (uint32_t)__popc(bits[8 * tid + i]); local += mine[i]; }
-                        uint32_t incl = local;
-#pragma unroll
-                        for (int dlt = 1; dlt < 64; dlt <<= 1) {
-                            const uint32_t up = __shfl_up(incl, dlt, 64);
-                            if (tid >= dlt) incl += up;
-                        }
+                        const uint32_t incl = wave_prefix_sum(local);
                         uint32_t before = incl - local;
 #pragma unroll
                         for (int i = 0; i < 8; ++i) { below_s[8 * tid + i] = before; before += mine[i]; }
@@ -303,12 +346,7 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
         uint32_t mine[4], local = 0u;
 #pragma unroll
         for (int b = 0; b < 4; ++b) { mine[b] = count_s[4 * tid + b]; local += mine[b]; }
-        uint32_t incl = local;        // n_cand <= 16384: no carry between the halves
-#pragma unroll
-        for (int dlt = 1; dlt < 64; dlt <<= 1) {
-            const uint32_t up = __shfl_up(incl, dlt, 64);
-            if (tid >= dlt) incl += up;
-        }
+        const uint32_t incl = wave_prefix_sum(local);        // n_cand <= 16384: no carry between the halves
         uint32_t before = incl - local;
 #pragma unroll
         for (int b = 0; b < 4; ++b) { count_s[4 * tid + b] = before; before += mine[b]; }
@@ -427,12 +465,7 @@ __device__ __forceinline__ void big_decide(const BigLayout& w, int pass, int kee
             uint32_t mine[4], local = 0u;
 #pragma unroll
             for (int b = 0; b < 4; ++b) { mine[b] = w.hist[q * 256 + 255 - 4 * tid - b]; local += mine[b]; }
-            uint32_t incl = local;
-#pragma unroll
-            for (int dlt = 1; dlt < 64; dlt <<= 1) {
-                const uint32_t up = __shfl_up(incl, dlt, 64);
-                if (tid >= dlt) incl += up;
-            }
+            const uint32_t incl = wave_prefix_sum(local);
             uint32_t before = incl - local;
             uint32_t byte = 0u, next_want = 0u, fin = 0u, hit = 0u;
 #pragma unroll
@@ -639,7 +672,7 @@ extern "C" int fsta_medusa_tree(const void* probs, int32_t probs_dtype, int32_t 
         return fail(FSTA_EINVAL, "fsta_medusa_tree: n_nodes=%d but only %lld candidate paths (+ the root)", n_nodes,
                     (long long)n_cand);
     if (!probs || !parent || !status) return fail(FSTA_EINVAL, "fsta_medusa_tree: null pointer");
-    const size_t lds = (size_t)n_cand * 8 + (size_t)depths * topk * 8 + (256 + 4) * 4;
+    const size_t lds = (size_t)n_cand * 8 + (size_t)depths * topk * 8 + (512 + 4) * 4;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (probs_dtype == FSTA_F32) {
         if (lds > 64 * 1024) {

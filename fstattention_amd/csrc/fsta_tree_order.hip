@@ -106,12 +106,7 @@ __global__ __launch_bounds__(kScanThreads) void order_scan_kernel(int32_t n, con
     const int lo = min(tid * per, n + 1), hi = min(lo + per, n + 1);
     int32_t local = 0;
     for (int x = lo; x < hi; ++x) local += kids[x];
-    int32_t incl = local;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int32_t up = __shfl_up(incl, d, 64);
-        if ((tid & 63) >= d) incl += up;
-    }
+    const int32_t incl = (int32_t)wave_prefix_sum((uint32_t)local);
     if ((tid & 63) == 63) wave_sum[tid >> 6] = incl;
     __syncthreads();
     int32_t base = 0;

@@ -295,6 +295,17 @@ def test_medusa_tree_built_on_the_gpu_matches_the_host_builder():
 
 
 
+@pytest.mark.parametrize("factor", [2.0 ** 9, 1.0, 2.0 ** -6, 2.0 ** -15, 2.0 ** -40, 2.0 ** -1060])
+@pytest.mark.parametrize("depths,topk", [(4, 10), (3, 10), (2, 100)])
+def test_medusa_tree_scores_in_and_outside_of_the_first_window(depths, topk, factor):
+    """The search for the n-th best score looks at scores from 2**-16 to 1 first; all of them, some or none lie there."""
+    probs = trees.medusa_probs(depths, topk, 0.3, 41)
+    probs[0] *= factor
+    for n in (2, 16, 90, 101):
+        np.testing.assert_array_equal(medusa_parents_gpu(torch.from_numpy(probs).cuda(), n).cpu().numpy(),
+                                      _best_paths_host(probs, n), err_msg=f"n={n}")
+
+
 def _best_paths_host(probs, n):
     """``trees.medusa_parents_from_probs`` for candidate sets too large to enumerate in Python tuples:
     the same scores (float64 products from the first rank on), the same order (score descending,
