@@ -82,9 +82,9 @@ template <int D, int M, int KS, bool RUNS, bool KV8> constexpr bool eight_waves_
     return D == 64 && M / 16 * KS == 8 && !RUNS && !KV8;
 }
 // Tiles in the ring where the whole list fits: six of 8 KB for blocks of 128 rows at head_dim 64 (four leaf tiles and two of
-// ancestors: the trees of the reference's benchmark), everything requested at the start, three workgroups per CU; longer
-// lists walk a ring of kMaxStages tiles, four workgroups per CU (the benchmark's tree of 65536 nodes: 1060 us against 1100
-// in a ring of four; 500 deep rows: 24.9 us against 19.9 in a ring of four).
+// ancestors: the trees of the reference's benchmark), everything requested at the start, three workgroups per CU (its tree of
+// 65536 nodes, us: 1060, in a ring of four 1100); longer lists walk a ring of kMaxStages tiles, four workgroups per CU (500 deep
+// rows: 19.9, in a ring of six 24.9).
 template <int D, int M> constexpr int ring_stages() { return D == 64 && M == 128 ? 6 : kMaxStages; }
 
 // KS > 0: waves that share one group of 16 query rows, each taking every KS-th tile with its own

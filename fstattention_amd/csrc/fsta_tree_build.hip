@@ -23,7 +23,8 @@
 // list of paths that reach it (same result, a tenth of the keys; 18.5 -> 13.3 us for that shape).
 // One workgroup, nothing busy: what it takes is its chain of LDS round trips and barriers.  Sums over a wave by register moves
 // instead of LDS permutes: 13.9 -> 12.5 us for that shape and 255 paths; a first pass over a window of 16 leading bits, the next
-// histogram cleared beside the sum, and one list request per four candidates: 12.5 -> 10.9.
+// histogram cleared beside the sum, and one list request per four candidates: 12.5 -> 10.9; no numbering of ties where the
+// search ended with every key of its last bin wanted: 10.9 -> 10.6.
 #include "fsta_common.h"
 
 namespace fsta {
@@ -71,6 +72,7 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
     // power of two), whose first and last bin take what lies outside; only a search that ends up there starts over by bytes.
     uint64_t threshold = 0ull;
     uint32_t want = 0u;
+    bool no_ties = false;                         // every key from the threshold up is wanted
     int buf = 0;                                  // the histogram that is clear
     constexpr int kWindow = 0x3ff0 - 255;         // leading 16 bits of the window's first value; those of 1.0 are its last
     auto select = [&](const uint64_t* src, int count, uint32_t k) {
@@ -144,6 +146,7 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
                 left = misc_s[1];
                 shift -= 8;
             }
+            no_ties = done;
             if (done || shift < 0) break;
         }
         threshold = prefix;
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
                 for (int e = tid; e < n_short; e += kBuildThreads) {
                     const uint64_t key = skey_s[e];
                     const uint32_t c = sidx_s[e];
-                    if (key > threshold) atomicOr(&kept_s[c >> 5], 1u << (c & 31));
+                    if (key > threshold || (no_ties && key == threshold)) atomicOr(&kept_s[c >> 5], 1u << (c & 31));
                     else if (key == threshold) atomicOr(&tie_s[c >> 5], 1u << (c & 31));
                 }
                 __syncthreads();
@@ -278,12 +281,14 @@ __global__ __launch_bounds__(kBuildThreads) void medusa_tree_kernel(const T* __r
                     return below_s[c >> 5] + (uint32_t)__popc(bits[c >> 5] & ((1u << (c & 31)) - 1u));
                 };
                 // the first `want` ties in index order are kept as well
-                count_below(tie_s);
-                for (int e = tid; e < n_short; e += kBuildThreads) {
-                    const uint32_t c = sidx_s[e];
-                    if (skey_s[e] == threshold && rank_in(tie_s, c) < want) atomicOr(&kept_s[c >> 5], 1u << (c & 31));
+                if (!no_ties) {       // (uniform)
+                    count_below(tie_s);
+                    for (int e = tid; e < n_short; e += kBuildThreads) {
+                        const uint32_t c = sidx_s[e];
+                        if (skey_s[e] == threshold && rank_in(tie_s, c) < want) atomicOr(&kept_s[c >> 5], 1u << (c & 31));
+                    }
+                    __syncthreads();
                 }
-                __syncthreads();
                 count_below(kept_s);
                 // ids = 1 + kept paths below in index order; the parent of a path is the path without its last rank
                 if (tid == 0) parent[0] = -1;
