@@ -72,7 +72,7 @@ struct AttnParams {
 
 // Sum over the lanes up to and including this one (all 64 active): four shifts within rows of 16 lanes, then the rows' totals
 // to the rows behind them.  Six register-to-register steps; by __shfl_up, whose every step is a round trip through the LDS
-// unit, such a sum took 0.3 us of the single-workgroup kernels' chains.
+// unit, such a sum took 0.2 us more of the single-workgroup kernels' chains.
 __device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t x) {
     auto from = [](uint32_t v, auto ctrl, auto rows) {
         return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);

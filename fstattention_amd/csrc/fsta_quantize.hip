@@ -23,6 +23,7 @@ constexpr float kFp8Max = 448.f;
 constexpr int kThreads = 512;            // two launches: threads per piece, a unit of 16 elements each
 constexpr int kOneThreads = 1024;        // one launch: threads per slice
 constexpr int kUnitElems = 16;
+constexpr double kGridThreads = 4294967296.0;      // a grid ends before 2^32 threads
 
 template <typename T> struct Unit {      // 16 elements as they lie in memory
     static constexpr int kWords = kUnitElems * (int)sizeof(T) / 16;
@@ -237,10 +238,21 @@ template <typename T> int launch_quantize(QuantArgs a, int tensors, int dtype, h
         else
             hipLaunchKernelGGL((quantize_slice_kernel<T, kMost>), grid, block, 0, stream, a);
     } else {
-        const dim3 grid((unsigned)(tensors * a.slices * (int64_t)a.pieces)), block(kThreads);
-        hipLaunchKernelGGL((quantize_pieces_kernel<T, false>), grid, block, 0, stream, a);
-        FSTA_HIP_OK(hipGetLastError());
-        hipLaunchKernelGGL((quantize_pieces_kernel<T, true>), grid, block, 0, stream, a);
+        // (both tensors in a grid, or one after the other where that would be more threads than a grid has)
+        const int64_t each = (int64_t)a.slices * a.pieces;
+        const int in_grid = (double)tensors * (double)each * kThreads < kGridThreads ? tensors : 1;
+        for (int t = 0; t < tensors; t += in_grid) {
+            if (t > 0) {
+                a.src[0] = a.src[1];
+                a.dst[0] = a.dst[1];
+                a.scale[0] = a.scale[1];
+            }
+            const dim3 grid((unsigned)(in_grid * each)), block(kThreads);
+            hipLaunchKernelGGL((quantize_pieces_kernel<T, false>), grid, block, 0, stream, a);
+            FSTA_HIP_OK(hipGetLastError());
+            hipLaunchKernelGGL((quantize_pieces_kernel<T, true>), grid, block, 0, stream, a);
+            FSTA_HIP_OK(hipGetLastError());
+        }
     }
     FSTA_HIP_OK(hipGetLastError());
     return FSTA_OK;
@@ -270,9 +282,8 @@ extern "C" int fsta_quantize_fp8(const void* a, const void* b, void* a8, void* b
     if (misaligned(a_scale, 4) || misaligned(b_scale, 4) || misaligned(workspace, 4))
         return fail(FSTA_EINVAL, "fsta_quantize_fp8: scales and workspace must be 4-byte aligned");
     const int64_t pieces = pieces_of(elements);
-    // (a grid ends at 2^32 threads)
     if (slices > 0x7fffffff || pieces > 0x7fffffff ||
-        2.0 * (double)slices * (one_launch(elements, dtype) ? (double)kOneThreads : (double)pieces * kThreads) >= 4294967296.0)
+        (double)slices * (one_launch(elements, dtype) ? 2.0 * kOneThreads : (double)pieces * kThreads) >= kGridThreads)
         return fail(FSTA_EUNSUPPORTED, "fsta_quantize_fp8: %lld slices of %lld elements", (long long)slices, (long long)elements);
     const size_t need = fsta_quantize_workspace_bytes(slices, elements, dtype);
     if (need && (!workspace || workspace_bytes < need))

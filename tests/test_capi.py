@@ -176,6 +176,16 @@ def test_quantize_refuses_grids_that_do_not_exist():
     assert call(1, 1 << 17, 4) == _lib.EINVAL and b"workspace" in lib.fsta_last_error()
 
 
+def test_quantize_takes_tensors_up_to_a_grid_each():
+    """Up to 2^32 threads of 16 elements per tensor (the two go one after the other where both in a grid are too many)."""
+    lib = _lib.load()
+    call = lambda slices, elements: lib.fsta_quantize_fp8(16, 16, 16, 16, 16, 16, slices, elements, _lib.BF16, 16, 4, None)
+    for slices, elements in (((1 << 18) + 1, 1 << 17), ((1 << 19) - 1, 1 << 17), (1, (1 << 36) - (1 << 13))):
+        assert call(slices, elements) == _lib.EINVAL and b"workspace" in lib.fsta_last_error()
+    for slices, elements in ((1 << 19, 1 << 17), (1, 1 << 36)):
+        assert call(slices, elements) == _lib.EUNSUPPORTED
+
+
 def test_workspace_planning_is_host_arithmetic():
     """How a shared prefix is cut into runs of keys depends on the shape and flags only."""
     lib = _lib.load()
