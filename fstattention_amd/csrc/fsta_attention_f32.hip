@@ -6,7 +6,9 @@
 // (batch, head) slice, and its waves take 16 keys each -- ancestors, then the shared prefix -- so that all K/V rows of a
 // block are on their way after the first round trip, wherever they are used.  Nothing is staged in LDS; the waves' running
 // softmaxes are joined there at the end.  (64 rows of 16 ancestors, 8 heads, head_dim 64: 7.4 us with the scalar kernel's
-// workgroup of 64 rows that walks its keys in tiles of 32.)
+// workgroup of 64 rows that walks its keys in tiles of 32.)  Sums, maxima and the row that empty slots repeat go from lane to
+// lane by register moves: a permute is a round trip through the LDS unit in the chain (in a graph 3.81 -> 3.69 us for that shape,
+// 256 rows, 12 heads 5.14 -> 5.00; the rows' V keys by sixteen such moves instead of four permutes: no change).
 //
 // 16x16x4 products: A holds row i = lane % 16, k = g = lane / 16; B column i, k = g; C register r row 4g + r of column i.
 //   S^T = K.Q^T   row: key, column: query.  The product over dims is split as 16 j + 4 g + e: product (j, e) takes dim
@@ -14,7 +16,7 @@
 //   O^T += V^T.P  register r of S^T is the B operand for keys 4g + r as it stands; V is loaded as 16 bytes per lane, dims
 //                 64 b + 4 i + e of key 4g + r, which makes O^T tile (b, e) rows i: a lane ends with dims 64 b + 16 g .. +15.
 // A row's own key (reference fstattention.py:86-91) needs no product: its wave starts from score, weight 1 and V row.
-#include "fsta_common.h"
+#include "fsta_mfma_common.h"
 
 namespace fsta {
 namespace {
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
             const int first = exists ? __builtin_ctz(exists) : 0;
             // an empty slot repeats the tile's first row: no row outside the list is read
             key = there ? (int)id : -1;
-            const int repeat = __shfl(key, first);
+            const int repeat = __builtin_amdgcn_readlane(key, first);
             if (key < 0) key = max(repeat, 0);
             ok = ((((w >> (kKeys * (t & 1))) & exists) >> (4 * g)) & 0xfu) | (~exists << 16);
         } else {
@@ -129,8 +131,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
 #pragma unroll
             for (int e = 0; e < 4; ++e) dot[e] = __builtin_fmaf(q[s][e], ko[s][e], dot[e]);
         float score = (dot[0] + dot[1]) + (dot[2] + dot[3]);
-        score += __shfl_xor(score, 16);
-        score += __shfl_xor(score, 32);
+        score = mfma::sum_quarters(score);
         if (there) {
             m_i = score * p.scale_log2e;
             l_i = g == 0 ? 1.f : 0.f;
@@ -161,8 +162,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
             sv[r] = (mine >> r) & 1u ? (s2[0][r] + s2[1][r]) * p.scale_log2e : -INFINITY;
             mx = fmaxf(mx, sv[r]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = mfma::max_quarters(mx);
         const float m_new = fmaxf(m_i, mx);
         const float base = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_i - base);       // exp2(-inf) = 0
@@ -198,8 +198,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void attn_f32_kernel(Attn
     // ---- join the waves that had keys
     const int busy = min(total, NW);
     if (wave < busy || own_wave) {
-        l_i += __shfl_xor(l_i, 16);
-        l_i += __shfl_xor(l_i, 32);
+        l_i = mfma::sum_quarters(l_i);
         if (g == 0) {
             m_s[wave][i] = m_i;
             l_s[wave][i] = l_i;
