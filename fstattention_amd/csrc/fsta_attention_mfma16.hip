@@ -87,6 +87,13 @@ template <int D, int M, int KS, bool RUNS, bool KV8> constexpr bool eight_waves_
 // rows: 19.9, in a ring of six 24.9).
 template <int D, int M> constexpr int ring_stages() { return D == 64 && M == 128 ? 6 : kMaxStages; }
 
+// Copies of a row group's 16 Q rows that the start-up parks in LDS: one where the two waves that share the group's tiles fetch
+// half of the rows each (a transfer of 1 KiB moves 512 / D rows: two or more per group from head_dim 64 on), else one per wave.
+// The kernel lays Q out by this, the launcher counts ring slots and LDS by it.
+template <int D, int KS> constexpr bool q_shared() { return KS == 2 && D >= 64; }
+template <int D, int M, int KS> constexpr int q_copies() { return M / 16 * (q_shared<D, KS>() ? 1 : KS < 0 ? -KS : KS); }
+template <int D, int M, int KS> constexpr int q_slots() { return (q_copies<D, M, KS>() * 16 + 2 * kTileN - 1) / (2 * kTileN); }
+
 // KS > 0: waves that share one group of 16 query rows, each taking every KS-th tile with its own
 // running softmax (merged through LDS at the end).  KS = -2: two waves share a group of rows by
 // the head dimension instead: both walk every tile and form the same weights, each accumulates
@@ -233,9 +240,9 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), (eight_waves_per_simd<
     // Record of block j: common part, then one group per 32 rows; this workgroup takes the
     // common part and its own M/32 groups, which land next to each other in LDS.
     // In a small launch (`early_leaf`) every wave copies the whole piece for itself (it is a few
-    // hundred bytes, all waves write the same values to the same place): a wave then depends on
-    // no other wave until the first tile is consumed.  Otherwise the waves share the copy and
-    // meet at a barrier.
+    // hundred bytes, all waves write the same values to the same place): a wave then waits for
+    // no other wave before its ancestor requests are out (nor, unless two waves share Q rows, before
+    // the first tile is consumed).  Otherwise the waves share the copy and meet at a barrier.
     {
         const int block_groups = block_rows / kTileN;
         const char* rec = reinterpret_cast<const char*>(p.plan) +
@@ -263,10 +270,10 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), (eight_waves_per_simd<
     // more): half the Q transfers in the burst a launch starts with, and one ring slot more for the first tiles (1024 deep rows,
     // 32 slices, D 128: 12.07 -> 11.89 us; 1500 deep rows, 80 slices: 37.4 -> 36.1; 2048 rows of window 64, 64 slices: 43.7 -> 42.7).
     // (Q straight into registers, 64 bytes of a row per instruction: 12.9, 45.9 us for the first and the last.)
-    constexpr bool kQShared = KS == 2 && 16 / kQRowsPerDma >= 2;
+    constexpr bool kQShared = q_shared<D, KS>();
     constexpr int kQDma = 16 / kQRowsPerDma / (kQShared ? 2 : 1);
     static_assert(kQDma >= 1, "a transfer covers at most the wave's 16 rows");
-    constexpr int kQCopies = kQShared ? kQGroups : kWaves;
+    constexpr int kQCopies = q_copies<D, M, KS>();
     const int q_at = kQShared ? qgroup : wave;
     // (a small grid has LDS to spare: Q then gets an area of its own behind the plan, the
     // whole ring is free from the start and the fragments are read after the ancestor tiles have
@@ -566,7 +573,7 @@ __global__ __launch_bounds__(M * 4 * (KS < 0 ? -KS : KS), (eight_waves_per_simd<
     }
     if (!early_leaf) {
         // (Q is parked in the last ring slots -- 8-bit K/V: in the widened tiles, the whole staging ring is free)
-        constexpr int kQSlots = KV8 ? 0 : (kQCopies * 16 + 2 * kTileN - 1) / (2 * kTileN);
+        constexpr int kQSlots = KV8 ? 0 : q_slots<D, M, KS>();
         refill_to(consumed + stages - kQSlots);
         read_q(issued - consumed);
         ring_barrier();   // everybody has read its Q rows: their slots are free
@@ -995,8 +1002,8 @@ int launch_ks(const AttnParams& p, int sub_shift, hipStream_t stream) {
     // the kernel's start-up parks Q in the last ring slots and requests up to two leaf tiles
     // into the first ones; ancestor lists too long to leave that much LDS go to the other kernel
     constexpr int kShares = KS < 0 ? -KS : KS;
-    constexpr int kWaves = M / 16 * kShares, kQSlots = (kWaves * 16 + 2 * kTileN - 1) / (2 * kTileN);
-    if (stages < kQSlots + (M / 32 < 2 ? M / 32 : 2)) {
+    constexpr int kWaves = M / 16 * kShares;
+    if (stages < q_slots<D, M, KS>() + (M / 32 < 2 ? M / 32 : 2)) {
         if (p.part_o) return FSTA_EUNSUPPORTED;   // the caller falls back to a launch without key splits
         return launch_attention_mfma(p, BF16 ? FSTA_BF16 : FSTA_F16, D, BF16 && !SPLIT, stream);
     }
@@ -1017,7 +1024,7 @@ int launch_ks(const AttnParams& p, int sub_shift, hipStream_t stream) {
                                     : dim3((unsigned)(kXcds * p.key_splits), (unsigned)(p.nb << sub_shift), (unsigned)slices_per_xcd);
     const int shift_arg = sub_shift | (linear_grid ? 0x100 : 0) | (late_first ? 0x200 : 0);
     // a launch whose workgroups all run at once: leaf tiles requested early, Q in an area of its own
-    constexpr size_t kQBytes = (size_t)kWaves * 16 * D * 2;
+    constexpr size_t kQBytes = (size_t)q_copies<D, M, KS>() * 16 * D * 2;
     const int early = grid <= kCus && !p.part_o && lds + kQBytes <= 160 * 1024 ? 1 : 0;
     if (early) lds += kQBytes;
     if (p.dry_run) return p.part_o && KS < 0 ? FSTA_EUNSUPPORTED : FSTA_OK;

@@ -20,7 +20,7 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kTileN = 32;     // keys per tile
 constexpr int kCus = 256;      // compute units of an MI355X
 constexpr int kXcds = 8;       // L2 domains of an MI355X; workgroup i runs on XCD i % 8
-constexpr int kMaxStages = 4;  // ring depth limit (LDS per workgroup = stages * 4 * 32 * D bytes)
+constexpr int kMaxStages = 4;  // ring depth (LDS per workgroup = stages * 4 * 32 * D bytes) unless a kernel names a longer one
 constexpr float kRescaleSlack = 8.f;  // log2 of the largest weight kept without raising the maximum
 
 template <bool BF16> struct Mma;

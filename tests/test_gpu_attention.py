@@ -453,6 +453,37 @@ def test_launches_of_one_to_two_workgroups_per_cu(n, block_m, heads, dtype):
     assert_close(o, want, dtype, f"n={n} m={block_m} heads={heads}")
 
 
+def run_ragged(parent, block_m, h, d, dtype, seed, want_kernel, max_anc=None):
+    """As many query rows as the tree has nodes, the last block cut off: float32 output, log-sum-exp and the output in the type
+    of q, every row against the dense oracle."""
+    from fstattention_amd import _lib
+    n = len(parent)
+    assert n % block_m != 0
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, block_m, max_anc)
+    q, k, v = rand_qkv(1, h, n, n, d, dtype, seed)
+    scale = 1.0 / math.sqrt(d)
+    want, want_lse = dense_oracle(q, k, v, parent, scale)
+    args = (q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), scale)
+    o, lse = fst_attention(*args, BLOCK_M=block_m, MAX_ANCESTORS=max_anc, out_dtype=torch.float32, return_lse=True)
+    assert want_kernel in _lib.load().fsta_last_attention_kernel().decode()
+    assert_close(o, want, dtype, f"n={n} m={block_m} d={d} {dtype}")
+    torch.testing.assert_close(lse.cpu().double().view(1, h, n), want_lse, atol=2e-3, rtol=2e-3)
+    o_native = fst_attention(*args, BLOCK_M=block_m, MAX_ANCESTORS=max_anc)
+    assert o_native.dtype == dtype
+    torch.testing.assert_close(o_native.float(), o.to(dtype).float(), atol=0, rtol=2 ** -7 if dtype == torch.bfloat16 else 2 ** -10)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,slots", [(128, 8161), (128, 9504), (64, 10881), (64, 11552)])
+@pytest.mark.parametrize("heads", [32, 56])
+def test_ancestor_budgets_that_leave_a_ring_of_three_tiles(d, slots, heads, dtype):
+    """Blocks of 64 rows whose two waves per row group fetch the group's Q rows together park them in one ring slot: two
+    more are enough to start with, so these budgets (the first and the last that leave LDS for three) belong to the default
+    kernel as well."""
+    parent = trees.random_recursive_parents(300, 41, window=40)
+    run_ragged(parent, 64, heads, d, dtype, 9, "attn_mfma16_kernel", max_anc=slots)
+
+
 def test_ragged_query_count():
     # nq not a multiple of block_m: rows past nq are neither read nor written
     parent = trees.random_recursive_parents(100, 3)
@@ -1096,16 +1127,17 @@ def test_cache_kernel_keeps_a_rows_own_value_to_itself(storage, nodes, d, prefix
     torch.testing.assert_close(o.cpu().double(), want, atol=2e-3, rtol=2e-3, equal_nan=True)
 
 
-@pytest.mark.parametrize("slots,kernel", [(2720, "attn_cache_kernel"), (3200, "attn_mfma16_kernel")])
-def test_lists_too_long_for_the_cache_kernel_keep_their_key_runs(slots, kernel):
+@pytest.mark.parametrize("slots,block_m,kernel", [(2720, 32, "attn_cache_kernel"), (3200, 32, "attn_mfma16_kernel"),
+                                                  (8161, 64, "attn_mfma16_kernel")])      # (a ring of three tiles)
+def test_lists_too_long_for_the_cache_kernel_keep_their_key_runs(slots, block_m, kernel):
     """Lists on both sides of what the LDS of the kernel for tree and prefix holds, in front of a prefix: the same result."""
     parent = trees.random_recursive_parents(64, 8, window=16)
-    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32, max_anc=slots)
+    a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, block_m, max_anc=slots)
     q, k, v = rand_qkv(1, 24, 64, 64 + 1500, 128, torch.bfloat16, 51)
     want, _ = dense_oracle(q, k, v, parent, 0.1, prefix=1500)
     a_idx, l_idx = shift_for_prefix(a_idx, l_idx, 1500)
     from fstattention_amd import _lib
-    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), 0.1, BLOCK_M=32,
+    o = fst_attention(q.cuda(), k.cuda(), v.cuda(), a_idx.cuda(), a_mask.cuda(), l_idx.cuda(), 0.1, BLOCK_M=block_m,
                       MAX_ANCESTORS=slots, out_dtype=torch.float32)
     assert kernel in _lib.load().fsta_last_attention_kernel().decode()
     assert_close(o, want, torch.bfloat16, f"{slots} slots")
