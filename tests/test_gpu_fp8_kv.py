@@ -134,6 +134,41 @@ def test_quantize_matches_the_formula(keys, d, dtype):
         assert bool(same.all()), f"{int((~same).sum())} bytes differ"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_quantize_one_tensor_after_the_other(dtype):
+    """Tensors too large for a grid of both go one after the other and share the workspace: a pair of ordinary size, the
+    grid's end set below it, against the launch of both."""
+    import ctypes
+    from fstattention_amd import _lib
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    fn = lib.fsta_internal_quantize_fp8
+    fn.restype = ctypes.c_int
+    fn.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t,
+                                           ctypes.c_double, ctypes.c_void_p]
+    code = _lib.BF16 if dtype is torch.bfloat16 else _lib.F32
+    slices, elements = 6, 1111 * 64
+    k, v, _ = (t.cuda() for t in rand_qkv(2, 3, 1111, 1111, 64, dtype, 77))
+    v = v * 3.0
+    need = _lib.load().fsta_quantize_workspace_bytes(slices, elements, code)
+    assert need > 0
+    per_tensor = slices * -(-elements // 8192) * 512       # threads
+    results = []
+    for grid_threads in (2.0 ** 32, 2.0 * per_tensor, 2.0 * per_tensor + 1, 0.0):
+        k8, v8 = (torch.full(t.shape, 0x55, dtype=torch.uint8, device="cuda") for t in (k, v))
+        ks, vs = torch.zeros(slices, device="cuda"), torch.zeros(slices, device="cuda")
+        work = torch.full((need,), 0xff, dtype=torch.uint8, device="cuda")
+        rc = fn(k.data_ptr(), v.data_ptr(), k8.data_ptr(), v8.data_ptr(), ks.data_ptr(), vs.data_ptr(), slices, elements, code,
+                work.data_ptr(), need, grid_threads, torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.OK
+        # (the shared workspace's second half is written by the launch of both only)
+        assert bool((work[need // 2:] == 0xff).all()) == (grid_threads <= 2.0 * per_tensor)
+        results.append([t.cpu() for t in (k8, v8, ks, vs)])
+    want = quantize_kv_fp8(k, v)
+    for r in results:
+        for got, ref in zip(r, want):
+            assert torch.equal(got.view(torch.uint8), ref.cpu().view(torch.uint8).view(got.view(torch.uint8).shape))
+
+
 def test_argument_errors():
     parent = trees.random_recursive_parents(64, 5)
     a_idx, a_mask, l_idx, max_anc = oracle_inputs(parent, 32)
