@@ -289,12 +289,15 @@ def test_cache_kernel_edges(dtype, nodes, block_m, d, z, h, prefix, splits):
     (160, 64, 2, 512, 1),
     (288, 128, 1, 513, 1),                  # nine row groups, one key more
     (288, 64, 2, 1200, 1),                  # two pairs of rounds and a rest
-    (256, 128, 2, 1700, 3),                 # 18 tiles a run: a pair and two tiles; the last run one tile shorter
+    (256, 128, 2, 1700, 3),                 # 54 tiles, 18 a run: a pair and two tiles; the last tile has four keys
+    (256, 128, 2, 1504, 3),                 # 47 tiles: two runs of one pair, the last run a tile short of it
+    (200, 64, 2, 1473, 3),                  # the same, one key in the last tile, seven row groups
     (160, 128, 60, 257, 1)])                # more workgroups than CUs: four waves, a pair is 256 keys
-def test_cache_kernel_row_groups_in_different_order(nodes, d, h, prefix, splits):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_cache_kernel_row_groups_in_different_order(nodes, d, h, prefix, splits, dtype):
     """Five and more row groups: every other one takes the rounds of a run two by two in the other order."""
     parent = trees.random_recursive_parents(nodes, nodes + prefix, window=24)
-    run_tree(parent, 32, 1, h, d, torch.bfloat16, 6, prefix=prefix, key_splits=splits, want_kernel="attn_cache_kernel")
+    run_tree(parent, 32, 1, h, d, dtype, 6, prefix=prefix, key_splits=splits, want_kernel="attn_cache_kernel")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -402,11 +405,24 @@ def test_two_tiles_per_step_with_peaked_weights(dtype, scale):
 def test_blocks_of_128_rows_with_the_whole_list_in_the_ring(dtype, ancestors):
     """head_dim 64, enough workgroups that no block is halved: lists of five and six tiles have a ring as long as
     the list, longer ones walk a ring of four."""
-    n = 300                                                      # a ragged last block
+    n = 300                                                      # (padded to whole blocks)
     parent = np.arange(-1, n - 1, dtype=np.int64) % ancestors     # a chain of that many nodes, all others its children
     parent[0] = -1
     parent[1:ancestors] = np.arange(ancestors - 1)
     run_tree(parent, 128, 2, 24, 64, dtype, 8, native_out=True, want_kernel=", 64, 128, ")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block_m,heads,ancestors", [(128, 88, 20), (128, 88, 64), (128, 88, 90), (64, 56, 40), (64, 56, 130)])
+def test_eight_waves_per_simd_in_launches_of_several_rounds(dtype, block_m, heads, ancestors):
+    """head_dim 64 in workgroups of eight waves, more than 256 of them: Q waits in the ring's last slots, with the first tiles
+    requested in front of it (blocks of 128: lists of five and six tiles in a ring of as many, seven in a ring of four; blocks
+    of 64: two waves share a row group's Q); a last block of 44 rows."""
+    n = 300
+    parent = np.arange(-1, n - 1, dtype=np.int64) % ancestors     # a chain of that many nodes, all others its children
+    parent[0] = -1
+    parent[1:ancestors] = np.arange(ancestors - 1)
+    run_ragged(parent, block_m, heads, 64, dtype, 12, ", 64, %d, " % block_m)
 
 
 def test_reference_test_shape_with_and_without_prefix():
