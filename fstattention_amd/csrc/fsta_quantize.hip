@@ -77,33 +77,34 @@ template <typename T> __device__ __forceinline__ float unit_value(const Unit<T>&
     }
 }
 
-// float -> e4m3, round to nearest even, magnitudes that round beyond 448 and NaN -> NaN
-__device__ __forceinline__ uint32_t fp8_any(float y) {
-    const uint32_t sign = (__builtin_bit_cast(uint32_t, y) >> 24) & 0x80u;
-    const float a = fabsf(y);
-    if (!(a < 480.f)) return sign | 0x7fu;
-    if (a < 0.015625f) return sign | (uint32_t)rintf(a * 512.f);     // below 2^-6: steps of 2^-9
-    int e;
-    const float m = frexpf(a, &e);                                   // a = m * 2^e, m in [0.5, 1)
-    return sign | (uint32_t)(((e + 6) << 3) + (int)rintf(m * 16.f) - 8);   // (a carry of the rounding goes into the exponent)
-}
-
+// Scales at the ends of the range, and slices with an infinity or a NaN (`plain` = false): divisor and values are brought to the
+// middle of the range by a power of two, where the short division below is as exact as elsewhere (what is lost of a value
+// underneath rounds to zero either way).  Denormal scales are coarse, so quotients past 448 have to be looked for.
 struct Scale {
-    float s, inv;
-    bool plain;      // s lies where the short division below is exact
+    float s;             // as stored
+    float div, inv, pre; // the quotient is (x * pre) / div, inv = 1 / div
+    bool plain;          // pre = 1, and no quotient exceeds 448 by more than a rounding
 };
 __device__ __forceinline__ Scale make_scale(float amax) {
     Scale sc;
     sc.s = amax > 0.f ? amax * (1.f / kFp8Max) : 1.f;                // (NaN: 1)
-    sc.inv = 1.f / sc.s;
-    sc.plain = amax >= 0.f && sc.s > 0x1p-60f && sc.s < 0x1p60f;      // no value then exceeds 448 by more than a rounding
+    sc.plain = amax >= 0.f && sc.s > 0x1p-60f && sc.s < 0x1p60f;
+    sc.pre = sc.plain || !(amax >= 0.f) ? 1.f : sc.s < 1.f ? 0x1p100f : 0x1p-100f;
+    sc.div = sc.s * sc.pre;
+    sc.inv = 1.f / sc.div;
+    if (sc.s == INFINITY) sc.div = sc.inv = 0.f;                      // finite values: x * 0 = 0, infinities: NaN
     return sc;
 }
 // x / s, correctly rounded: with inv = 1/s correctly rounded, one residual step on x * inv gives the rounded quotient
 // (Markstein); 3 instructions in place of the ten of a full division.  A zero loses its sign.
 __device__ __forceinline__ float divide(float x, const Scale& sc) {
     const float q0 = x * sc.inv;
-    return __builtin_fmaf(__builtin_fmaf(-q0, sc.s, x), sc.inv, q0);
+    return __builtin_fmaf(__builtin_fmaf(-q0, sc.div, x), sc.inv, q0);
+}
+// The same for any scale; magnitudes that round beyond 448 become NaN, as the format has no infinity (464 is a tie, to 448).
+__device__ __forceinline__ float divide_any(float x, const Scale& sc) {
+    const float q = fabsf(divide(x * sc.pre, sc));
+    return q <= 464.f ? fminf(q, kFp8Max) : __builtin_nanf("");
 }
 // The signs of elements 4w .. 4w+3 in bit 7 of their bytes (the scale is positive: they are the bytes' signs, zeros' and
 // NaNs' too; two instructions for four elements instead of one each).
@@ -118,20 +119,18 @@ template <typename T> __device__ __forceinline__ uint32_t signs(const Unit<T>& u
     }
 }
 // PAST: around the caches
-template <bool PAST, typename T>
-__device__ __forceinline__ void store_unit(const Unit<T>& u, const Scale& sc, const T* src, uint8_t* dst) {
-    if (!sc.plain) {      // (rare, and kept short: element by element from memory)
-#pragma unroll 1
-        for (int i = 0; i < kUnitElems; ++i) dst[i] = (uint8_t)fp8_any(to_float(src[i]) / sc.s);
-        return;
-    }
+template <bool PAST, typename T> __device__ __forceinline__ void store_unit(const Unit<T>& u, const Scale& sc, uint8_t* dst) {
     u32x4 out;
+    auto bytes = [&](auto quotient) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        int pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w), sc), divide(unit_value(u, 4 * w + 1), sc), 0, false);
-        pk = __builtin_amdgcn_cvt_pk_fp8_f32(divide(unit_value(u, 4 * w + 2), sc), divide(unit_value(u, 4 * w + 3), sc), pk, true);
-        out[w] = ((uint32_t)pk & 0x7f7f7f7fu) | signs(u, w);
-    }
+        for (int w = 0; w < 4; ++w) {
+            int pk = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(unit_value(u, 4 * w), sc), quotient(unit_value(u, 4 * w + 1), sc), 0, false);
+            pk = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(unit_value(u, 4 * w + 2), sc), quotient(unit_value(u, 4 * w + 3), sc), pk, true);
+            out[w] = ((uint32_t)pk & 0x7f7f7f7fu) | signs(u, w);
+        }
+    };
+    if (sc.plain) bytes([](float x, const Scale& c) { return divide(x, c); });
+    else bytes([](float x, const Scale& c) { return divide_any(x, c); });
     if constexpr (PAST) __builtin_nontemporal_store(out, reinterpret_cast<u32x4*>(dst));
     else *reinterpret_cast<u32x4*>(dst) = out;
 }
@@ -177,7 +176,7 @@ __global__ __launch_bounds__(kOneThreads) void quantize_slice_kernel(QuantArgs a
     for (int i = 0; i < N; ++i)
         if (tid + i * kOneThreads < units) {
             const size_t at = (size_t)(tid + i * kOneThreads) * kUnitElems;
-            store_unit<false>(u[i], sc, src + at, dst + at);
+            store_unit<false>(u[i], sc, dst + at);
         }
     if (tid == 0) (tensor ? a.scale[1] : a.scale[0])[slice] = sc.s;
 }
@@ -210,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void quantize_pieces_kernel(QuantArgs a) 
     } else {
         const Scale sc = make_scale(from_bits<T>(mx));
         uint8_t* dst = (tensor ? a.dst[1] : a.dst[0]) + (size_t)slice * a.elems;
-        if (at < a.elems) store_unit<true>(u, sc, src + at, dst + at);
+        if (at < a.elems) store_unit<true>(u, sc, dst + at);
         if (tid == 0 && piece == 0) (tensor ? a.scale[1] : a.scale[0])[slice] = sc.s;
     }
 }

@@ -134,6 +134,34 @@ def test_quantize_matches_the_formula(keys, d, dtype):
         assert bool(same.all()), f"{int((~same).sum())} bytes differ"
 
 
+@pytest.mark.parametrize("keys", [64, 2100])      # one launch, two
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_quantize_at_the_ends_of_the_range(keys, dtype):
+    """Slices whose scale is huge, tiny, denormal or rounds to zero, with zeros, infinities and NaN among them: the bytes and
+    scales of the formula, evaluated on the host."""
+    info = torch.finfo(dtype)
+    g = torch.Generator().manual_seed(keys)
+    x = torch.randn((1, 12, keys, 64), generator=g, dtype=torch.float64)
+    x = x / x.abs().amax(dim=(2, 3), keepdim=True)
+    x[0, :, :, 0] *= 2.0 ** -7                                # quotients down to the smallest bytes
+    x[0, :, :, 1] *= 2.0 ** -16
+    x[0, :, 0, 2:6] = torch.tensor([0.0, -0.0, 1.0, -1.0])
+    tops = [info.max, info.max / 3, 2.0 ** 69, 2.0 ** 68.9, 2.0 ** -51, 2.0 ** -52, info.tiny, info.tiny * 448, info.tiny / 50,
+            info.tiny * info.eps * 300, info.tiny * info.eps * 3, info.max]
+    k = (x * torch.tensor([min(t, info.max) for t in tops], dtype=torch.float64).view(1, -1, 1, 1)).to(dtype)
+    v = k.flip(1).clone()
+    v[0, 0, 1, 1], v[0, 1, 1, 2], v[0, 4, 2, 3], v[0, 11, 0, 0] = float("inf"), -float("inf"), float("nan"), -float("nan")
+    got = quantize_kv_fp8(k.cuda(), v.cuda())
+    for t, t8, scale in ((k, got[0], got[2]), (v, got[1], got[3])):
+        amax = t.float().abs().amax(dim=(2, 3))
+        want = torch.where(amax > 0, amax * torch.tensor(1.0 / 448.0, dtype=torch.float32), torch.ones_like(amax))
+        assert torch.equal(scale.cpu().nan_to_num(nan=-1.0), want.view(-1).nan_to_num(nan=-1.0))
+        want8 = (t.float() / want[:, :, None, None]).to(torch.float8_e4m3fn)      # (scale 1 where a NaN is the largest)
+        a, b = t8.cpu().view(torch.uint8), want8.view(torch.uint8)
+        same = (a == b) | ((a & 0x7f == 0x7f) & (b & 0x7f == 0x7f))
+        assert bool(same.all()), f"{int((~same).sum())} bytes differ, slices {(~same).any(-1).any(-1).nonzero().tolist()}"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_quantize_one_tensor_after_the_other(dtype):
     """Tensors too large for a grid of both go one after the other and share the workspace: a pair of ordinary size, the
