@@ -295,6 +295,26 @@ def test_medusa_tree_built_on_the_gpu_matches_the_host_builder():
 
 
 
+@pytest.mark.parametrize("low", [-15.94, -16.0, -16.06, -24.0, -31.0, -60.0, -79.0, -79.5, -80.0, -400.0])
+def test_medusa_tree_thresholds_below_the_first_window(low):
+    """Thresholds in every part of the search: around the first window's lower end (2^-15.94), in the coarser one below it, and
+    underneath that (2^-79), with candidates on both sides and with ties at the threshold."""
+    rng = np.random.default_rng(int(-low * 100))
+    spread = np.sort(rng.uniform(-0.6, 0.6, (4, 10)))[:, ::-1]
+    probs = 2.0 ** (spread + low / 3.5)                           # thresholds of deep trees lie around 2^low
+    ties = 2.0 ** np.round(4 * (spread + low / 3.5))
+    ties = np.where(ties > 0, np.minimum(ties ** 0.25, 1.0), 0.0)
+    for p in (probs, ties):
+        for n in (12, 200, 1000, 5000, 10500):
+            np.testing.assert_array_equal(medusa_parents_gpu(torch.from_numpy(p).cuda(), n).cpu().numpy(), _best_paths_host(p, n),
+                                          err_msg=f"n={n}")
+    one = np.full((2, 70), 2.0 ** (low / 2))                      # 70 paths at half of it, 4900 at 2^low exactly
+    one[1, 35:] *= 1.0 - 2.0 ** -30                               # .. or a hair below
+    for n in (60, 71, 72, 1500, 2521, 2522, 4000, 4971):
+        np.testing.assert_array_equal(medusa_parents_gpu(torch.from_numpy(one).cuda(), n).cpu().numpy(), _best_paths_host(one, n),
+                                      err_msg=f"n={n}")
+
+
 @pytest.mark.parametrize("factor", [2.0 ** 9, 1.0, 2.0 ** -6, 2.0 ** -15, 2.0 ** -40, 2.0 ** -1060])
 @pytest.mark.parametrize("depths,topk", [(4, 10), (3, 10), (2, 100)])
 def test_medusa_tree_scores_in_and_outside_of_the_first_window(depths, topk, factor):
