@@ -113,11 +113,13 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
 // and runs of prefix tiles (runs = 0: not at all).  Shape and flags only.
 //
 // The number of runs is the one with the shortest predicted time.  The constants are those that choose best, not those that
-// predict best: fitted to the choice over 91000 timings of 14000 shapes (8-256 rows, 8-512 slices, 64-32768 keys, K and V of
-// three calls in turn), the run count they pick costs 0.6 % over the best candidate on average, 2.2 % at the ninetieth
-// percentile, 25 % at worst (shapes held out of the fit: the same; 45000 older timings with up to 1024 rows: 1.1, 4, 58 %),
-// where a prediction without `cu_rate` and the products' type, fitted to the times, cost 2.2, 8 and 66 % (84 slices of
-// 32 rows behind 12055 keys, D 64: 73 us in one run, 45 in three; 64 slices of 49 rows, 32694 keys: 173, 105).
+// predict best, over 28199 shapes (8-512 rows, 8-bit K/V up to 4096; 1-512 slices; 64-32768 keys), every candidate timed with K
+// and V from HBM, as a step through a model's layers finds them, and from the Infinity Cache; HBM counts more.  They cost 0.8 to
+// 1.2 % over the best candidate on average, 3 to 4 % at the ninetieth percentile, 47 % at worst (8790 shapes of another
+// day: 0.8-1.3, 3-5, 33 %).  Constants fitted to K and V of three calls in turn, mostly from the Infinity Cache, took too few
+// runs where fewer workgroups than CUs leave HBM idle (32 slices of 87 rows behind 2829 keys, D 128: 23.2 us in two runs, 22.4 in
+// five; of 12513 shapes at head_dim 128 in 16 bits 129 were more than 4 % slower from HBM than under the constants before
+// those, 29 are now); constants without `cu_rate`, fitted to the times, cost 1.7-2.3, 6-7 and 66 %.
 //   1.6 (launch) + rounds of workgroups * start_end + the larger of
 //     workgroups on the fullest CU * tiles * tile   (a CU's matrix cores, L2 and LDS)      [us]
 //     rounds * tiles per wave * wave_tile           (one wave's chain)
@@ -125,16 +127,14 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
 //   but no less than start_end + the prefix read once at `tb1` or, with several row groups, `tb` TB/s (rereading by the other
 //   groups: a fraction `again` each), and no faster than `cu_rate` B/ns for each CU that has a workgroup,
 //   + for more than one run `join` and the float32 parts, written and read once at `join_tb` TB/s.
-// Several runs are taken only where they are predicted at less than `several` of one run's time: of 8078 shapes of the three
-// kinds with 0.92, 26 instead of 57 are more than 4 % slower than under the earlier constants (662 instead of 766 as much
-// faster; 0.1 % on average).  At head_dim 128 in 16 bits it would be more of them, not fewer.
+// Several runs are taken only where they are predicted at less than `several` of one run's time.
 struct CacheCost {
     float start_end8, start_end4, tile, wave_tile, f16, join, join_tb, tb1, tb, again, cu_rate, several;
 };
-constexpr CacheCost kCost16[2] = {{2.71f, 2.42f, 0.0481f, 1.1f, 1.06f, 2.84f, 2.83f, 9.67f, 8.05f, 0.34f, 50.2f, 0.92f},       // head_dim 64
-                                  {4.11f, 0.236f, 0.346f, 0.555f, 1.04f, 1.56f, 1.27f, 9.0f, 11.5f, 0.64f, 46.3f, 1.0f}};      // head_dim 128
+constexpr CacheCost kCost16[2] = {{2.06f, 1.71f, 0.273f, 1.5f, 0.932f, 4.11f, 1.0f, 5.4f, 4.24f, 0.193f, 29.7f, 1.0f},         // head_dim 64
+                                  {3.65f, 1.23f, 0.5f, 1.39f, 1.0f, 3.26f, 1.71f, 6.01f, 7.0f, 0.61f, 35.6f, 0.956f}};         // head_dim 128
 constexpr CacheCost kCost8[2] = {{2.42f, 3.46f, 0.112f, 0.602f, 1.01f, 2.39f, 16.8f, 6.09f, 4.28f, 0.08f, 33.7f, 0.92f},        // the same on 8-bit K/V
-                                 {2.76f, 5.56f, 0.208f, 0.628f, 1.16f, 3.14f, 15.4f, 8.89f, 6.05f, 0.412f, 66.8f, 0.92f}};
+                                 {1.78f, 1.26f, 0.436f, 0.45f, 0.961f, 2.68f, 1.22f, 3.25f, 3.96f, 0.8f, 67.9f, 0.931f}};
 // Longer trees: 16-bit K/V go to the dense prefix kernel and the tree kernel, which read the prefix once per 128 and 64
 // rows; a workgroup of the cache kernel reads it for 32 rows.
 constexpr int kCacheMaxRows = 512;
@@ -184,6 +184,12 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
         const int64_t wgs = wgs1 * runs;
         // more workgroups than CUs: four waves each, so that one workgroup's start and end lie under another's tiles
         const int waves = wgs > kGpuCus ? 4 : 8;
+        // Half of the CUs busy with one or two row groups in one run, at most three tiles a wave in two: K and V from HBM up to
+        // 8 % faster, from the Infinity Cache 15 % slower (64 slices of 37 and 46 rows behind 1310 keys, bf16; fp16, without the
+        // second weight half, 10-16 % faster and 2-9 % slower: two runs).
+        if (i > 0 && !forced && !kv8 && head_dim == 128 && dtype == FSTA_BF16 && groups <= 2 && waves == 8 && 2 * wgs1 >= kGpuCus &&
+            per <= 3 * waves)
+            continue;
         const double on_cu = (double)((wgs + kGpuCus - 1) / kGpuCus);
         const int at_once = (head_dim == 128 ? 1 : 2) * (waves == 4 ? 2 : 1);
         const double rounds = (double)(((int64_t)on_cu + at_once - 1) / at_once);
@@ -232,6 +238,12 @@ int launch_cache(AttnParams p, int dtype, int out_dtype, int head_dim, bool kv8,
 }
 
 }  // namespace
+
+// Runs the cache kernel would take this problem in, 0 where it would not: what tests pin the choice by.  Not part of the interface.
+extern "C" int fsta_internal_cache_runs(int64_t slices, int32_t nq, int32_t nk, int32_t head_dim, int32_t dtype, int32_t block_m,
+                                        int32_t max_ancestors, int32_t kv8) {
+    return plan_cache(slices, nq, nk, head_dim, dtype, block_m, max_ancestors, 0.1f, 0u, kv8 != 0).runs;
+}
 
 extern "C" size_t fsta_attention_workspace_bytes(int32_t batch, int32_t heads, int32_t nq, int32_t nk,
                                                  int32_t head_dim, int32_t dtype, int32_t block_m,

@@ -235,6 +235,34 @@ def test_workspace_planning_is_host_arithmetic():
     assert odd == _lib.EINVAL and b"aligned" in lib.fsta_last_error()
 
 
+@pytest.mark.parametrize("kv8,head_dim,dtype,slices,rows,keys,runs", [
+    # 16 bits: few bytes on their way with fewer workgroups than CUs (K and V from HBM: 32 slices of 87 rows behind 2829 keys
+    # 23.2 us in two runs, 22.4 in five; 32, 63, 960: 14.5 in one, 12.2 in four; 80, 122, 3421: one run 14 % over three)
+    (0, 128, "BF16", 32, 71, 2867, 5), (0, 128, "BF16", 32, 87, 2829, 5), (0, 128, "F16", 32, 63, 960, 4),
+    (0, 128, "BF16", 16, 117, 899, 4), (0, 128, "BF16", 80, 122, 3421, 3), (0, 128, "F16", 80, 128, 3039, 3),
+    (0, 64, "F16", 32, 27, 1340, 7), (0, 64, "BF16", 8, 63, 1290, 6), (0, 64, "BF16", 80, 49, 4019, 3),
+    # 64 to 127 workgroups behind long prefixes: what a workgroup draws on its own
+    (0, 128, "BF16", 80, 25, 1859, 3), (0, 128, "BF16", 48, 49, 20588, 8), (0, 64, "F16", 84, 32, 12055, 3),
+    (0, 64, "BF16", 64, 49, 32694, 2), (1, 128, "BF16", 84, 12, 9886, 3), (1, 64, "BF16", 64, 20, 8590, 4),
+    # one run where several promise too little (8 bits, 120, 21, 1676: 17.1 us, 21.1 in two; 128, 89, 5525: 60.2, 73.6)
+    (0, 128, "BF16", 32, 256, 1000, 1), (0, 128, "F16", 128, 61, 3001, 1), (1, 128, "BF16", 120, 21, 1676, 1),
+    (1, 128, "BF16", 128, 32, 1838, 1), (1, 128, "F16", 128, 89, 5525, 1),
+    # two of eight waves, runs of a tile for each wave
+    (0, 128, "F16", 32, 96, 1934, 2), (1, 128, "BF16", 32, 128, 8192, 2), (1, 128, "BF16", 32, 12, 833, 4)])
+def test_number_of_key_runs_behind_a_kv_cache(kv8, head_dim, dtype, slices, rows, keys, runs):
+    """The choice of runs is a fit to timings: pinned where a wrong count was measured to cost."""
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    fn = lib.fsta_internal_cache_runs
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int64] + [ctypes.c_int32] * 7
+    assert fn(slices, rows, rows + keys, head_dim, getattr(_lib, dtype), 32, 64, kv8) == runs
+    if kv8:      # (the workspace is that of the runs, or none)
+        size = _lib.load().fsta_attention_kv8_workspace_bytes(1, slices, rows, rows + keys, head_dim, getattr(_lib, dtype), 32, 64, 0.1)
+        assert size == (runs * slices * rows * (head_dim + 1) * 4 if runs > 1 else 0)
+    else:
+        uses = _lib.load().fsta_attention_uses_workspace(1, slices, rows, rows + keys, head_dim, getattr(_lib, dtype), 32, 64, 0.1, 0)
+        assert uses == (1 if runs > 1 else 0)
+
+
 def test_python_entry_points_refuse_to_run_without_a_gpu_path():
     import torch
     from fstattention_amd import create_fst_attention_kernel_inputs, fst_attention, trees
