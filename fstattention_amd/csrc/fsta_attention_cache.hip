@@ -160,8 +160,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_cache_kernel(AttnParams p, Ca
     // 5.5).  So every other group takes the rounds of a run (a tile per wave) two by two in the other order: twice the bytes on
     // their way, and what one group fetched from memory its neighbour finds in L2 a round later.  Measured with K and V in HBM,
     // as a step through a model's layers finds them (32 slices, bf16, D 128): 256 rows behind 600, 1100, 6000 keys 12.0 ->
-    // 10.3, 16.3 -> 14.6, 54.0 -> 51.7 us, 130 rows, 1100 keys 16.0 -> 14.4; with K and V in the Infinity Cache, where the way is
-    // short, 0-3 % slower.  Two to four groups have enough on their way (128 rows, 2000 keys: 4 % slower, 61 rows: 7 %); whole
+    // 10.3, 16.3 -> 14.6, 54.0 -> 51.7 us, 130 rows, 1100 keys 16.0 -> 14.4; 1506 launches of 8-32 slices behind 64-4096 keys:
+    // 0.90-1.00 of the time in every class of slices and bytes, the smallest (8 slices, under 2.5 MB) 0.98-0.99.  With K and V
+    // in the Infinity Cache, where the way is short, 0.96-1.02, 1.02-1.05 above 15 MB at D 64: no line in the bytes would win
+    // more than it gives.  Two to four groups have enough on their way (128 rows, 2000 keys: 4 % slower, 61 rows: 7 %); whole
     // runs or four rounds in other orders bring more at once and overfill the L2; 8-bit tiles are half as large and their
     // arithmetic is longer than the way (no gain).
     const bool swapped = !KV8 && gr.chunks >= 5 && (chunk & 1);
