@@ -114,12 +114,12 @@ int plan_dense_prefix(int64_t slices, int nq, int nk, int head_dim, int dtype, i
 //
 // The number of runs is the one with the shortest predicted time.  The constants are those that choose best, not those that
 // predict best, over 28199 shapes (8-512 rows, 8-bit K/V up to 4096; 1-512 slices; 64-32768 keys), every candidate timed with K
-// and V from HBM, as a step through a model's layers finds them, and from the Infinity Cache; HBM counts more.  They cost 0.8 to
+// and V from HBM, as a step through a model's layers finds them, and from the Infinity Cache; HBM counts more.  They cost 0.9 to
 // 1.2 % over the best candidate on average, 3 to 4 % at the ninetieth percentile, 47 % at worst (8790 shapes of another
-// day: 0.8-1.3, 3-5, 33 %).  Constants fitted to K and V of three calls in turn, mostly from the Infinity Cache, took too few
+// day: 0.9-1.3, 3-5, 33 %).  Constants fitted to K and V of three calls in turn, mostly from the Infinity Cache, took too few
 // runs where fewer workgroups than CUs leave HBM idle (32 slices of 87 rows behind 2829 keys, D 128: 23.2 us in two runs, 22.4 in
 // five; of 12513 shapes at head_dim 128 in 16 bits 129 were more than 4 % slower from HBM than under the constants before
-// those, 29 are now); constants without `cu_rate`, fitted to the times, cost 1.7-2.3, 6-7 and 66 %.
+// those, 48 are now); constants without `cu_rate`, fitted to the times, cost 1.7-2.3, 6-7 and 66 %.
 //   1.6 (launch) + rounds of workgroups * start_end + the larger of
 //     workgroups on the fullest CU * tiles * tile   (a CU's matrix cores, L2 and LDS)      [us]
 //     rounds * tiles per wave * wave_tile           (one wave's chain)
@@ -135,6 +135,16 @@ constexpr CacheCost kCost16[2] = {{2.06f, 1.71f, 0.273f, 1.5f, 0.932f, 4.11f, 1.
                                   {3.65f, 1.23f, 0.5f, 1.39f, 1.0f, 3.26f, 1.71f, 6.01f, 7.0f, 0.61f, 35.6f, 0.956f}};         // head_dim 128
 constexpr CacheCost kCost8[2] = {{2.42f, 3.46f, 0.112f, 0.602f, 1.01f, 2.39f, 16.8f, 6.09f, 4.28f, 0.08f, 33.7f, 0.92f},        // the same on 8-bit K/V
                                  {1.78f, 1.26f, 0.436f, 0.45f, 0.961f, 2.68f, 1.22f, 3.25f, 3.96f, 0.8f, 67.9f, 0.931f}};
+// Prefixes of at most 7 MB, 32 layers of which the Infinity Cache holds: constants searched on K and V of three calls in turn.  What
+// those above gain from HBM there (7 % where they choose otherwise, nearly always more runs) they lose from the cache at head_dim
+// 128 (9 %; 24 layers of 8 slices, 165 rows behind 744 keys: 261 us a step, 221 this way), and calls that short wait for the
+// host, for which a second launch is half a call more (24 layers of 8 slices, 63 rows behind 1290 keys, head_dim 64: 204 to 247 us
+// a step on three hosts in six runs, 213 in one).
+constexpr CacheCost kFew16[2] = {{2.71f, 2.42f, 0.0481f, 1.1f, 1.06f, 2.84f, 2.83f, 9.67f, 8.05f, 0.34f, 50.2f, 0.92f},
+                                 {4.11f, 0.236f, 0.346f, 0.555f, 1.04f, 1.56f, 1.27f, 9.0f, 11.5f, 0.64f, 46.3f, 1.0f}};
+constexpr CacheCost kFew8[2] = {{2.42f, 3.46f, 0.112f, 0.602f, 1.01f, 2.39f, 16.8f, 6.09f, 4.28f, 0.08f, 33.7f, 0.92f},
+                                {2.76f, 5.56f, 0.208f, 0.628f, 1.16f, 3.14f, 15.4f, 8.89f, 6.05f, 0.412f, 66.8f, 0.92f}};
+constexpr double kFewBytes = 7.0;      // MB of K and V
 // Longer trees: 16-bit K/V go to the dense prefix kernel and the tree kernel, which read the prefix once per 128 and 64
 // rows; a workgroup of the cache kernel reads it for 32 rows.
 constexpr int kCacheMaxRows = 512;
@@ -168,8 +178,8 @@ CachePlan plan_cache(int64_t slices, int nq, int nk, int head_dim, int dtype, in
         if (head_dim == 128 && wgs1 > 512 && (prefix < 600 || (wgs1 > 1200 && nq > 96 && prefix < kDenseMinKeys))) return c;
     }
     const int forced = (int)((flags >> 8) & 0xffu);
-    const CacheCost& k = (kv8 ? kCost8 : kCost16)[head_dim == 128 ? 1 : 0];
     const double bytes = (double)slices * prefix * head_dim * (kv8 ? 2.0 : 4.0) * 1e-6;      // prefix K and V, MB
+    const CacheCost& k = (bytes <= kFewBytes ? (kv8 ? kFew8 : kFew16) : (kv8 ? kCost8 : kCost16))[head_dim == 128 ? 1 : 0];
     const double product = dtype == FSTA_F16 ? k.f16 : 1.0;
     double best = 0.0, one = 0.0;
     // candidates: one run, the counts that fill the CUs once, twice, .., and those whose runs are one, two, .. tiles for
